@@ -1036,8 +1036,6 @@ def gmsd_stats_bwd(x, y, mean, std, g_mean, g_std, T, eps, downsample, need_dx, 
     """dL/dx, dL/dy of L = g_mean . mean + g_std . std (float64 arithmetic)."""
     x, y = _contig(x), _contig(y)
     n, c, h, w = (int(v) for v in x.shape)
-    hd, wd = (h // 2, w // 2) if downsample else (h, w)
-    aux = torch.empty((4, n * c, hd - 2, wd - 2), dtype=torch.float64, device=x.device)
     gm = None if g_mean is None else g_mean.to(torch.float64).contiguous()
     gs = None if g_std is None else g_std.to(torch.float64).contiguous()
     dx = torch.empty_like(x) if need_dx else None
@@ -1045,7 +1043,7 @@ def gmsd_stats_bwd(x, y, mean, std, g_mean, g_std, T, eps, downsample, need_dx, 
     dev, stream = _site(x)
     _run("fa_gpu_gmsd_backward", _ptr(x), _ptr(y), _DTYPE_CODE[x.dtype], n, c, h, w,
          float(T), float(eps), int(bool(downsample)), _ptr(mean), _ptr(std), _ptr(gm),
-         _ptr(gs), _ptr(aux), _ptr(dx), _ptr(dy), dev, stream)
+         _ptr(gs), None, _ptr(dx), _ptr(dy), dev, stream)
     return dx, dy
 
 

@@ -759,174 +759,300 @@ __global__ __launch_bounds__(BLOCK) void gmsd_finalize_kernel(
 
 // --------------------------------------------------------------------------
 // backward (an extension): gradients of per-image mean and standard
-// deviation of q, for x / y of float32 or float64, all in float64.
+// deviation of q, for x / y of float32 or float64, all in float64, in one pass.
 //
-//   coefficient pass: per output pixel, with w = dL/dq = g_mean/n +
-//     g_std (q - m)/(n std), dq/dg1 = 2 (g2 - g1)(g2 (g1 + g2) + T)/D^2 (the
-//     factored form, exact in sign and accurate where g1 ~ g2) and
-//     dg/dgx = gx/g: the four maps dL/dgx1, dL/dgy1, dL/dgx2, dL/dgy2.
-//     A workgroup stages the (16 + 2) x (64 + 2) samples of its tile in LDS.
-//   scatter: per input pixel, the Prewitt adjoint of those maps at its
-//     sample (12 taps per tensor, zero outside the map), a quarter of it with
-//     downsampling, none for the dropped odd row / column.
+// With w = dL/dq = g_mean/n + g_std (q - m)/(n std) and dq/dg1 =
+// 2 (g2 - g1)(g2 (g1 + g2) + T)/D^2 (the factored form, exact in sign and
+// accurate where g1 ~ g2), the gradient of the samples is the Prewitt adjoint of
+// dL/dg1 gx1/g1 and dL/dg1 gy1/g1 (and the same for y): a 3 x 3 stencil of a
+// 3 x 3 stencil, so a sample's gradient needs the samples within two of it.
+//
+// A wave walks a strip of 64 sample columns down a run of rows, one column per
+// lane, with everything in registers: a three-row window of samples forms an
+// output row's coefficients, whose horizontal adjoint (neighbours by DPP both
+// times) enters a three-row window of partial sums that completes one gradient
+// row per step.  No LDS, no barrier and no coefficient maps in memory: 60 of
+// the 64 columns are the strip's own and a run starts four rows early.
+//
+// What bounds it: the vector ALU (~150 instructions a step) and the loads (x
+// and y once, dx once) about equally.  8 x 3 x 540 x 960 float32 with
+// downsampling, dx alone: 30.5 us (4.9 TB/s), against 120.3 us for a
+// coefficient pass into four float64 maps and a scatter that gathered from them.
 // --------------------------------------------------------------------------
-constexpr int GB_TR = 16;  // output rows per coefficient tile
-constexpr int GB_TC = 64;  // output columns per coefficient tile
+constexpr int GB_OUTW = WAVE - 4;  // gradient columns per strip
+constexpr int GB_HALO = 4;         // sample rows a run reads besides its own
+constexpr int GB_WAVES_PER_SIMD = 3;
 
 struct GmsdBwdArgs {
   const void* x;
   const void* y;
   int C, H, W, Hd, Wd, Hout, Wout;
   double T, eps;
+  double k2;             // (s / 3)^2: gradient components from raw Prewitt sums of the
+                         //   unnormalised samples (s = 1/4 with downsampling, else 1)
   const double* mean;
   const double* std_;
   const double* g_mean;  // may be null: zero
   const double* g_std;   // may be null: zero
-  double* aux;           // 4 maps [planes, Hout, Wout]
-  int64_t map_stride;    // planes * Hout * Wout
   void* dx;
   void* dy;
-  int tiles_x, tiles_y;
+  int strips, chunks, rows;  // per plane; sample rows per run
+  int64_t tasks;             // planes * chunks * strips, one wave each
+};
+
+// Lane i receives lane i-1's value; lane 0 receives 0 (DPP wave_shr:1).
+__device__ inline double wave_prev(double v) {
+  const int64_t b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, static_cast<int>(b & 0xffffffff), 0x138, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, static_cast<int>(b >> 32), 0x138, 0xf, 0xf, true);
+  return __longlong_as_double((static_cast<int64_t>(hi) << 32) |
+                              static_cast<int64_t>(static_cast<uint32_t>(lo)));
+}
+
+// 1 / v to within an ulp: v_rcp_f64 and two Newton steps (a third of the
+// instructions of the IEEE division; 1 / 0 stays inf through the select).
+__device__ inline double gb_rcp(double v) {
+  const double r0 = __builtin_amdgcn_rcp(v);
+  const double r1 = fma(fma(-v, r0, 1.0), r0, r0);
+  const double r2 = fma(fma(-v, r1, 1.0), r1, r1);
+  return v == 0.0 ? r0 : r2;
+}
+
+// sqrt(v) and 1 / sqrt(v) together by Goldschmidt's iteration on v_rsq_f64:
+// g -> sqrt v, h -> 1 / (2 sqrt v), then one correction of g.  v = 0 (a flat
+// patch with eps = 0) gives 0 and inf, whose products are the NaN of 0 / 0.
+__device__ inline void gb_sqrt(double v, double& root, double& inv) {
+  const double y = __builtin_amdgcn_rsq(v);
+  double g = v * y, h = 0.5 * y;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const double r = fma(-h, g, 0.5);
+    g = fma(g, r, g);
+    h = fma(h, r, h);
+  }
+  g = fma(fma(-g, g, v), h, g);
+  root = v == 0.0 ? 0.0 : g;
+  inv = v == 0.0 ? y : 2.0 * h;
+}
+
+// Two samples-to-be of one input row as one load or store; rows of odd W start
+// off the pair's own alignment, which a 4- / 8-byte aligned vector access takes.
+template <typename T>
+struct GbPair {
+  T a, b;
 };
 
 template <typename T, bool DOWN>
-__device__ inline double gb_sample(const T* plane, int W, int r, int c) {
-  if constexpr (DOWN) {
-    const int64_t o = static_cast<int64_t>(2 * r) * W + 2 * c;
-    return 0.25 * ((Elem<T>::d(plane[o]) + Elem<T>::d(plane[o + 1])) +
-                   (Elem<T>::d(plane[o + W]) + Elem<T>::d(plane[o + W + 1])));
-  } else {
-    return Elem<T>::d(plane[static_cast<int64_t>(r) * W + c]);
-  }
-}
+struct GbRaw {
+  GbPair<T> x[DOWN ? 2 : 1], y[DOWN ? 2 : 1];
+};
 
-template <typename T, bool DOWN>
-__global__ __launch_bounds__(BLOCK) void gmsd_coef_kernel(GmsdBwdArgs a) {
-  __shared__ double sx[GB_TR + 2][GB_TC + 2];
-  __shared__ double sy[GB_TR + 2][GB_TC + 2];
-  const int per_plane = a.tiles_x * a.tiles_y;
-  const int plane = blockIdx.x / per_plane;
-  const int t = blockIdx.x - plane * per_plane;
-  const int R0 = (t / a.tiles_x) * GB_TR;
-  const int C0 = (t % a.tiles_x) * GB_TC;
-  const int64_t poff = static_cast<int64_t>(plane) * a.H * a.W;
+template <typename T, bool DOWN, bool DX, bool DY>
+__global__ __launch_bounds__(BLOCK) void gmsd_backward_kernel(GmsdBwdArgs a) {
+  const int64_t wg = xcd_tile(blockIdx.x, gridDim.x);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int64_t task = wg * WAVES_PER_BLOCK + wave;
+  if (task >= a.tasks) return;  // whole wave; no barrier follows
+  const int lane = threadIdx.x % WAVE;
+  const int strip = static_cast<int>(task % a.strips);
+  const int64_t pc = task / a.strips;
+  const int chunk = static_cast<int>(pc % a.chunks);
+  const int64_t plane = pc / a.chunks;
+  const int r0 = chunk * a.rows;               // first gradient row (sample grid)
+  const int rows = min(a.rows, a.Hd - r0);
+  const int c = strip * GB_OUTW - 2 + lane;    // this lane's sample column
+  const int64_t poff = plane * a.H * a.W;
   const T* px = static_cast<const T*>(a.x) + poff;
   const T* py = static_cast<const T*>(a.y) + poff;
-  // stage the samples; rows / columns past the sample grid are clamped (they
-  // only feed outputs outside the map)
-  for (int e = threadIdx.x; e < (GB_TR + 2) * (GB_TC + 2); e += BLOCK) {
-    const int r = e / (GB_TC + 2), c = e - r * (GB_TC + 2);
-    const int gr = min(R0 + r, a.Hd - 1), gc = min(C0 + c, a.Wd - 1);
-    sx[r][c] = gb_sample<T, DOWN>(px, a.W, gr, gc);
-    sy[r][c] = gb_sample<T, DOWN>(py, a.W, gr, gc);
-  }
-  __syncthreads();
+  // loads are clamped into the grid: what lies past it only feeds masked outputs
+  const int cl = c < 0 ? 0 : (c < a.Wd ? c : a.Wd - 1);
 
-  const int n = plane / a.C;
+  const int n = static_cast<int>(plane / a.C);
   const double cnt = static_cast<double>(a.C) * a.Hout * a.Wout;
-  const double gm = a.g_mean ? a.g_mean[n] : 0.0;
   const double gsd = a.g_std ? a.g_std[n] : 0.0;
   const double sd = a.std_[n];
   const double ks = sd > 0.0 ? gsd / (cnt * sd) : 0.0;
   const double m = a.mean[n];
-  const double third = 1.0 / 3.0;
-  for (int e = threadIdx.x; e < GB_TR * GB_TC; e += BLOCK) {
-    const int i = e / GB_TC, j = e - i * GB_TC;
-    const int oi = R0 + i, oj = C0 + j;
-    if (oi >= a.Hout || oj >= a.Wout) continue;
-    double gx1 = 0.0, gy1 = 0.0, gx2 = 0.0, gy2 = 0.0;
-#pragma unroll
-    for (int u = 0; u < 3; ++u) {
-      gx1 += sx[i + u][j] - sx[i + u][j + 2];
-      gy1 += sx[i][j + u] - sx[i + 2][j + u];
-      gx2 += sy[i + u][j] - sy[i + u][j + 2];
-      gy2 += sy[i][j + u] - sy[i + 2][j + u];
-    }
-    gx1 *= third;
-    gy1 *= third;
-    gx2 *= third;
-    gy2 *= third;
-    const double G1 = fma(gx1, gx1, fma(gy1, gy1, a.eps));
-    const double G2 = fma(gx2, gx2, fma(gy2, gy2, a.eps));
-    const double g1 = sqrt(G1), g2 = sqrt(G2);
-    const double D = G1 + G2 + a.T;
-    const double q = fma(2.0 * g1, g2, a.T) / D;
-    const double w = gm / cnt + ks * (q - m);
-    // g2 - g1 = (G2 - G1) / (g1 + g2), with G2 - G1 in factored form
-    const double dG = fma(gx2 - gx1, gx2 + gx1, (gy2 - gy1) * (gy2 + gy1));
-    const double dg = dG / (g1 + g2);
-    const double iD2 = 1.0 / (D * D);
-    const double d1 = w * 2.0 * dg * fma(g2, g1 + g2, a.T) * iD2;   // w dq/dg1
-    const double d2 = -w * 2.0 * dg * fma(g1, g1 + g2, a.T) * iD2;  // w dq/dg2
-    const int64_t o = static_cast<int64_t>(plane) * a.Hout * a.Wout +
-                      static_cast<int64_t>(oi) * a.Wout + oj;
-    a.aux[o] = d1 * gx1 / g1;
-    a.aux[a.map_stride + o] = d1 * gy1 / g1;
-    a.aux[2 * a.map_stride + o] = d2 * gx2 / g2;
-    a.aux[3 * a.map_stride + o] = d2 * gy2 / g2;
-  }
-}
+  const double wm = (a.g_mean ? a.g_mean[n] : 0.0) / cnt;
+  const double Tc = a.T, eps = a.eps, k2 = a.k2;
+  const double w2 = 2.0 * k2;  // 2 of dq/dg, k of gx = k P, k of the adjoint
 
-// (1/3) sum_u [Gx(a-u, b) - Gx(a-u, b-2)] + (1/3) sum_u [Gy(a, b-u) - Gy(a-2, b-u)]
-__device__ inline double prewitt_adjoint(const double* gx, const double* gy, int Hout, int Wout,
-                                         int r, int c) {
-  auto at = [&](const double* m, int i, int j) {
-    return (i >= 0 && i < Hout && j >= 0 && j < Wout) ? m[static_cast<int64_t>(i) * Wout + j]
-                                                      : 0.0;
+  auto load = [&](int r) {
+    const int rr = r < 0 ? 0 : (r < a.Hd ? r : a.Hd - 1);
+    GbRaw<T, DOWN> v;
+    if constexpr (DOWN) {
+      const int64_t o = static_cast<int64_t>(2 * rr) * a.W + 2 * cl;
+      __builtin_memcpy(&v.x[0], px + o, sizeof(v.x[0]));
+      __builtin_memcpy(&v.x[1], px + o + a.W, sizeof(v.x[1]));
+      __builtin_memcpy(&v.y[0], py + o, sizeof(v.y[0]));
+      __builtin_memcpy(&v.y[1], py + o + a.W, sizeof(v.y[1]));
+    } else {
+      const int64_t o = static_cast<int64_t>(rr) * a.W + cl;
+      v.x[0].a = px[o];
+      v.y[0].a = py[o];
+    }
+    return v;
   };
-  double s = 0.0;
-#pragma unroll
-  for (int u = 0; u < 3; ++u) {
-    s += at(gx, r - u, c) - at(gx, r - u, c - 2);
-    s += at(gy, r, c - u) - at(gy, r - 2, c - u);
+  auto sample = [&](const GbPair<T>* p) {
+    if constexpr (DOWN)
+      return (static_cast<double>(p[0].a) + static_cast<double>(p[0].b)) +
+             (static_cast<double>(p[1].a) + static_cast<double>(p[1].b));
+    else
+      return static_cast<double>(p[0].a);
+  };
+
+  // the samples of rows s - 2 and s - 1 at step s, and the horizontal adjoints
+  // of the two output rows before this step's: hx = Gx(c) - Gx(c - 2),
+  // hy = Gy(c) + Gy(c - 1) + Gy(c - 2)
+  double xa = 0.0, xb = 0.0, ya = 0.0, yb = 0.0;
+  double hx1[2] = {0.0, 0.0}, hy1[2] = {0.0, 0.0}, hx2[2] = {0.0, 0.0}, hy2[2] = {0.0, 0.0};
+  const bool col_on = c >= 0 && c < a.Wout;                       // an output column
+  const bool own = lane >= 2 && lane < WAVE - 2 && c < a.Wd;      // a gradient column
+
+  auto step = [&](int s, const GbRaw<T, DOWN>& raw) {
+    const double xc = sample(raw.x), yc = sample(raw.y);
+    // raw Prewitt sums of the window rows s - 2 .. s (output row i = s - 2)
+    auto prewitt_at = [&](double t0, double t1, double t2, double& gx, double& gy) {
+      const double cs = t0 + t1 + t2, rd = t0 - t2;
+      const double rd1 = wave_next(rd);
+      gx = cs - wave_next(wave_next(cs));
+      gy = rd + rd1 + wave_next(rd1);
+    };
+    double gx1, gy1, gx2, gy2;
+    prewitt_at(xa, xb, xc, gx1, gy1);
+    prewitt_at(ya, yb, yc, gx2, gy2);
+    xa = xb;
+    xb = xc;
+    ya = yb;
+    yb = yc;
+    const double G1 = fma(k2, fma(gx1, gx1, gy1 * gy1), eps);
+    const double G2 = fma(k2, fma(gx2, gx2, gy2 * gy2), eps);
+    double g1, i1, g2, i2;
+    gb_sqrt(G1, g1, i1);
+    gb_sqrt(G2, g2, i2);
+    const double gs = g1 + g2;
+    const double D = G1 + G2 + Tc;
+    const double iD = gb_rcp(D), is = gb_rcp(gs);
+    const double q = fma(2.0 * g1, g2, Tc) * iD;
+    const double w = fma(ks, q - m, wm);
+    // g2 - g1 = (G2 - G1) / (g1 + g2), with G2 - G1 in factored form
+    const double dG = k2 * fma(gx2 - gx1, gx2 + gx1, (gy2 - gy1) * (gy2 + gy1));
+    const double f = w * w2 * (dG * is) * (iD * iD);
+    const int i = s - 2;
+    const bool on = col_on && i >= 0 && i < a.Hout;  // outside the map: no share
+    auto adjoint = [&](double t, double gx, double gy, double (&hx)[2], double (&hy)[2]) {
+      const double cx = on ? t * gx : 0.0, cy = on ? t * gy : 0.0;
+      const double cy1 = wave_prev(cy);
+      const double nx = cx - wave_prev(wave_prev(cx));
+      const double ny = cy + cy1 + wave_prev(cy1);
+      const double v = (nx + hx[1] + hx[0]) + (ny - hy[0]);
+      hx[0] = hx[1];
+      hx[1] = nx;
+      hy[0] = hy[1];
+      hy[1] = ny;
+      return v;
+    };
+    double vx = 0.0, vy = 0.0;
+    if constexpr (DX) vx = adjoint(f * fma(g2, gs, Tc) * i1, gx1, gy1, hx1, hy1);
+    if constexpr (DY) vy = adjoint(-f * fma(g1, gs, Tc) * i2, gx2, gy2, hx2, hy2);
+    if (own && i >= r0) {  // gradient row i is complete
+      auto put = [&](void* d, double v) {
+        T* out = static_cast<T*>(d) + poff;
+        if constexpr (DOWN) {
+          const GbPair<T> t = {static_cast<T>(v), static_cast<T>(v)};
+          const int64_t o = static_cast<int64_t>(2 * i) * a.W + 2 * c;
+          __builtin_memcpy(out + o, &t, sizeof(t));
+          __builtin_memcpy(out + o + a.W, &t, sizeof(t));
+          if (c == a.Wd - 1 && 2 * a.Wd < a.W) {  // the column the 2 x 2 mean drops
+            out[o + 2] = T(0);
+            out[o + a.W + 2] = T(0);
+          }
+        } else {
+          out[static_cast<int64_t>(i) * a.W + c] = static_cast<T>(v);
+        }
+      };
+      if constexpr (DX) put(a.dx, vx);
+      if constexpr (DY) put(a.dy, vy);
+    }
+  };
+
+  // Sample rows r0 - 2 .. r0 + rows + 1: the first two only fill the window,
+  // each later one completes an output row; two rows of loads in flight.
+  const int s0 = r0, steps = rows + GB_HALO - 2;
+  const GbRaw<T, DOWN> p0 = load(s0 - 2), p1 = load(s0 - 1);
+  GbRaw<T, DOWN> buf0 = load(s0), buf1 = load(s0 + 1);
+  xa = sample(p0.x);
+  ya = sample(p0.y);
+  xb = sample(p1.x);
+  yb = sample(p1.y);
+  for (int j = 0; j < steps; j += 2) {  // uniform
+    const GbRaw<T, DOWN> cur0 = buf0, cur1 = buf1;
+    buf0 = load(s0 + j + 2);
+    buf1 = load(s0 + j + 3);
+    step(s0 + j, cur0);
+    if (j + 1 < steps) step(s0 + j + 1, cur1);
   }
-  return s * (1.0 / 3.0);
+  if constexpr (DOWN) {  // the row the 2 x 2 mean drops
+    if (chunk == a.chunks - 1 && 2 * a.Hd < a.H && own) {
+      auto zero = [&](void* d) {
+        T* out = static_cast<T*>(d) + poff + static_cast<int64_t>(a.H - 1) * a.W + 2 * c;
+        out[0] = T(0);
+        out[1] = T(0);
+        if (c == a.Wd - 1 && 2 * a.Wd < a.W) out[2] = T(0);
+      };
+      if constexpr (DX) zero(a.dx);
+      if constexpr (DY) zero(a.dy);
+    }
+  }
 }
 
-template <typename T, bool DOWN>
-__global__ __launch_bounds__(BLOCK) void gmsd_scatter_kernel(GmsdBwdArgs a, int64_t total) {
-  for (int64_t e = static_cast<int64_t>(blockIdx.x) * BLOCK + threadIdx.x; e < total;
-       e += static_cast<int64_t>(gridDim.x) * BLOCK) {
-    const int64_t plane = e / (static_cast<int64_t>(a.H) * a.W);
-    const int64_t rem = e - plane * a.H * a.W;
-    const int h = static_cast<int>(rem / a.W), w = static_cast<int>(rem - (rem / a.W) * a.W);
-    const int r = DOWN ? h / 2 : h, c = DOWN ? w / 2 : w;
-    const bool in = r < a.Hd && c < a.Wd;  // the dropped odd row / column
-    const int64_t mo = plane * a.Hout * a.Wout;
-    const double scale = DOWN ? 0.25 : 1.0;
-    if (a.dx) {
-      const double v = in ? scale * prewitt_adjoint(a.aux + mo, a.aux + a.map_stride + mo,
-                                                    a.Hout, a.Wout, r, c)
-                          : 0.0;
-      static_cast<T*>(a.dx)[e] = static_cast<T>(v);
+template <typename T, bool DOWN, bool DX, bool DY>
+static int launch_gmsd_bwd_k(GmsdBwdArgs& a, int64_t planes, int device, hipStream_t st) {
+  static const int occ = [] {
+    int v = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
+            &v, reinterpret_cast<const void*>(&gmsd_backward_kernel<T, DOWN, DX, DY>), BLOCK, 0) !=
+            hipSuccess ||
+        v <= 0)
+      v = 1;
+    return v;
+  }();
+  // Rows per run: rounds of waves times the rows a wave walks.  A round is
+  // GB_WAVES_PER_SIMD waves per SIMD, not all that fit: each step is ~150 vector
+  // instructions, so two or three waves keep a SIMD issuing, and more waves only
+  // mean shorter runs under the same four halo rows.  8 x 3 x 540 x 960 float32,
+  // dx alone, 1 / 2 / 3 / 4 / 5 / 6 waves: 35.0 / 30.7 / 30.8 / 31.6 / 33.6 /
+  // 35.0 us.
+  const int64_t resident = static_cast<int64_t>(cu_count(device)) *
+                           std::min(occ, GB_WAVES_PER_SIMD) * WAVES_PER_BLOCK;
+  a.strips = (a.Wd + GB_OUTW - 1) / GB_OUTW;
+  int64_t best = INT64_MAX;
+  for (int ch = 1; ch <= a.Hd; ++ch) {
+    const int rows = (a.Hd + ch - 1) / ch;
+    if (rows < 4 && ch > 1) break;
+    const int64_t waves = planes * a.strips * ch;
+    const int64_t cost = ((waves + resident - 1) / resident) * (rows + GB_HALO);
+    if (cost < best) {
+      best = cost;
+      a.rows = rows;
     }
-    if (a.dy) {
-      const double v = in ? scale * prewitt_adjoint(a.aux + 2 * a.map_stride + mo,
-                                                    a.aux + 3 * a.map_stride + mo, a.Hout,
-                                                    a.Wout, r, c)
-                          : 0.0;
-      static_cast<T*>(a.dy)[e] = static_cast<T>(v);
-    }
+    if (waves > 4 * resident) break;  // more rounds only add halo rows
   }
+  a.chunks = (a.Hd + a.rows - 1) / a.rows;
+  a.tasks = planes * a.strips * a.chunks;
+  const int64_t wgs = (a.tasks + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
+  if (wgs > INT32_MAX / BLOCK) return FA_E_SHAPE;
+  hipLaunchKernelGGL((gmsd_backward_kernel<T, DOWN, DX, DY>), dim3(static_cast<unsigned>(wgs)),
+                     dim3(BLOCK), 0, st, a);
+  FA_LAUNCH_CHECK();
+  return FA_OK;
 }
 
 template <typename T, bool DOWN>
 static int launch_gmsd_bwd(GmsdBwdArgs& a, int64_t planes, int device, hipStream_t st) {
-  a.tiles_x = (a.Wout + GB_TC - 1) / GB_TC;
-  a.tiles_y = (a.Hout + GB_TR - 1) / GB_TR;
-  const int64_t wgs = planes * a.tiles_x * a.tiles_y;
-  if (wgs > INT32_MAX) return FA_E_SHAPE;
-  hipLaunchKernelGGL((gmsd_coef_kernel<T, DOWN>), dim3(static_cast<unsigned>(wgs)), dim3(BLOCK),
-                     0, st, a);
-  FA_LAUNCH_CHECK();
-  const int64_t total = planes * a.H * a.W;
-  const int64_t want = (total + BLOCK - 1) / BLOCK;
-  const int64_t cap = static_cast<int64_t>(cu_count(device)) * 16;
-  hipLaunchKernelGGL((gmsd_scatter_kernel<T, DOWN>),
-                     dim3(static_cast<unsigned>(want < cap ? want : cap)), dim3(BLOCK), 0, st, a,
-                     total);
-  FA_LAUNCH_CHECK();
-  return FA_OK;
+  if (a.dx && a.dy) return launch_gmsd_bwd_k<T, DOWN, true, true>(a, planes, device, st);
+  return a.dx ? launch_gmsd_bwd_k<T, DOWN, true, false>(a, planes, device, st)
+              : launch_gmsd_bwd_k<T, DOWN, false, true>(a, planes, device, st);
 }
 
 struct GGeom {
@@ -1194,14 +1320,16 @@ FA_API int fa_gpu_gmsd_once(const void* x, const void* y, int dtype, int N, int 
 //   L = sum_n g_mean[n] mean_n(q) + g_std[n] std_n(q)
 // with respect to contiguous x and y (N x C x H x W, FA_F32 or FA_F64); mean /
 // std are fa_gpu_gmsd's outputs for the same inputs; g_mean / g_std are
-// device arrays of N (either may be null: zero); aux is 4 * N*C*Hout*Wout
-// float64 scratch; dx / dy (either may be null) are written in full.
+// device arrays of N (either may be null: zero); aux, which earlier builds
+// kept coefficient maps in, is not used; dx / dy (either may be null) are
+// written in full.
 FA_API int fa_gpu_gmsd_backward(const void* x, const void* y, int dtype, int N, int C, int H,
                                 int W, double Tc, double eps, int downsample,
                                 const double* mean, const double* std_dev,
                                 const double* g_mean, const double* g_std, double* aux,
                                 void* dx, void* dy, int device, void* stream) {
-  if (!x || !y || !mean || !std_dev || !aux) return FA_E_ARG;
+  (void)aux;
+  if (!x || !y || !mean || !std_dev) return FA_E_ARG;
   if (!dx && !dy) return FA_E_ARG;
   if (dtype != FA_F32 && dtype != FA_F64) return FA_E_DTYPE;
   if (N <= 0 || C <= 0) return FA_E_SHAPE;
@@ -1224,9 +1352,8 @@ FA_API int fa_gpu_gmsd_backward(const void* x, const void* y, int dtype, int N, 
   a.std_ = std_dev;
   a.g_mean = g_mean;
   a.g_std = g_std;
-  a.aux = aux;
+  a.k2 = downsample ? 1.0 / 144.0 : 1.0 / 9.0;
   const int64_t planes = static_cast<int64_t>(N) * C;
-  a.map_stride = planes * g.Hout * g.Wout;
   a.dx = dx;
   a.dy = dy;
   FA_DEVICE_SCOPE(device);

@@ -541,6 +541,36 @@ def test_gms_gmsd_gradient_matches_oracle(gpu, down, dt):
         assert err <= 1e-6, err
 
 
+@pytest.mark.parametrize("hw", [(6, 7), (7, 119), (8, 120), (9, 121), (21, 122), (40, 125),
+                                (65, 127), (130, 241), (3, 60), (5, 61)])
+@pytest.mark.parametrize("wrt", ["x", "y", "xy"])
+def test_gms_gradient_strip_edges(gpu, hw, wrt):
+    """The one-pass backward around its strips of 60 gradient columns, its runs
+    of rows and the row and column a downsample drops; x, y or both.  float32
+    results of float64 arithmetic: 2^-24 per value, bar 1e-6 normwise."""
+    h, w = hw
+    for down in (True, False):
+        if min(h, w) // (2 if down else 1) < 3:
+            continue
+        rng = np.random.default_rng(h * 1000 + w)
+        a = rng.random((2, 2, h, w), dtype=np.float32)
+        b = np.clip(a + 0.1 * rng.standard_normal(a.shape), 0, 1).astype(np.float32)
+        x = torch.from_numpy(a).to(gpu).requires_grad_("x" in wrt)
+        y = torch.from_numpy(b).to(gpu).requires_grad_("y" in wrt)
+        gm, gs = np.array([0.7, -1.2]), np.array([1.4, 0.5])
+        kw = dict(data_range=1.0, downsample=down, reduction="none")
+        ((fa.gms(x, y, **kw) * torch.tensor(gm, device=gpu)).sum()
+         + (fa.gmsd(x, y, **kw) * torch.tensor(gs, device=gpu)).sum()).backward()
+        want = ref.gms_stats_grad(a.astype(np.float64), b.astype(np.float64), 1.0,
+                                  downsample=down, g_mean=gm, g_std=gs)
+        for t, g in ((x, want[0]), (y, want[1])):
+            if t.requires_grad:
+                got = t.grad.cpu().double().numpy()
+                assert np.abs(got - g).max() <= 1e-6 * np.abs(g).max(), (hw, down)
+            else:
+                assert t.grad is None
+
+
 def test_gms_loss_gradient_finite(gpu):
     x = torch.rand(1, 1, 64, 64, device=gpu, requires_grad=True)
     y = x.detach().clone()
