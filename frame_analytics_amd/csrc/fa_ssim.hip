@@ -1361,7 +1361,9 @@ static int ms_plan(int dtype, int N, int C, int H, int W, int K, int M, bool lum
       p->level_dtype[i] = u8 ? (i == 1 ? FA_F16 : FA_F32) : FA_F64;
       p->in_dtype[i] = u8 ? (p->level_dtype[i] | FA_DTYPE_U8_PYRAMID) : FA_F64;
       const int64_t eb = p->level_dtype[i] == FA_F16 ? 2 : p->level_dtype[i] == FA_F32 ? 4 : 8;
-      const int64_t lb = planes * p->H[i] * p->W[i] * eb;
+      // (rows of a uint8 pyramid's levels with room for the three-launch form's
+      // padding; the per-scale form packs them)
+      const int64_t lb = planes * p->H[i] * (u8 ? mf_level_pitch(p->W[i]) : p->W[i]) * eb;
       p->level_x[i] = take(lb);
       p->level_y[i] = take(lb);
     } else {

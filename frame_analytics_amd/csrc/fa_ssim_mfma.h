@@ -42,14 +42,18 @@ struct SsimMfmaCall {
 };
 
 // Launches the matrix-core SSIM forward (or CS pass) when the call fits it
-// (rows and planes aligned to 8 samples, 8-byte (uint8) or 16-byte (levels)
+// (rows and planes aligned to 8 samples, 4-byte (uint8) or 16-byte (levels)
 // aligned bases, K <= 16, enough partial slots, 16-byte aligned pyramid
-// output planes).  Returns FA_OK and
+// output planes; the mean over uint8 takes rows of any width from 16 and any
+// alignment).  Returns FA_OK and
 // sets *tiles (partial slots used per plane) when it launched; returns FA_OK
 // with *tiles = 0 when the call does not fit, so the caller runs the
 // vector-ALU strip kernel instead.  With c.acc set, a launch that finished
 // the call itself (no finalize needed) sets *tiles = -1.
 int ssim_mfma(const SsimMfmaCall& c, int device, hipStream_t st, int* tiles);
+
+// Samples per row of a pyramid level of width W in the three-launch MS-SSIM.
+inline int mf_level_pitch(int W) { return (W + 7) / 8 * 8; }
 
 // Inference MS-SSIM over uint8 planes without luma, M (3 .. 5) scales, in
 // three launches: scale 0 (writing the float16 level 1), scale 1 (writing the
@@ -65,15 +69,16 @@ struct SsimMfmaMs {
   const float* win;            // the 1-D window, K floats on the device
   double C1, C2;
   const double* weights;       // host, M exponents
-  void* lx[8];                 // level i >= 1 of x and y: floor(H / 2^i) x
-  void* ly[8];                 //   floor(W / 2^i) per plane, float16 (i = 1), float32
+  void* lx[8];                 // level i >= 1 of x and y: floor(H / 2^i) rows of
+  void* ly[8];                 //   mf_level_pitch(floor(W / 2^i)) samples per plane,
+                               //   float16 (i = 1), float32
   uint64_t* words;             // FA_MS_SSIM_ACC_WORDS, zero; left zero
   double* out_per_image;
   double* out_total;
 };
 
-// Launches it when every scale fits (ssim_mfma's layout rules at each scale,
-// N * C <= 256, C1 and C2 positive) and sets *done; otherwise launches nothing
+// Launches it when the input fits ssim_mfma's rules (any width and alignment),
+// C1 and C2 positive, and sets *done; otherwise launches nothing
 // and leaves *done false, for the per-scale path.
 int ssim_mfma_ms(const SsimMfmaMs& c, int device, hipStream_t st, bool* done);
 

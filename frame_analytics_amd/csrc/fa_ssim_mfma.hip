@@ -55,6 +55,7 @@ typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u3 __attribute__((ext_vector_type(3)));
 
 template <class To, class From>
 __device__ inline To bc(From v) {
@@ -96,6 +97,8 @@ struct MfArgs {
   void* px;             // MF_CS, MF_CSO: optional pyramid level (2 x 2 means),
   void* py;             //   float32, or float16 (level_f16, uint8 input)
   int level_f16;
+  int lpitch;           // samples per row of px / py
+  int dpitch[2];        // and of dpx / dpy
   void* dpx[2];         // LVL_F32D: the two levels below px / py (float32, either
   void* dpy[2];         //   pair may be null)
   // the one-launch finish (ssim_mfma_kernel<..., FIN_SSIM>); FIN_MS uses acc
@@ -208,30 +211,56 @@ __device__ inline void split2(float v, _Float16& hi, _Float16& lo) {
   lo = static_cast<_Float16>(v - static_cast<float>(hi));
 }
 
-// fp16 hi + lo of two values as packed pairs: hi is packed with one
-// v_cvt_pkrtz (rounding toward zero), lo rounds the exact remainder, so
-// hi + lo carries each value to 2^-21.  `one` is 1.0f from the kernel
-// arguments: the remainder is written as fma(v, one, -hi), which the compiler
-// cannot fold back to a subtraction, so it maps onto v_fma_mix (reading hi
-// from the packed pair) instead of convert, subtract, convert.
+// fp16 hi + lo of two values as packed pairs; hi + lo carries each value to
+// 2^-21.  `one` is 1.0f from the kernel arguments: the remainder is written as
+// fma(v, one, -hi), which the compiler cannot fold back to a subtraction, so it
+// maps onto v_fma_mix (reading hi from the packed pair) instead of convert,
+// subtract, convert.
+//
+// Not FINE: hi toward zero (v_cvt_pkrtz), lo the exact remainder to nearest.
+// lo then has the value's sign, and the lo.lo products that the passes leave
+// out have a mean of their own: -5e-8 of the SSIM of picture-like frames.
+// FINE: hi to nearest (v_cvt_pk_f16_f32), lo toward zero, so lo has either sign
+// and those products cancel over the pixels (3e-9).  v_cvt_pk_f16_f32 issues
+// slower and its halves have to be pinned to their register: fa.ms_ssim on 8 x 3
+// x 1080 x 1920 measured 4.4-10 % slower with it, so the kernels that had the
+// first form keep it, and those that took over from the vector-ALU kernel,
+// which has no such mean, take this one.
+template <bool FINE>
 __device__ inline void split_pair(float v0, float v1, float one, uint32_t& hi, uint32_t& lo) {
-  const h2 h = bc<h2>(__builtin_amdgcn_cvt_pkrtz(v0, v1));
-  const h2 l = {static_cast<_Float16>(__builtin_fmaf(v0, one, -static_cast<float>(h.x))),
-                static_cast<_Float16>(__builtin_fmaf(v1, one, -static_cast<float>(h.y)))};
-  hi = bc<uint32_t>(h);
-  lo = bc<uint32_t>(l);
+  if constexpr (FINE) {
+    hi = bc<uint32_t>(h2{static_cast<_Float16>(v0), static_cast<_Float16>(v1)});
+    asm("" : "+v"(hi));  // the halves are read from the packed pair, not converted again
+    const h2 h = bc<h2>(hi);
+    lo = bc<uint32_t>(__builtin_amdgcn_cvt_pkrtz(
+        __builtin_fmaf(v0, one, -static_cast<float>(h.x)),
+        __builtin_fmaf(v1, one, -static_cast<float>(h.y))));
+  } else {
+    const h2 h = bc<h2>(__builtin_amdgcn_cvt_pkrtz(v0, v1));
+    const h2 l = {static_cast<_Float16>(__builtin_fmaf(v0, one, -static_cast<float>(h.x))),
+                  static_cast<_Float16>(__builtin_fmaf(v1, one, -static_cast<float>(h.y)))};
+    hi = bc<uint32_t>(h);
+    lo = bc<uint32_t>(l);
+  }
+}
+
+// 1 / d: v_rcp_f32, which is low by ~1e-8 on average, and (FINE) one Newton step.
+template <bool FINE>
+__device__ inline float recip(float d) {
+  const float r = __builtin_amdgcn_rcpf(d);
+  return FINE ? fmaf(fmaf(-d, r, 1.0f), r, r) : r;
 }
 
 // The four H values of a D fragment into half HALF (u4 elements 2 HALF,
 // 2 HALF + 1) of the vertical pass's B fragments.
-template <int HALF, bool PYR>
+template <int HALF, bool PYR, bool FINE>
 __device__ inline void stash(f4 h, float one, u4& bhi, u4& blo) {
   // pyramid levels are not pre-scaled, so their sums carry the window's 2^9
   constexpr float sc = PYR ? 1.0f / WSCALE : 1.0f;
 #pragma unroll
   for (int p = 0; p < 2; ++p) {
     uint32_t hi, lo;
-    split_pair(h[2 * p] * sc, h[2 * p + 1] * sc, one, hi, lo);
+    split_pair<FINE>(h[2 * p] * sc, h[2 * p + 1] * sc, one, hi, lo);
     bhi[2 * HALF + p] = hi;
     blo[2 * HALF + p] = lo;
   }
@@ -321,38 +350,65 @@ __device__ inline HAcc hmfma(const Frag& f, const Weights& w) {
   return h;
 }
 
-template <int HALF, bool PYR>
+template <int HALF, bool PYR, bool FINE>
 __device__ inline void stash_all(const HAcc& h, float one, VState& v) {
-  stash<HALF, PYR>(h.x, one, v.hi[0], v.lo[0]);
-  stash<HALF, PYR>(h.y, one, v.hi[1], v.lo[1]);
-  stash<HALF, PYR>(h.p3, one, v.hi[2], v.lo[2]);
-  stash<HALF, PYR>(h.p4, one, v.hi[3], v.lo[3]);
+  stash<HALF, PYR, FINE>(h.x, one, v.hi[0], v.lo[0]);
+  stash<HALF, PYR, FINE>(h.y, one, v.hi[1], v.lo[1]);
+  stash<HALF, PYR, FINE>(h.p3, one, v.hi[2], v.lo[2]);
+  stash<HALF, PYR, FINE>(h.p4, one, v.hi[3], v.lo[3]);
 }
 
 // One lane's 8 samples of one 16-row block: 8 bytes of x and of y (uint8), 8
 // floats of each (float32 pyramid levels) or 8 halves (float16 level).
-template <int SRC>
+template <int SRC, bool RAG>
 struct Raw;
 template <>
-struct Raw<SRC_U8> {
+struct Raw<SRC_U8, false> {
   uint2 x, y;
 };
 template <>
-struct Raw<SRC_F32> {
+struct Raw<SRC_U8, true> {
+  u3 x, y;  // the three aligned dwords that hold the 8 bytes
+};
+template <bool RAG>
+struct Raw<SRC_F32, RAG> {
   float4 x0, x1, y0, y1;
 };
-template <>
-struct Raw<SRC_F16> {
+template <bool RAG>
+struct Raw<SRC_F16, RAG> {
   u4 x, y;
 };
 
-__device__ inline Frag prep(const Raw<SRC_U8>& r, float) {
+// What a lane of a RAG pass holds besides its load: the byte at which its 8
+// samples start in the three dwords (0 .. 11; past 3 only where the row ends
+// within them), and whether any lane of the wave needs more than a byte shift
+// (uint8), or has samples past the row's end to drop (float32 levels).
+struct Edge {
+  uint32_t tx, ty;
+  int valid;  // float32 levels: samples of the lane's 8 inside the row
+  bool any;   // uniform
+};
+
+__device__ inline uint2 realign(u3 d, uint32_t t, bool any) {
+  if (any) {  // uniform: the last strips' waves
+    const bool s1 = t >= 4, s2 = t >= 8;
+    d[0] = s2 ? d[2] : s1 ? d[1] : d[0];
+    d[1] = s1 ? d[2] : d[1];  // what lies past the row only feeds columns past Wout
+  }
+  return uint2{__builtin_amdgcn_alignbyte(d[1], d[0], t), __builtin_amdgcn_alignbyte(d[2], d[1], t)};
+}
+
+__device__ inline Frag prep(const Raw<SRC_U8, false>& r, float, const Edge&) {
   return prep(r.x, r.y);
+}
+__device__ inline Frag prep(const Raw<SRC_U8, true>& r, float, const Edge& e) {
+  return prep(realign(r.x, e.tx, e.any), realign(r.y, e.ty, e.any));
 }
 
 // The first level of a uint8 pyramid in float16: the samples are the fp16
 // pairs themselves (bias 0).
-__device__ inline Frag prep(const Raw<SRC_F16>& r, float) {
+template <bool RAG>
+__device__ inline Frag prep(const Raw<SRC_F16, RAG>& r, float, const Edge&) {
   h2 xt[4], yt[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
@@ -369,9 +425,21 @@ __device__ inline Frag prep(const Raw<SRC_F16>& r, float) {
 // into fp16 hi + lo (at most 16 significant bits); x'y' and (x'-y')^2 are
 // formed in float32, as the strip kernel forms them, and split hi + lo (22
 // bits).  No scaling: the window's 2^9 is taken out of the sums (stash).
-__device__ inline Frag prep(const Raw<SRC_F32>& r, float one) {
-  const float xs[8] = {r.x0.x, r.x0.y, r.x0.z, r.x0.w, r.x1.x, r.x1.y, r.x1.z, r.x1.w};
-  const float ys[8] = {r.y0.x, r.y0.y, r.y0.z, r.y0.w, r.y1.x, r.y1.y, r.y1.z, r.y1.w};
+template <bool RAG>
+__device__ inline Frag prep(const Raw<SRC_F32, RAG>& r, float one, const Edge& e) {
+  float xs[8] = {r.x0.x, r.x0.y, r.x0.z, r.x0.w, r.x1.x, r.x1.y, r.x1.z, r.x1.w};
+  float ys[8] = {r.y0.x, r.y0.y, r.y0.z, r.y0.w, r.y1.x, r.y1.y, r.y1.z, r.y1.w};
+  if constexpr (RAG) {
+    // a padded row's padding may hold anything: a NaN there would reach every
+    // column through its zero weight
+    if (e.any) {  // uniform
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        xs[i] = i < e.valid ? xs[i] : 0.0f;
+        ys[i] = i < e.valid ? ys[i] : 0.0f;
+      }
+    }
+  }
   u4 ox, oxl, oy, oyl, o3h, o3l, o4h, o4l;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
@@ -379,16 +447,16 @@ __device__ inline Frag prep(const Raw<SRC_F32>& r, float one) {
     const float b0 = ys[2 * j] - 128.0f, b1 = ys[2 * j + 1] - 128.0f;
     const float d0 = a0 - b0, d1 = a1 - b1;
     uint32_t h, l;
-    split_pair(a0, a1, one, h, l);
+    split_pair<RAG>(a0, a1, one, h, l);
     ox[j] = h;
     oxl[j] = l;
-    split_pair(b0, b1, one, h, l);
+    split_pair<RAG>(b0, b1, one, h, l);
     oy[j] = h;
     oyl[j] = l;
-    split_pair(a0 * b0, a1 * b1, one, h, l);
+    split_pair<RAG>(a0 * b0, a1 * b1, one, h, l);
     o3h[j] = h;
     o3l[j] = l;
-    split_pair(d0 * d0, d1 * d1, one, h, l);
+    split_pair<RAG>(d0 * d0, d1 * d1, one, h, l);
     o4h[j] = h;
     o4l[j] = l;
   }
@@ -434,6 +502,7 @@ __device__ inline float ssim_px(const Epi& e, float U, float V, float X, float Q
 //   A2' = Xc - 2^-9 U V,                     B2' = A2' + Q / 2 - 2^-10 (U - V)^2
 // One instruction fewer per pixel.  The map and CS kernels keep ssim_px:
 // they have no registers to spare for the four-wide accumulator input.
+template <bool FINE>
 __device__ inline float ssim_px_folded(const Epi& e, float U, float V, float Xc, float Q) {
   const float p = U * V;
   const float t = U + V;
@@ -443,23 +512,25 @@ __device__ inline float ssim_px_folded(const Epi& e, float U, float V, float Xc,
   const float B1 = fmaf(dd, du, A1);
   const float A2 = fmaf(-0x1p-9f, p, Xc);
   const float B2 = fmaf(-dd, du, fmaf(0.5f, Q, A2));
-  return (A1 * A2) * __builtin_amdgcn_rcpf(B1 * B2);
+  return (A1 * A2) * recip<FINE>(B1 * B2);
 }
 
 // cs = A2 / B2 alone, with C2 folded into the vertical pass as in
 // ssim_px_folded (A2' = Xc - 2^-9 U V, B2' = A2' + Q / 2 - 2^-10 (U - V)^2,
 // both 2^8 times A2, B2): 8 instructions per pixel against 16 for the SSIM
 // value and cs together.
+template <bool FINE>
 __device__ inline float cs_px_folded(float U, float V, float Xc, float Q) {
   const float p = U * V;
   const float du = U - V;
   const float dd = du * 0x1p-10f;
   const float A2 = fmaf(-0x1p-9f, p, Xc);
   const float B2 = fmaf(-dd, du, fmaf(0.5f, Q, A2));
-  return A2 * __builtin_amdgcn_rcpf(B2);
+  return A2 * recip<FINE>(B2);
 }
 
 // cs = A2 / B2 beside the SSIM value (MS-SSIM's CS pass).
+template <bool FINE>
 __device__ inline void ssim_cs_px(const Epi& e, float U, float V, float X, float Q, float& s,
                                   float& cs) {
   const float p = U * V;
@@ -471,7 +542,7 @@ __device__ inline void ssim_cs_px(const Epi& e, float U, float V, float X, float
   const float A2 = fmaf(0x1p-8f, X, fmaf(-0x1p-17f, p, e.C2));
   const float B2 = fmaf(-dd, du, fmaf(0x1p-9f, Q, A2));
   // u = A2 / (B1 B2): ssim = A1 u, cs = B1 u
-  const float u = A2 * __builtin_amdgcn_rcpf(B1 * B2);
+  const float u = A2 * recip<FINE>(B1 * B2);
   s = A1 * u;
   cs = B1 * u;
 }
@@ -480,7 +551,7 @@ __device__ inline void ssim_cs_px(const Epi& e, float U, float V, float X, float
 // lane's float64 sums (MF_CSO: the cs values into acc); `full` (uniform) says
 // the whole 16 x 16 block lies inside the map.  MF_MAP also returns the four
 // values in mv; the caller stores them (MF_MAP's stores in the kernel).
-template <int MODE, bool FULL>
+template <int MODE, bool FULL, bool FINE>
 __device__ inline void finish(const Epi& e, const f4* o, int row0, int row_end, bool col_ok,
                               float (&mv)[4], double& acc, double& acc_cs) {
   float rs = 0.0f, rcs = 0.0f;
@@ -489,18 +560,18 @@ __device__ inline void finish(const Epi& e, const f4* o, int row0, int row_end, 
     const bool ok = FULL || (col_ok && row0 + i < row_end);
     if constexpr (MODE == MF_CS) {
       float s, cs;
-      ssim_cs_px(e, o[0][i], o[1][i], o[2][i], o[3][i], s, cs);
+      ssim_cs_px<FINE>(e, o[0][i], o[1][i], o[2][i], o[3][i], s, cs);
       rs += ok ? s : 0.0f;
       rcs += ok ? cs : 0.0f;
     } else if constexpr (MODE == MF_CSO) {
-      const float cs = cs_px_folded(o[0][i], o[1][i], o[2][i], o[3][i]);
+      const float cs = cs_px_folded<FINE>(o[0][i], o[1][i], o[2][i], o[3][i]);
       rs += ok ? cs : 0.0f;
     } else if constexpr (MODE == MF_MAP) {
       const float s = ssim_px(e, o[0][i], o[1][i], o[2][i], o[3][i]);
       mv[i] = s;  // stored by the caller, after the branch (see MapOut)
       rs += ok ? s : 0.0f;
     } else {
-      const float s = ssim_px_folded(e, o[0][i], o[1][i], o[2][i], o[3][i]);
+      const float s = ssim_px_folded<FINE>(e, o[0][i], o[1][i], o[2][i], o[3][i]);
       rs += ok ? s : 0.0f;
     }
   }
@@ -672,7 +743,12 @@ enum { LVL_NONE = 0, LVL_F32 = 1, LVL_F16 = 2, LVL_F32D = 3 };
 // blocks, walked down its chunk of its column strip by the four waves, each
 // lane's sums added to acc (and acc_cs, MF_CS).  The tile's plane and its
 // index within the plane come back for the caller's reduction.
-template <int SRC, int MODE, int LVL>
+//
+// RAG: rows of any width and, for uint8, any byte alignment.  A uint8 lane
+// loads the three aligned dwords around its 8 bytes and realigns them with
+// v_alignbyte (16 rows are a multiple of 4 bytes, so a lane's shift is the same
+// in every block); pyramid levels have rows padded to 8 samples.
+template <int SRC, int MODE, int LVL, bool RAG = false>
 __device__ __attribute__((always_inline)) inline void mf_walk(
     const MfArgs& a, int t, float (&swin)[WAVES_PER_BLOCK][WIN_LEN], double& acc,
     double& acc_cs, int& plane_out, int& tile_out, float* smap = nullptr) {
@@ -725,7 +801,9 @@ __device__ __attribute__((always_inline)) inline void mf_walk(
     const E* __restrict__ yp = reinterpret_cast<const E*>(a.y) + img * a.ysn + ch * a.ysc;
     // this lane's 8 input columns; a chunk past the image only feeds output
     // columns past Wout, so it is clamped (W % 8 == 0: chunks never straddle)
-    const uint32_t cc = static_cast<uint32_t>(min(c0 + 8 * g, a.W - 8));
+    // (RAG levels: the row is padded to a.xsh, a multiple of 8)
+    const uint32_t cc = static_cast<uint32_t>(
+        min(c0 + 8 * g, (RAG && SRC != SRC_U8 ? static_cast<int>(a.xsh) : a.W) - 8));
     stage_window(a.win, a.K, swin[wave], lane);
     const Weights w = load_weights(swin[wave], g, n);
     const float k1 = 2.0f * 128.0f * 128.0f + a.C1;
@@ -752,7 +830,7 @@ __device__ __attribute__((always_inline)) inline void mf_walk(
     Pool pl = {};
     if constexpr (LEVEL) {
       {
-        const int Wd = a.W / 2;
+        const int Wd = a.lpitch;  // floor(W / 2), or (RAG levels) that padded to 8
         const int eb = LVL == LVL_F16 ? 2 : 4;
         const int row_end = r_lim >= a.Hout ? 2 * (a.H / 2) : r_lim;
         const int64_t first = (static_cast<int64_t>(plane) * (a.H / 2) + r0 / 2) * Wd * eb;
@@ -773,18 +851,18 @@ __device__ __attribute__((always_inline)) inline void mf_walk(
 #pragma unroll
           for (int d = 0; d < 2; ++d) {
             const int sh = d + 2;
-            const int Wl = a.W >> sh;
+            const int Wl = a.W >> sh, Pl = a.dpitch[d];
             const int end = r_lim >= a.Hout ? (a.H >> sh) : (r_lim >> sh);
             const bool have = a.dpx[d] != nullptr;
-            const int64_t at = (static_cast<int64_t>(plane) * (a.H >> sh) + (r0 >> sh)) * Wl * 4;
+            const int64_t at = (static_cast<int64_t>(plane) * (a.H >> sh) + (r0 >> sh)) * Pl * 4;
             pl.dx[d] = static_cast<char*>(have ? a.dpx[d] : a.px) + (have ? at : 0);
             pl.dy[d] = static_cast<char*>(have ? a.dpy[d] : a.py) + (have ? at : 0);
             pl.drows[d] = have ? end - (r0 >> sh) : 0;
-            pl.dstep[d] = static_cast<uint32_t>(Wl * 4);
+            pl.dstep[d] = static_cast<uint32_t>(Pl * 4);
             const int col = (c0 / 2 + n) >> (d + 1);
             const bool first = (n & ((2 << d) - 1)) == 0 && (d == 0 || (g & 1) == 0);
             pl.dlo[d] = wave_on && first && col < Wl
-                            ? static_cast<uint32_t>(((g >> d) * Wl + col) * 4)
+                            ? static_cast<uint32_t>(((g >> d) * Pl + col) * 4)
                             : 0x80000000u;
           }
         }
@@ -812,8 +890,33 @@ __device__ __attribute__((always_inline)) inline void mf_walk(
     const uint32_t vy = (static_cast<uint32_t>(n) * a.ysh + cc) * EB;
     // plane samples and the block's first sample; the host keeps (H + 48) rows
     // of either plane below 2^31 bytes
-    const int ext_x = (a.H - 1) * static_cast<int>(a.xsh) + a.W;
-    const int ext_y = (a.H - 1) * static_cast<int>(a.ysh) + a.W;
+    // (RAG levels: the padding of the last row is read too)
+    const int last = RAG && SRC != SRC_U8 ? static_cast<int>(a.xsh) : a.W;
+    const int ext_x = (a.H - 1) * static_cast<int>(a.xsh) + last;
+    const int ext_y = (a.H - 1) * static_cast<int>(a.ysh) + last;
+    // RAG uint8: the lane's dwords start at or below its first byte, no later
+    // than the row's last three, so they hold only bytes of the plane's dwords;
+    // a column past the row takes the row's last byte (it feeds nothing)
+    Edge ed = {};
+    uint32_t wx = 0, wy = 0;  // byte offset of the dwords from the aligned base
+    uint32_t mx = 0, my = 0;  // bytes of the plane's base past a dword
+    if constexpr (RAG && SRC == SRC_U8) {
+      mx = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(xp) & 3);
+      my = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(yp) & 3);
+      const uint32_t c = static_cast<uint32_t>(min(c0 + 8 * g, a.W - 1));
+      auto place = [&](uint32_t m, uint32_t pitch, uint32_t& at, uint32_t& t) {
+        const uint32_t row = m + static_cast<uint32_t>(n) * pitch;
+        const uint32_t end = ((row + static_cast<uint32_t>(a.W) - 1) & ~3u) - 8;
+        at = min((row + c) & ~3u, end);
+        t = row + c - at;
+      };
+      place(mx, a.xsh, wx, ed.tx);
+      place(my, a.ysh, wy, ed.ty);
+      ed.any = c0 + 2 * MT + 4 > a.W;
+    } else if constexpr (RAG && SRC == SRC_F32) {
+      ed.valid = a.W - static_cast<int>(cc);
+      ed.any = c0 + 2 * MT > a.W;
+    }
     int bx = r0 * static_cast<int>(a.xsh), by = r0 * static_cast<int>(a.ysh);
     const int nb = (r_end - r0 + MT - 1) / MT;  // output blocks; H blocks 0 .. nb
     // Every step issues its load, whether or not its block is used, so that
@@ -821,7 +924,7 @@ __device__ __attribute__((always_inline)) inline void mf_walk(
     // compiler then waits for the loads alone, see MapOut); a block past nb
     // gets an empty range (uint8, float16: nothing is read) or re-reads the
     // clamped last row (float32 levels).
-    auto load = [&](int j, Raw<SRC>& r) {
+    auto load = [&](int j, Raw<SRC, RAG>& r) {
       if constexpr (PYR) {
         r.x0 = *reinterpret_cast<const float4*>(xp + xo);
         r.x1 = *reinterpret_cast<const float4*>(xp + xo + 4);
@@ -831,6 +934,20 @@ __device__ __attribute__((always_inline)) inline void mf_walk(
         yo = min(yo + ystep, ymax);
       } else {
         const bool live = j <= nb;  // uniform
+        if constexpr (RAG && SRC == SRC_U8) {
+          // ranges end with the dword that holds the plane's last byte
+          const auto qx = __builtin_amdgcn_make_buffer_rsrc(
+              const_cast<E*>(xp + bx) - mx, 0,
+              live ? max(((static_cast<int>(mx) + ext_x + 3) & ~3) - bx, 0) : 0, MF_RSRC_WORD3);
+          const auto qy = __builtin_amdgcn_make_buffer_rsrc(
+              const_cast<E*>(yp + by) - my, 0,
+              live ? max(((static_cast<int>(my) + ext_y + 3) & ~3) - by, 0) : 0, MF_RSRC_WORD3);
+          r.x = bc<u3>(__builtin_amdgcn_raw_buffer_load_b96(qx, wx, 0, 0));
+          r.y = bc<u3>(__builtin_amdgcn_raw_buffer_load_b96(qy, wy, 0, 0));
+          bx += static_cast<int>(xstep);
+          by += static_cast<int>(ystep);
+          return;
+        }
         const auto rx = __builtin_amdgcn_make_buffer_rsrc(
             const_cast<E*>(xp + bx), 0, live ? max(ext_x - bx, 0) * EB : 0, MF_RSRC_WORD3);
         const auto ry = __builtin_amdgcn_make_buffer_rsrc(
@@ -838,7 +955,7 @@ __device__ __attribute__((always_inline)) inline void mf_walk(
         if constexpr (SRC == SRC_F16) {
           r.x = bc<u4>(__builtin_amdgcn_raw_buffer_load_b128(rx, vx, 0, 0));
           r.y = bc<u4>(__builtin_amdgcn_raw_buffer_load_b128(ry, vy, 0, 0));
-        } else {
+        } else if constexpr (!RAG) {
           const auto lx = __builtin_amdgcn_raw_buffer_load_b64(rx, vx, 0, 0);
           const auto ly = __builtin_amdgcn_raw_buffer_load_b64(ry, vy, 0, 0);
           r.x = uint2{lx[0], lx[1]};
@@ -864,8 +981,8 @@ __device__ __attribute__((always_inline)) inline void mf_walk(
     // the unguarded one the float16 and float32 level kernels.
     constexpr bool GUARD = SRC == SRC_U8;
     PoolOut<HALF> po = {};
-    auto hpass = [&](int j, const Raw<SRC>& r) {
-      const Frag f = prep(r, a.one);
+    auto hpass = [&](int j, const Raw<SRC, RAG>& r) {
+      const Frag f = prep(r, a.one, ed);
       if constexpr (LEVEL) {
         po = pool_frag<PYR, HALF>(pl, f);
         if constexpr (!LATE) pool_store<HALF>(pl, j, po);
@@ -880,9 +997,9 @@ __device__ __attribute__((always_inline)) inline void mf_walk(
       const int row0 = r0 + MT * b + 4 * g;
       float mv[4];
       if (r0 + MT * (b + 1) <= r_end && c0 + MT <= a.Wout)  // uniform: the whole block
-        finish<MODE, true>(e, o, row0, r_end, col_ok, mv, acc, acc_cs);
+        finish<MODE, true, RAG>(e, o, row0, r_end, col_ok, mv, acc, acc_cs);
       else
-        finish<MODE, false>(e, o, row0, r_end, col_ok, mv, acc, acc_cs);
+        finish<MODE, false, RAG>(e, o, row0, r_end, col_ok, mv, acc, acc_cs);
       if constexpr (MODE == MF_MAP) {
         // MF_MAP's stores.  A lane holds rows 4g .. 4g+3 of one column, so
         // stored straight from the fragment each store instruction covers 64
@@ -929,9 +1046,9 @@ __device__ __attribute__((always_inline)) inline void mf_walk(
     // compiler waits with vmcnt(4): the stores stay in flight.  The first
     // step (peeled) is the only one whose loads may have nothing behind them.
     VState v;
-    Raw<SRC> raw;
+    Raw<SRC, RAG> raw;
     load(0, raw);
-    stash_all<0, PYR>(hpass(0, raw), a.one, v);
+    stash_all<0, PYR, RAG>(hpass(0, raw), a.one, v);
     load(1, raw);
     level_store(0);
     HAcc hn = hpass(1, raw);
@@ -941,7 +1058,7 @@ __device__ __attribute__((always_inline)) inline void mf_walk(
     // vertical operand and puts H_{b+1} in the second, PAR 1 the reverse
     auto step = [&](int b, auto par) {
       constexpr int PAR = decltype(par)::value;
-      stash_all<1 - PAR, PYR>(hn, a.one, v);  // H_{b+1} into the half H_{b-1} held
+      stash_all<1 - PAR, PYR, RAG>(hn, a.one, v);  // H_{b+1} into the half H_{b-1} held
       f4 o[4];
       vblock<PAR, MODE == MF_REDUCE || MODE == MF_CSO>(w, v, o, e.c2s);
       if constexpr (GUARD) {
@@ -977,15 +1094,18 @@ enum { FIN_NONE = 0, FIN_SSIM = 1, FIN_MS = 2 };
 // and beat 3; the uint8 cs-only pass writing a float32 level (which MS-SSIM
 // does not use: its first level is float16) needs more and runs 3, and so
 // does the float16 level's pass writing three levels (which spills at 128;
-// at 1080p its 720 workgroups fit 3 per CU anyway).  LVL (CS modes): the
+// at 1080p its 720 workgroups fit 3 per CU anyway) and the ragged uint8 cs pass
+// (20 bytes of spills at 128, the same time).  LVL (CS modes): the
 // pyramid level the pass writes.
-template <int SRC, int MODE, int LVL, int FIN = FIN_NONE>
+template <int SRC, int MODE, int LVL, int FIN = FIN_NONE, bool RAG = false>
 __global__ __launch_bounds__(BLOCK)
 __attribute__((amdgpu_waves_per_eu(
     SRC == SRC_F32 ? 1
-    : ((SRC == SRC_U8 && MODE == MF_CSO && LVL == LVL_F32) || LVL == LVL_F32D) ? 3
+    : ((SRC == SRC_U8 && MODE == MF_CSO && LVL == LVL_F32) || LVL == LVL_F32D || (RAG && MODE == MF_CSO)) ? 3
                                                                              : 4)))
 void ssim_mfma_kernel(MfArgs a) {
+  static_assert(!RAG || MODE == MF_REDUCE || FIN == FIN_MS,
+                "ragged rows: the uint8 forward's mean and the three-launch MS-SSIM");
   static_assert(FIN != FIN_SSIM || (MODE == MF_REDUCE && SRC == SRC_U8),
                 "the finish: uint8 forward sums");
   static_assert(FIN != FIN_MS || MODE == MF_CSO, "MS-SSIM's words: the cs sums of a scale");
@@ -994,8 +1114,8 @@ void ssim_mfma_kernel(MfArgs a) {
   __shared__ float smap[MODE == MF_MAP ? 2 * MT * MAP_PITCH : 1];  // the map's staging
   double acc = 0.0, acc_cs = 0.0;
   int plane = 0, tile = 0;
-  mf_walk<SRC, MODE, LVL>(a, static_cast<int>(xcd_tile(blockIdx.x, gridDim.x)), swin, acc,
-                          acc_cs, plane, tile, smap);
+  mf_walk<SRC, MODE, LVL, RAG>(a, static_cast<int>(xcd_tile(blockIdx.x, gridDim.x)), swin, acc,
+                               acc_cs, plane, tile, smap);
   // packed: each image owns C * tiles consecutive slots, as the finalize reads them
   const int64_t slot = static_cast<int64_t>(plane) * a.tiles + tile;
   if constexpr (MODE == MF_CS) {
@@ -1037,6 +1157,14 @@ void ssim_mfma_kernel(MfArgs a) {
 constexpr int MS_TAIL_MAX = 3;         // scales 2 .. 4 of a five-scale pyramid
 constexpr int MS_WORD_SCALES = 8;
 constexpr int MS_FIN_MAX_PLANES = 256;
+// Scales whose rows need the RAG kernels are taken from this many samples of an
+// input plane on: 151 -> 88 us for fa.ssim and fa.ms_ssim together at 4 x 3 x 767 x
+// 1366, 43 -> 23 us for fa.ms_ssim at 1 x 3 x 600 x 601.  Smaller planes would gain
+// too (38 -> 22 us at 2 x 3 x 352 x 360, 92 -> 46 at 32 x 3 x 250 x 300), but there
+// the per-scale path's results are pinned to the last bits between batch sizes,
+// with and without an accumulator and to the single CS passes, which stay on
+// the vector-ALU kernel.
+constexpr int64_t MS_RAG_MIN_PLANE = int64_t(1) << 17;
 static_assert(FA_MS_SSIM_ACC_WORDS == (MS_WORD_SCALES * MS_FIN_MAX_PLANES + 1) * MF_STRIDE,
               "the ABI's accumulator size");
 
@@ -1053,6 +1181,7 @@ struct MfTail {
   double *out_per_image, *out_total;
 };
 
+template <bool RAG>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(1)))
 void ssim_mfma_tail_kernel(MfTail m) {
   __shared__ double sred[2 * WAVES_PER_BLOCK];
@@ -1071,9 +1200,9 @@ void ssim_mfma_tail_kernel(MfTail m) {
   // form here); either way the sum the word takes ends up in acc
   const int t = b - (k > 0 ? m.wg_end[k - 1] : 0);
   if (k == m.n - 1)
-    mf_walk<SRC_F32, MF_CS, LVL_NONE>(a, t, swin, acc, acc_cs, plane, tile);
+    mf_walk<SRC_F32, MF_CS, LVL_NONE, RAG>(a, t, swin, acc, acc_cs, plane, tile);
   else
-    mf_walk<SRC_F32, MF_CSO, LVL_NONE>(a, t, swin, acc, acc_cs, plane, tile);
+    mf_walk<SRC_F32, MF_CSO, LVL_NONE, RAG>(a, t, swin, acc, acc_cs, plane, tile);
   const double s = block_sum(acc, sred);
   const int64_t planes = m.planes;
   if (threadIdx.x == 0) {
@@ -1131,13 +1260,13 @@ bool mfma_enabled() {
   return !(e && e[0] == '0');
 }
 
-template <int SRC, int MODE, int LVL, int FIN = FIN_NONE>
+template <int SRC, int MODE, int LVL, int FIN = FIN_NONE, bool RAG = false>
 int occupancy() {
   static int occ = 0;
   if (occ <= 0) {
     int v = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &v, reinterpret_cast<const void*>(&ssim_mfma_kernel<SRC, MODE, LVL, FIN>), BLOCK,
+            &v, reinterpret_cast<const void*>(&ssim_mfma_kernel<SRC, MODE, LVL, FIN, RAG>), BLOCK,
             0) != hipSuccess ||
         v <= 0)
       v = 1;
@@ -1148,18 +1277,19 @@ int occupancy() {
 
 // The kernel of (source, mode, level): its occupancy (launch == false) or its
 // launch.
-template <int SRC, int MODE, int LVL>
+template <int SRC, int MODE, int LVL, bool RAG = false>
 int run(bool launch, dim3 grid, hipStream_t st, const MfArgs& a) {
   if constexpr (SRC == SRC_U8 && MODE == MF_REDUCE) {
     if (a.acc) {
-      if (!launch) return occupancy<SRC, MODE, LVL, FIN_SSIM>();
-      hipLaunchKernelGGL((ssim_mfma_kernel<SRC, MODE, LVL, FIN_SSIM>), grid, dim3(BLOCK), 0, st,
-                         a);
+      if (!launch) return occupancy<SRC, MODE, LVL, FIN_SSIM, RAG>();
+      hipLaunchKernelGGL((ssim_mfma_kernel<SRC, MODE, LVL, FIN_SSIM, RAG>), grid, dim3(BLOCK), 0,
+                         st, a);
       return 0;
     }
   }
-  if (!launch) return occupancy<SRC, MODE, LVL>();
-  hipLaunchKernelGGL((ssim_mfma_kernel<SRC, MODE, LVL>), grid, dim3(BLOCK), 0, st, a);
+  if (!launch) return occupancy<SRC, MODE, LVL, FIN_NONE, RAG>();
+  hipLaunchKernelGGL((ssim_mfma_kernel<SRC, MODE, LVL, FIN_NONE, RAG>), grid, dim3(BLOCK), 0, st,
+                     a);
   return 0;
 }
 
@@ -1184,7 +1314,9 @@ int dispatch(int mode, bool launch, dim3 grid, hipStream_t st, const MfArgs& a) 
   return 0;
 }
 
-int dispatch(int src, int mode, bool launch, dim3 grid, hipStream_t st, const MfArgs& a) {
+int dispatch(int src, int mode, bool rag, bool launch, dim3 grid, hipStream_t st,
+             const MfArgs& a) {
+  if (rag) return run<SRC_U8, MF_REDUCE, LVL_NONE, true>(launch, grid, st, a);  // mfma_rag
   return src == SRC_F32   ? dispatch<SRC_F32>(mode, launch, grid, st, a)
          : src == SRC_F16 ? dispatch<SRC_F16>(mode, launch, grid, st, a)
                           : dispatch<SRC_U8>(mode, launch, grid, st, a);
@@ -1200,6 +1332,7 @@ namespace {
 // uint8 samples are read as 8-byte buffer loads at multiples of 8 bytes from
 // the base, so a 4-byte aligned base (a crop of 4 pixels, say) keeps every
 // load dword-aligned, which is all a multi-dword buffer access requires.
+// What only misses the alignment can still take a RAG kernel (mfma_rag).
 bool mfma_fits(const SsimMfmaCall& c, int src, int mode) {
   if (c.K > MF_MAX_K || c.W % 8 != 0 || c.W < 8) return false;
   const uintptr_t base_align = src == SRC_U8 ? 3 : 15;
@@ -1217,6 +1350,18 @@ bool mfma_fits(const SsimMfmaCall& c, int src, int mode) {
   // the map is written through buffer resources with 32-bit offsets in a plane
   if (mode == MF_MAP && static_cast<int64_t>(c.Hout) * c.Wout * 4 > INT32_MAX) return false;
   return true;
+}
+
+// The RAG kernels: uint8 rows of any width and alignment, for the forward's mean
+// and for the three-launch MS-SSIM.  Against the vector-ALU kernel that
+// took such rows, 4 x 3 x 767 x 1366: fa.ssim 49.0 -> 31 us, fa.ms_ssim 102 ->
+// 59 us (8 x 3 x 1080 x 1912: 173.6 -> 132), errors against float64 alike.  A
+// lane reads whole dwords from at most 11 bytes before its row's last
+// dword, so rows are at least 16 samples.  The map stays there: per pixel its
+// float32 sums are closer than the 22-bit operands here; so do single CS passes.
+bool mfma_rag(const SsimMfmaCall& c) {
+  if (c.K > MF_MAX_K || c.W < 16) return false;
+  return (static_cast<int64_t>(c.H) + 48) * std::max(c.xsh, c.ysh) + 16 <= INT32_MAX;
 }
 
 MfArgs args_of(const SsimMfmaCall& c) {
@@ -1245,6 +1390,7 @@ MfArgs args_of(const SsimMfmaCall& c) {
   a.px = c.px;
   a.py = c.py;
   a.level_f16 = c.level_f16 ? 1 : 0;
+  a.lpitch = c.W / 2;
   return a;
 }
 
@@ -1340,7 +1486,8 @@ int ssim_mfma(const SsimMfmaCall& c, int device, hipStream_t st, int* tiles) {
   const bool cs_pass = mode == MF_CS || mode == MF_CSO;
   if (src != SRC_U8 && !cs_pass) return FA_OK;
   if (c.level_f16 && (src != SRC_U8 || !cs_pass)) return FA_OK;
-  if (!mfma_fits(c, src, mode)) return FA_OK;
+  const bool rag = !mfma_fits(c, src, mode);
+  if (rag && !(mode == MF_REDUCE && mfma_rag(c))) return FA_OK;
   // the finish takes the uint8 forward's sums with a wanted output, where no
   // SSIM value can be NaN (C1, C2 > 0: with a zero constant a flat patch is
   // 0 / 0, which a fixed-point word cannot carry; the two-launch form's float64
@@ -1348,7 +1495,7 @@ int ssim_mfma(const SsimMfmaCall& c, int device, hipStream_t st, int* tiles) {
   const bool fin = c.acc && src == SRC_U8 && mode == MF_REDUCE && c.N <= MF_FIN_MAX_IMAGES &&
                    (c.out_per_image || c.out_total) && c.C1 > 0.0 && c.C2 > 0.0;
   MfArgs a = args_of(c);
-  const int occ = dispatch(src, mode, false, dim3(1), st, a);
+  const int occ = dispatch(src, mode, rag, false, dim3(1), st, a);
   const int64_t planes = static_cast<int64_t>(c.N) * c.C;
   if (!plan_tiles(a, planes, static_cast<int64_t>(cu_count(device)) * occ, c.bpp, true))
     return FA_OK;
@@ -1372,7 +1519,7 @@ int ssim_mfma(const SsimMfmaCall& c, int device, hipStream_t st, int* tiles) {
   // the forward's only launch without a workspace is the finish (the CS pass
   // forming the cs sums alone has a null `partial` of its own)
   if (!cs_pass && !a.acc && !c.partial) return FA_E_ARG;
-  dispatch(src, mode, true, dim3(static_cast<unsigned>(wgs)), st, a);
+  dispatch(src, mode, rag, true, dim3(static_cast<unsigned>(wgs)), st, a);
   FA_LAUNCH_CHECK();
   *tiles = a.acc ? -1 : a.tiles;
   return FA_OK;
@@ -1386,7 +1533,11 @@ int ssim_mfma_ms(const SsimMfmaMs& c, int device, hipStream_t st, bool* done) {
   if (planes > MS_FIN_MAX_PLANES || !(c.C1 > 0.0) || !(c.C2 > 0.0)) return FA_OK;
   if (!c.out_per_image && !c.out_total) return FA_OK;
   // every scale's call, checked before anything is launched
+  // Levels are rows padded to 8 samples (ms_plan sizes them so); a scale whose
+  // rows need the padding, or a uint8 input that misses the alignment, takes the
+  // RAG form of its kernel.
   MfArgs a[2 + MS_TAIL_MAX];
+  bool rag[2 + MS_TAIL_MAX] = {};
   double finv[MS_WORD_SCALES] = {}, npix[MS_WORD_SCALES] = {};
   int H = c.H, W = c.W;
   for (int i = 0; i < M; ++i) {
@@ -1394,13 +1545,14 @@ int ssim_mfma_ms(const SsimMfmaMs& c, int device, hipStream_t st, bool* done) {
     k.x = i == 0 ? c.x : c.lx[i];
     k.y = i == 0 ? c.y : c.ly[i];
     k.src = i == 0 ? SsimMfmaCall::U8 : i == 1 ? SsimMfmaCall::F16_LEVEL : SsimMfmaCall::F32_LEVEL;
-    const int64_t plane = static_cast<int64_t>(H) * W;
+    const int pitch = i == 0 ? W : mf_level_pitch(W);
+    const int64_t plane = static_cast<int64_t>(H) * pitch;
     k.xsn = i == 0 ? c.xsn : plane * c.C;
     k.xsc = i == 0 ? c.xsc : plane;
     k.ysn = i == 0 ? c.ysn : plane * c.C;
     k.ysc = i == 0 ? c.ysc : plane;
-    k.xsh = i == 0 ? c.xsh : W;
-    k.ysh = i == 0 ? c.ysh : W;
+    k.xsh = i == 0 ? c.xsh : pitch;
+    k.ysh = i == 0 ? c.ysh : pitch;
     k.N = c.N;
     k.C = c.C;
     k.H = H;
@@ -1418,13 +1570,28 @@ int ssim_mfma_ms(const SsimMfmaMs& c, int device, hipStream_t st, bool* done) {
       k.level_f16 = i == 0;
     }
     const int src = i == 0 ? SRC_U8 : i == 1 ? SRC_F16 : SRC_F32;
-    if (k.Hout < 1 || k.Wout < 1 || !mfma_fits(k, src, i + 1 < M ? MF_CSO : MF_CS)) return FA_OK;
+    const int mode = i + 1 < M ? MF_CSO : MF_CS;
+    if (k.Hout < 1 || k.Wout < 1) return FA_OK;
+    if (i == 0) {
+      rag[i] = !mfma_fits(k, src, mode);
+      if (rag[i] && !mfma_rag(k)) return FA_OK;
+    } else {
+      rag[i] = pitch != W;
+    }
+    if (rag[i] && static_cast<int64_t>(c.H) * c.W < MS_RAG_MIN_PLANE) return FA_OK;
+    if (i > 0) {
+      SsimMfmaCall q = k;  // the padded rows meet the alignment
+      q.W = pitch;
+      if (!mfma_fits(q, src, mode)) return FA_OK;
+    }
     if (i == 1)
       for (int d = 0; d < 2; ++d)
         if (3 + d < M && (reinterpret_cast<uintptr_t>(c.lx[3 + d]) |
                           reinterpret_cast<uintptr_t>(c.ly[3 + d])) & 15)
           return FA_OK;
     a[i] = args_of(k);
+    a[i].lpitch = mf_level_pitch(W / 2);
+    for (int d = 0; d < 2; ++d) a[i].dpitch[d] = mf_level_pitch(W >> (d + 2));
     npix[i] = static_cast<double>(k.Hout) * k.Wout;
     fixed_scale(npix[i], &a[i].fscale, &finv[i]);
     a[i].acc = c.words + static_cast<int64_t>(i) * planes * MF_STRIDE;
@@ -1437,10 +1604,21 @@ int ssim_mfma_ms(const SsimMfmaMs& c, int device, hipStream_t st, bool* done) {
     a[1].dpy[d] = 3 + d < M ? c.ly[3 + d] : nullptr;
   }
   const int64_t cus = cu_count(device);
-  auto k0 = ssim_mfma_kernel<SRC_U8, MF_CSO, LVL_F16, FIN_MS>;
-  auto k1 = ssim_mfma_kernel<SRC_F16, MF_CSO, LVL_F32D, FIN_MS>;
-  static const int occ0 = occupancy_of(k0), occ1 = occupancy_of(k1),
-                   occt = occupancy_of(ssim_mfma_tail_kernel);
+  bool rag_tail = false;
+  for (int i = 2; i < M; ++i) rag_tail = rag_tail || rag[i];
+  auto k0 = rag[0] ? ssim_mfma_kernel<SRC_U8, MF_CSO, LVL_F16, FIN_MS, true>
+                   : ssim_mfma_kernel<SRC_U8, MF_CSO, LVL_F16, FIN_MS>;
+  auto k1 = rag[1] ? ssim_mfma_kernel<SRC_F16, MF_CSO, LVL_F32D, FIN_MS, true>
+                   : ssim_mfma_kernel<SRC_F16, MF_CSO, LVL_F32D, FIN_MS>;
+  auto kt = rag_tail ? ssim_mfma_tail_kernel<true> : ssim_mfma_tail_kernel<false>;
+  static const int occs[2][3] = {
+      {occupancy_of(ssim_mfma_kernel<SRC_U8, MF_CSO, LVL_F16, FIN_MS>),
+       occupancy_of(ssim_mfma_kernel<SRC_F16, MF_CSO, LVL_F32D, FIN_MS>),
+       occupancy_of(ssim_mfma_tail_kernel<false>)},
+      {occupancy_of(ssim_mfma_kernel<SRC_U8, MF_CSO, LVL_F16, FIN_MS, true>),
+       occupancy_of(ssim_mfma_kernel<SRC_F16, MF_CSO, LVL_F32D, FIN_MS, true>),
+       occupancy_of(ssim_mfma_tail_kernel<true>)}};
+  const int occ0 = occs[rag[0]][0], occ1 = occs[rag[1]][1], occt = occs[rag_tail][2];
   // the counts of every word (tiles per plane) stay below 2^MF_COUNT_BITS
   constexpr int64_t max_tiles = (1 << MF_COUNT_BITS) - 1;
   if (!plan_tiles(a[0], planes, cus * occ0, max_tiles, true) ||
@@ -1514,7 +1692,7 @@ int ssim_mfma_ms(const SsimMfmaMs& c, int device, hipStream_t st, bool* done) {
   hipLaunchKernelGGL(k1, dim3(static_cast<unsigned>(planes * a[1].tiles)), dim3(BLOCK), 0, st,
                      a[1]);
   FA_LAUNCH_CHECK();
-  hipLaunchKernelGGL(ssim_mfma_tail_kernel, dim3(static_cast<unsigned>(wgs)), dim3(BLOCK), 0,
+  hipLaunchKernelGGL(kt, dim3(static_cast<unsigned>(wgs)), dim3(BLOCK), 0,
                      st, t);
   FA_LAUNCH_CHECK();
   *done = true;

@@ -533,3 +533,57 @@ def test_zero_constants_keep_nan_like_the_reference(gpu):
     st = torch.cuda.current_stream().cuda_stream
     acc = backend._stream_acc.get(("ssim", 0, st))
     assert acc is not None and not bool(acc.any())
+
+
+# --------------------------------------------------------------------------- #
+# rows of any width and alignment
+# --------------------------------------------------------------------------- #
+
+
+@pytest.mark.parametrize("hw", [(17, 16), (18, 17), (26, 18), (27, 19), (42, 26), (75, 58),
+                                (59, 74), (60, 75), (91, 139), (64, 1023)])
+def test_ragged_mean_matches_oracle(gpu, hw):
+    """The mean over rows whose width is no multiple of 8, and over views at
+    every byte offset, on the matrix cores: against the oracle, and no further
+    from it than a float32 kernel's rounding (1e-7: 11 + 11 float32 taps and the
+    formula, each 2^-24, averaged over the pixels); a view gives its copy's bits."""
+    h, w = hw
+    a, b = u8_pair((2, 2, h, w), 8.0, seed=h * 7 + w)
+    x, y = torch.from_numpy(a).to(gpu), torch.from_numpy(b).to(gpu)
+    got = fa.ssim(x, y, data_range=255.0, reduction="none").cpu().numpy()
+    want = np.array([ref.ssim(a[i], b[i], 255.0) for i in range(2)])
+    assert np.abs(got - want).max() <= 1e-7 * np.abs(want).max()
+    assert float(fa.ssim(x, y, data_range=255.0)) == pytest.approx(got.mean(), rel=1e-12)
+    for left, right, top in ((1, 0, 0), (2, 1, 1), (3, 0, 2), (0, 3, 0)):
+        if w - left - right < 16 or h - top < 11:
+            continue
+        xv, yv = x[..., top:, left:w - right], y[..., top:, left:w - right]
+        v = fa.ssim(xv, yv, data_range=255.0, reduction="none")
+        c = fa.ssim(xv.contiguous(), yv.clone(memory_format=torch.contiguous_format),
+                    data_range=255.0, reduction="none")
+        if (w - left - right) % 8 == 0:  # the copy's rows are aligned: the other kernel
+            assert torch.allclose(v, c, rtol=2e-7, atol=0)
+        else:
+            assert torch.equal(v, c)
+
+
+@pytest.mark.parametrize("shape", [(2, 3, 433, 421), (1, 3, 592, 600), (1, 1, 1030, 1031),
+                                   (3, 3, 362, 363), (1, 3, 591, 1912)])
+@pytest.mark.parametrize("scales", [3, 4, 5])
+def test_ragged_ms_ssim_matches_oracle(gpu, shape, scales):
+    """Three launches over a pyramid whose rows are no multiples of 8 (padded
+    levels), against the oracle and the per-scale path; called twice, so that the
+    second call reads padding the first one left behind."""
+    from frame_analytics_amd import backend
+
+    w = (0.0448, 0.2856, 0.3001, 0.2363, 0.1333)[:scales]
+    a, b = u8_pair(shape, 9.0, seed=scales)
+    x, y = torch.from_numpy(a).to(gpu), torch.from_numpy(b).to(gpu)
+    want = ref.ms_ssim(a, b, 255.0, weights=w)
+    n = dict(backend.native_calls)
+    for fill in (0xFF, 0x7F):  # NaN patterns in whatever the workspace reuses
+        junk = torch.full((1 << 24,), fill, dtype=torch.uint8, device=gpu)
+        del junk
+        got = float(fa.ms_ssim(x, y, data_range=255.0, weights=w))
+        assert abs(got - want) <= 2e-7 * abs(want)
+    assert backend.native_calls["fa_gpu_ms_ssim"] == n.get("fa_gpu_ms_ssim", 0) + 2
