@@ -201,6 +201,29 @@ struct DeviceScope {
   }
 };
 
+// The relative time of a launch of `wgs` equal workgroups that each walk `rows`
+// rows (their own plus what a workgroup pays once, in rows) on `cus` compute
+// units that hold `occ` of them each: what the SSIM planners minimise over the
+// chunk heights.
+//
+// These kernels are bound by the vector ALU, which a compute unit's workgroups
+// share, so what counts is how many workgroups a unit runs in all, k = wgs / cus,
+// not how many rounds of resident ones the launch makes.  Up to `even` per unit
+// they all start at once and the fullest unit sets the time (k rounded up);
+// beyond that the dispatcher evens them out, to `tail` workgroups.  A unit with
+// fewer than the kernel's occupancy hides less latency: with 1, 2 and 3 waves per
+// SIMD of a kernel that takes more it reaches `rate` of its full rate.
+struct WalkFit {
+  int even;
+  double tail, rate[3];
+};
+inline double walk_cost(const WalkFit& f, int64_t wgs, int64_t cus, int occ, double rows) {
+  const int64_t up = (wgs + cus - 1) / cus;
+  const double load = up <= f.even ? static_cast<double>(up)
+                                   : static_cast<double>(wgs) / static_cast<double>(cus) + f.tail;
+  return load * rows / (up <= 3 && up < occ ? f.rate[up - 1] : 1.0);
+}
+
 // Compute-unit count of `device`, cached: the attribute query costs as much
 // as a small kernel.
 int cu_count(int device);

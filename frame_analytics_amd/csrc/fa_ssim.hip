@@ -40,12 +40,10 @@ enum { MODE_REDUCE = 0, MODE_MAP = 1, MODE_CS = 2, MODE_PREP = 3, MODE_PREP_CS =
 
 // Output rows per workgroup (TH), a multiple of 4 up to 128.  A workgroup
 // walks its rows in sequence and re-reads K-1 halo rows, so a launch trades
-// rounds of resident workgroups against rows per workgroup (tiling_for):
-// configs of many large frames take long chunks (configs[1]: TH = 68, 3072
-// workgroups = 3 rounds of 1024), while single frames,
-// the coarse MS-SSIM scales and small crops get the parallelism back, and the
-// float64 backward kernels (one workgroup per CU) are cut only as fine as
-// they can use.  Every TH is a multiple of the phase height and even, so
+// the rows a workgroup pays besides its own against an even load of the compute
+// units (tiling_for): batches of large frames take long chunks, while single
+// frames, the coarse MS-SSIM scales and small crops get the parallelism back.
+// Every TH is a multiple of the phase height and even, so
 // pyramid row pairs never straddle two chunks.  The partial buffers are
 // sized for the smallest TH (the *_workspace queries) and a launch uses the
 // first strips * chunks slots of each plane.
@@ -62,28 +60,35 @@ struct Tiling {
   int TH, strips, tiles;  // tiles = strips * chunks, per plane
 };
 
-// The tiling of one launch over `planes` planes of an out_H x out_W grid
-// when the chip holds `resident` workgroups at once: the TH that minimises
-// rounds x work per workgroup, ceil(wgs / resident) * (TH + (K + 1) / 2),
-// in output rows; ties keep the larger TH.  A halo row only forms its
-// moments, so the K - 1 halo rows and the set-up weigh about half as much as
-// the output rows.  Measured on MI355X (TH any multiple of 4 up to 128):
-//                           charged TH+K+1   TH+(K+1)/2   (64/32/16/8/4, TH+K+1)
-//   configs[1] kernel         156.7 us        147.4         147.6
-//   1x3x1080x1920 call         27.6            27.6          30.4
-//   MS-SSIM configs[4] call   274.4           264.4         264.5
-//   MS-SSIM loss step        1887            1848          1920
-// (Charging a partial round only its share was measured slower: MS-SSIM
-// 301 vs 291 us, the float64 backward 155 vs 133 us.)
-inline Tiling tiling_for(int64_t planes, int out_H, int out_W, int K, int64_t resident) {
+// The tiling of one launch over `planes` planes of an out_H x out_W grid on
+// `cus` compute units that hold `occ` workgroups each: the TH of least cost, ties
+// to the larger.
+//
+// float32 kernels (4 waves per SIMD): walk_cost, with the halo rows and the set-up
+// of a workgroup at a third of K + 1 output rows.  Fitted to sweeps of TH over 19
+// forward launches (128 x 128 patches to eight RGB 1080p frames): the pick is 1.4 %
+// slower than the best TH on average, rounds of resident workgroups were 4 %
+// and up to 18 % (fa.ssim on a 1021 x 1357 luma plane 17.8 -> 15 us, on 1 x 3 x
+// 512 x 512 float32 13.3 -> 12.1, on 8 x 3 x 1080 x 1920 164 -> 157).
+//
+// float64 kernels (2 or 3): rounds of resident workgroups x (TH + (K + 1) / 2); a
+// halo row only forms its moments, so the K - 1 halo rows weigh about half.
+// Over 26 launches of the training pass and the scatter that pick is 0.7 % off
+// the best, and no fit of walk_cost improved every one of them.
+constexpr WalkFit STRIP_FIT = {4, 0.5, {0.55, 0.85, 0.92}};
+
+inline Tiling tiling_for(int64_t planes, int out_H, int out_W, int K, int64_t cus, int occ,
+                         bool f64) {
   Tiling best = {0, 0, 0};
-  int64_t best_cost = INT64_MAX;
+  double best_cost = 0.0;
   for (int th = SSIM_TH_MAX; th >= SSIM_TH_MIN; th -= SSIM_TH_STEP) {
     int strips = 0, chunks = 0;
     strip_grid(out_H, out_W, K, th, &strips, &chunks);
     const int64_t wgs = planes * strips * chunks;
-    const int64_t cost = ((wgs + resident - 1) / resident) * (th + (K + 1) / 2);
-    if (cost < best_cost) {
+    const double cost =
+        f64 ? static_cast<double>((wgs + cus * occ - 1) / (cus * occ) * (th + (K + 1) / 2))
+            : walk_cost(STRIP_FIT, wgs, cus, occ, th + static_cast<double>(K + 1) / 3.0);
+    if (best.TH == 0 || cost < best_cost) {
       best_cost = cost;
       best = Tiling{th, strips, strips * chunks};
     }
@@ -938,9 +943,9 @@ static bool strip_plan_ok(SsimArgs& a) {
 // Tiles `kern` over `planes` planes of an out_H x out_W grid for its
 // occupancy `occ` and launches it; a.TH / a.strips / a.bpp report the tiling.
 template <typename Args>
-static int launch_strips(void (*kern)(Args), int occ, Args& a, int64_t planes, int out_H,
-                         int out_W, int K, int device, hipStream_t st) {
-  const Tiling t = tiling_for(planes, out_H, out_W, K, static_cast<int64_t>(cu_count(device)) * occ);
+static int launch_strips(void (*kern)(Args), int occ, bool f64, Args& a, int64_t planes,
+                         int out_H, int out_W, int K, int device, hipStream_t st) {
+  const Tiling t = tiling_for(planes, out_H, out_W, K, cu_count(device), occ, f64);
   a.TH = t.TH;
   a.strips = t.strips;
   a.bpp = t.tiles;
@@ -957,8 +962,8 @@ template <typename T, typename CT, int MODE, int KW, bool LUMA>
 static int launch_ssim_kw(SsimArgs& a, int64_t planes, int device, hipStream_t st) {
   static const int occ =
       occupancy_wgs(reinterpret_cast<const void*>(&ssim_kernel<T, CT, MODE, KW, LUMA>));
-  return launch_strips(ssim_kernel<T, CT, MODE, KW, LUMA>, occ, a, planes, a.Hout, a.Wout,
-                       KW, device, st);
+  return launch_strips(ssim_kernel<T, CT, MODE, KW, LUMA>, occ, sizeof(CT) == 8, a, planes,
+                       a.Hout, a.Wout, KW, device, st);
 }
 
 template <typename T, typename CT, int MODE, bool LUMA = false>
@@ -997,7 +1002,7 @@ static int launch_ssim(int dtype, int K, bool luma, SsimArgs& a, int64_t planes,
 template <typename T, int KW, bool DY>
 static int launch_scatter_kw(ScatterArgs& a, int64_t planes, int device, hipStream_t st) {
   static const int occ = occupancy_wgs(reinterpret_cast<const void*>(&scatter_kernel<T, KW, DY>));
-  return launch_strips(scatter_kernel<T, KW, DY>, occ, a, planes, a.H, a.W, KW, device, st);
+  return launch_strips(scatter_kernel<T, KW, DY>, occ, true, a, planes, a.H, a.W, KW, device, st);
 }
 
 template <typename T, bool DY>
