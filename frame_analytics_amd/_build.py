@@ -17,6 +17,7 @@ import concurrent.futures as _cf
 import os
 import shutil
 import subprocess
+import sysconfig
 from pathlib import Path
 from typing import List, Sequence
 
@@ -29,6 +30,8 @@ LIBNAME = "libfa_gpu.so"
 CPU_LIBNAME = "libfa_cpu.so"
 # measurement only: the read-bandwidth ceiling kernel bench.py reports
 READBW_LIBNAME = "libfa_readbw.so"
+# the Python extension module that calls the GPU library's entry points
+CALL_NAME = "_fa_call"
 
 
 def library_path() -> Path:
@@ -41,6 +44,14 @@ def cpu_library_path() -> Path:
 
 def readbw_library_path() -> Path:
     return LIBDIR / READBW_LIBNAME
+
+
+def call_module_path() -> Path:
+    return LIBDIR / f"{CALL_NAME}.so"
+
+
+def call_sources() -> List[Path]:
+    return sorted((CSRC / "host").glob("*.cpp"))
 
 
 def cpu_sources() -> List[Path]:
@@ -118,10 +129,24 @@ def build_cpu(verbose: bool = False) -> Path:
     return out
 
 
+def build_call(verbose: bool = False) -> Path:
+    """Compile the extension module ``_fa_call`` (plain CPython C API, links
+    nothing of its own); returns its path."""
+    LIBDIR.mkdir(exist_ok=True)
+    out = call_module_path()
+    tmp = out.with_name(f".{out.name}.{os.getpid()}.tmp")
+    _run([cxx(), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", f"-I{INCLUDE}",
+          f"-I{sysconfig.get_paths()['include']}", *map(str, call_sources()), "-o", str(tmp)],
+         verbose)
+    os.replace(tmp, out)
+    return out
+
+
 def build(verbose: bool = False, jobs: int = 0) -> Path:
     """Compile every kernel source and link ``libfa_gpu.so`` (and build
-    ``libfa_cpu.so``); returns the GPU library's path."""
+    ``libfa_cpu.so`` and ``_fa_call``); returns the GPU library's path."""
     build_cpu(verbose)
+    build_call(verbose)
     cc = hipcc()
     objdir = PKG / "_build"
     objdir.mkdir(exist_ok=True)
@@ -154,7 +179,8 @@ def build(verbose: bool = False, jobs: int = 0) -> Path:
 
 def is_stale() -> bool:
     """True when a library is missing or older than any source or header."""
-    for lib, srcs in ((library_path(), sources()), (cpu_library_path(), cpu_sources())):
+    for lib, srcs in ((library_path(), sources()), (cpu_library_path(), cpu_sources()),
+                      (call_module_path(), call_sources())):
         if not lib.exists():
             return True
         t = lib.stat().st_mtime

@@ -69,6 +69,7 @@ class _Native:
         self.gpu: Any = None
         self.gpu_origin: Optional[str] = None
         self.gpu_error: Optional[str] = None
+        self.callers: dict = {}  # entry point -> _fa_call callable
 
     @property
     def has_gpu(self) -> bool:
@@ -104,6 +105,7 @@ def load(force: bool = False) -> Optional[_Native]:
     native = _Native()
     try:
         native.gpu, native.gpu_origin = _cabi.load_gpu()
+        native.callers = _cabi.load_callers(native.gpu)
     except Exception as exc:
         _load_error = f"{type(exc).__name__}: {exc}"
         raise RuntimeError(
@@ -190,23 +192,31 @@ def _contig(t: torch.Tensor) -> torch.Tensor:
     return t if t.is_contiguous() else t.contiguous()
 
 
+_int64x3 = ctypes.c_int64 * 3
+
+
 def _view_strides(t: torch.Tensor):
     """``(tensor, strides)``: a unit-column-stride view passes its (image,
     channel, row) strides as an int64[3] host array; anything else is copied
     contiguous and passes null."""
     if t.is_contiguous():
         return t, None
-    if t.stride(-1) != 1 or min(t.stride()) < 0:
+    s = t.stride()
+    if s[3] != 1 or min(s) < 0:
         return t.contiguous(), None
-    return t, (ctypes.c_int64 * 3)(t.stride(0), t.stride(1), t.stride(2))
+    return t, _int64x3(s[0], s[1], s[2])
+
+
+@functools.lru_cache(maxsize=64)
+def _luma_array(luma: tuple):
+    kr, kg, kb, off = (luma + (0.0,))[:4]
+    return (ctypes.c_double * 4)(float(kr), float(kg), float(kb), float(off))
 
 
 def _luma_arg(luma: Optional[tuple]):
-    """{kr, kg, kb, offset} as a double[4] host array, or None."""
-    if luma is None:
-        return None
-    kr, kg, kb, off = (tuple(luma) + (0.0,))[:4]
-    return (ctypes.c_double * 4)(float(kr), float(kg), float(kb), float(off))
+    """{kr, kg, kb, offset} as a double[4] host array (read only, one per
+    convention and range), or None."""
+    return None if luma is None else _luma_array(tuple(luma))
 
 
 def _ptr(t: Optional[torch.Tensor]):
@@ -235,10 +245,17 @@ def call_gpu(name: str, *args) -> int:
 
     Every GPU launch of this package goes through here, so
     :data:`native_calls` counts them."""
-    ext = load()
-    if ext is None or not ext.has_gpu:
+    ext = _ext if _ext is not None else load()
+    if ext is None or ext.gpu is None:
         raise RuntimeError(f"{name}: the gfx950 kernel library is not loaded")
-    code = getattr(ext.gpu, name)(*args)
+    fast = ext.callers.get(name)
+    if fast is None:
+        code = getattr(ext.gpu, name)(*args)
+    else:
+        try:
+            code = fast(*args)
+        except TypeError:  # an argument only ctypes takes (byref, a ctypes scalar)
+            code = getattr(ext.gpu, name)(*args)
     native_calls[name] += 1
     return int(code)
 
@@ -322,8 +339,8 @@ def _gpu_ext(x: torch.Tensor) -> Optional[_Native]:
     """The loaded library when ``x`` lives on the GPU, else ``None``."""
     if not x.is_cuda:
         return None
-    ext = load()
-    if ext is None or not ext.has_gpu:
+    ext = _ext if _ext is not None else load()
+    if ext is None or ext.gpu is None:
         return None
     return ext
 
@@ -429,7 +446,7 @@ def pixel_gpu(ext: _Native, x: torch.Tensor, y: torch.Tensor, *, op: int,
     (cropped) views and ``luma`` = (kr, kg, kb, offset) go through
     ``fa_gpu_pixel_reduce_ex``, which reads them in place."""
     del ext  # the library is reached through call_gpu
-    n, c, h, w = (int(v) for v in x.shape)
+    n, c, h, w = x.shape
     x, xs = _view_strides(x)
     y, ys = _view_strides(y)
     per = c * h * w
@@ -438,14 +455,19 @@ def pixel_gpu(ext: _Native, x: torch.Tensor, y: torch.Tensor, *, op: int,
     out = _f64(x.device, n) if per_image else _f64(x.device)
     # the four ABI sinks, in order: mean per image, mean total, dB per image,
     # dB total; exactly one is written
-    slot = (2 if psnr_bias != _PSNR_NONE else 0) + (0 if per_image else 1)
-    sinks = [_ptr(out) if i == slot else None for i in range(4)]
+    po = out.data_ptr()
+    if psnr_bias != _PSNR_NONE:
+        sinks = (None, None, po, None) if per_image else (None, None, None, po)
+    else:
+        sinks = (po, None, None, None) if per_image else (None, po, None, None)
     if luma is None and xs is None and ys is None:
         acc = _acc_for("pixel", x.device, dev, stream) if x.dtype == torch.uint8 else None
 
+        head = (x.data_ptr(), y.data_ptr(), _DTYPE_CODE[x.dtype], n, per, op, param, psnr_bias)
+        tail = (bpi, _ptr(acc), *sinks, dev, stream)
+
         def args(partial):
-            return (_ptr(x), _ptr(y), _DTYPE_CODE[x.dtype], n, per, op, float(param),
-                    float(psnr_bias), partial, bpi, _ptr(acc), *sinks, dev, stream)
+            return (*head, partial, *tail)
 
         if acc is None:
             _run("fa_gpu_pixel_reduce_once", *args(_ptr(_f64(x.device, n, bpi))))
@@ -646,7 +668,7 @@ def _ssim_native(x: torch.Tensor, y: torch.Tensor, *, win_size: int, sigma: floa
     ext = _gpu_ext(x)
     if ext is None or not _usable(x, y) or win_size not in _WINDOWS:
         return None
-    n, c, h, w = (int(v) for v in x.shape)
+    n, c, h, w = x.shape
     if luma is not None and c != 3:
         return None
     from .functional import gaussian_window_1d
@@ -666,7 +688,7 @@ def _ssim_native(x: torch.Tensor, y: torch.Tensor, *, win_size: int, sigma: floa
         per_image = _f64(x.device, n)
     else:
         total = _f64(x.device)
-    head = (_ptr(x), _ptr(y), _DTYPE_CODE[x.dtype], n, c, h, w)
+    head = (x.data_ptr(), y.data_ptr(), _DTYPE_CODE[x.dtype], n, c, h, w)
 
     def tail(partial):
         return (_ptr(win), win_size, float(shift), float(C1), float(C2), _ptr(smap), partial,
@@ -674,11 +696,11 @@ def _ssim_native(x: torch.Tensor, y: torch.Tensor, *, win_size: int, sigma: floa
 
     if smap is None:
         acc = _acc_for("ssim", x.device, dev, stream)
-        lw = _luma_arg(luma)
+        head = (*head, xs, ys, _luma_arg(luma), win.data_ptr(), win_size, shift, C1, C2, None)
+        end = (bpp, _ptr(acc), _ptr(per_image), _ptr(total), dev, stream)
 
         def args(partial):
-            t = tail(partial)
-            return (*head, xs, ys, lw, *t[:8], _ptr(acc), *t[8:])
+            return (*head, partial, *end)
 
         if acc is None:
             _run("fa_gpu_ssim_once", *args(_ptr(_f64(x.device, planes, bpp))))

@@ -22,6 +22,8 @@ from typing import Optional, Sequence, Tuple
 import torch
 import torch.nn.functional as F
 
+from . import backend
+
 __all__ = [
     "mse",
     "psnr",
@@ -179,8 +181,6 @@ def _check_reduction(reduction: str) -> None:
 
 
 def _sum_sq(x, y, dtype, per_image):
-    from . import backend
-
     backend.note_portable("mse", x)
     d = x.to(dtype) - y.to(dtype)
     if per_image:
@@ -199,8 +199,6 @@ def mse(x: torch.Tensor, y: torch.Tensor, *, reduction: str = "mean",
     wdt = _work_dtype(x4, dtype)
     _check_reduction(reduction)
     per_image = reduction == "none"
-    from . import backend
-
     # luma is formed inside the kernel and crops are read in place
     fast = backend.try_mse(x4, y4, per_image=per_image, dtype=out_dtype,
                            luma=_luma_arg_checked(x4, mode, L))
@@ -222,8 +220,6 @@ def psnr(x: torch.Tensor, y: torch.Tensor, *, data_range: Optional[float] = None
     _check_reduction(reduction)
     x4, y4, L, mode = _prep(x, y, luma, crop_border, data_range)
     bias = 10.0 * math.log10(L * L)
-    from . import backend
-
     if not eps:
         # the dB conversion happens inside the reduction's finalize kernel, the
         # luma plane inside the reduction, and crops are read in place
@@ -254,7 +250,7 @@ def gaussian_window_1d(win_size: int = 11, sigma: float = 1.5, *, device=None,
     normalised 2-D window.  Cached per (size, sigma, device, dtype) so that no
     call after the first performs a host-to-device copy.
     """
-    key = (int(win_size), float(sigma), str(device), dtype)
+    key = (win_size, sigma, device, dtype)
     w = _window_cache.get(key)
     if w is None:
         half = (win_size - 1) / 2.0
@@ -278,8 +274,6 @@ def _moments_filtered(x4, y4, win, wdt, shift):
 
     Returns a tuple of five (N, C, H-K+1, W-K+1) tensors.
     """
-    from . import backend
-
     backend.note_portable("ssim_moments", x4)
     xs = x4.to(wdt) - shift
     ys = y4.to(wdt) - shift
@@ -349,8 +343,6 @@ class _NativeSSIM(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, y, win, consts, form, pool_dtype, use=None):
-        from . import backend
-
         shift, C1, C2 = consts
         ctx.set_materialize_grads(False)
         ctx.save_for_backward(x, y, win)
@@ -379,8 +371,6 @@ class _NativeSSIM(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, *grads):
-        from . import backend
-
         _reject_double_backward()
         need_dx, need_dy = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
         nothing = (None,) * 7
@@ -438,8 +428,6 @@ def ssim(x: torch.Tensor, y: torch.Tensor, *, data_range: Optional[float] = None
     wdt = _work_dtype(x4, dtype)
     C1 = (float(K[0]) * L) ** 2
     C2 = (float(K[1]) * L) ** 2
-    from . import backend
-
     # Inference on the GPU: the kernel forms the luma plane and reads crops in
     # place, so neither is materialised first.
     grad = torch.is_grad_enabled() and (x4.requires_grad or y4.requires_grad)
@@ -550,8 +538,6 @@ class _MsHead(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, weights, per_image, *terms):
-        from . import backend
-
         ctx.save_for_backward(*terms)
         ctx.weights, ctx.per_image = weights, per_image
         ctx.set_materialize_grads(False)
@@ -559,8 +545,6 @@ class _MsHead(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, g):
-        from . import backend
-
         _reject_double_backward()
         terms = ctx.saved_tensors
         needs = ctx.needs_input_grad[2:]
@@ -582,8 +566,6 @@ def _combine_scales(terms, weights, device) -> torch.Tensor:
 
 def _ssim_cs_pair(x4, y4, win, wdt, shift, C1, C2, backend_hint):
     """``(ssim, cs)`` plane means, each ``(N, C)``."""
-    from . import backend
-
     n, c = x4.shape[0], x4.shape[1]
     if (backend_hint != "torch" and (x4.requires_grad or y4.requires_grad)
             and torch.is_grad_enabled()
@@ -628,8 +610,6 @@ def ms_ssim(x: torch.Tensor, y: torch.Tensor, *, data_range: Optional[float] = N
         raise ValueError(
             f"image {tuple(x4.shape[-2:])} is too small for {scales} scales with a "
             f"{win_size}x{win_size} window; needs at least {need} px on a side")
-
-    from . import backend
 
     win = gaussian_window_1d(win_size, sigma, device=x4.device, dtype=wdt)
     terms = []
@@ -719,8 +699,6 @@ def _prewitt_bank(device: str, dtype: torch.dtype) -> torch.Tensor:
 
 
 def _gms_map(x4, y4, wdt, T, eps, downsample):
-    from . import backend
-
     backend.note_portable("gms_map", x4)
     xf, yf = x4.to(wdt), y4.to(wdt)
     if downsample:
@@ -743,8 +721,6 @@ class _FusedGMSD(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, y, T, eps, downsample):
-        from . import backend
-
         mean, std = backend.gmsd_stats_fwd(x, y, T, eps, downsample)
         ctx.save_for_backward(x, y, mean, std)
         ctx.consts = (T, eps, downsample)
@@ -753,8 +729,6 @@ class _FusedGMSD(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, g_mean, g_std):
-        from . import backend
-
         _reject_double_backward()
         x, y, mean, std = ctx.saved_tensors
         T, eps, downsample = ctx.consts
@@ -778,16 +752,12 @@ def _gmsd_common(x, y, data_range, T, eps, downsample, dtype, luma, crop_border,
     if backend_hint != "torch" and grad and not return_map:
         # training: luma (if any) is an autograd op in front, then the native
         # statistics with a float64 backward
-        from . import backend
-
         xl, yl = _apply_luma(x4, y4, mode, L, wdt)
         if xl.dtype in (torch.float16, torch.bfloat16):
             xl, yl = xl.float(), yl.float()
         if backend.gmsd_autograd_available(xl, yl):
             return None, _FusedGMSD.apply(xl, yl, Tv, ev, downsample)
     if backend_hint != "torch":
-        from . import backend
-
         # The kernel forms the luma plane itself (its offset cancels out of
         # every gradient) and reads crops in place; its statistics are
         # float64-accurate, so a float64 working dtype needs no other path.
@@ -807,8 +777,7 @@ def _gmsd_common(x, y, data_range, T, eps, downsample, dtype, luma, crop_border,
             raise RuntimeError("native GMSD backend unavailable for these inputs")
     x4, y4 = _apply_luma(x4, y4, mode, L, wdt)
     if mode is not None and backend_hint != "torch" and not return_map:
-        from . import backend  # host kernels: luma formed here
-
+        # host kernels: luma formed here
         fast = backend.try_gmsd(x4, y4, T=Tv, eps=ev, downsample=downsample)
         if fast is not None:
             return None, fast
@@ -880,8 +849,6 @@ def _pixel_loss(name, x, y, param, reduction, dtype, out_dtype, luma, crop_borde
     x4, y4, L, mode = _prep(x, y, luma, crop_border, None)
     wdt = _work_dtype(x4, dtype)
     per_image = reduction == "none"
-    from . import backend
-
     if backend_hint != "torch":
         fast = backend.try_pixel(x4, y4, op=_PIXEL_OPS[name], param=param,
                                  per_image=per_image, dtype=out_dtype,

@@ -1,0 +1,71 @@
+"""The extension module that calls libfa_gpu.so (csrc/host/fa_call.cpp) against
+ctypes on the same library: refusals the library makes before any HIP call, so no
+GPU is needed."""
+
+from __future__ import annotations
+
+import ctypes
+
+import pytest
+
+from frame_analytics_amd import _build, _cabi
+
+if not _build.library_path().exists():  # pragma: no cover
+    pytest.skip("libfa_gpu.so is not built", allow_module_level=True)
+
+
+@pytest.fixture(scope="module")
+def both():
+    lib, _ = _cabi.load_gpu()
+    callers = _cabi.load_callers(lib)
+    assert callers, "the extension module did not load"
+    return lib, callers
+
+
+def _null_args(name):
+    """One refused call: null pointers, zero sizes."""
+    kinds, _ = _cabi.SIGNATURES[name]
+    return [None if k is ctypes.c_void_p else 0.5 if k is ctypes.c_double else 0 for k in kinds]
+
+
+def test_statuses_match_ctypes(both):
+    lib, callers = both
+    for name, fast in callers.items():
+        args = _null_args(name)
+        want = getattr(lib, name)(*args)
+        assert want != 0 and fast(*args) == want, name
+
+
+def test_arguments_reach_their_places(both):
+    """Each of these refusals depends on one argument after doubles, arrays and
+    addresses: a shifted or narrowed argument gives another status."""
+    lib, callers = both
+    fast = callers["fa_gpu_ssim_once"]
+    buf = ctypes.create_string_buffer(4096)
+    p = ctypes.addressof(buf)
+    strides = (ctypes.c_int64 * 3)(3 * 64 * 64, 64 * 64, 32)  # rows of 64 overlap
+    luma = (ctypes.c_double * 4)(0.3, 0.6, 0.1, 0.0)
+
+    def args(xs=None, lw=None, k=11, bpp=None, c=1):
+        n = ctypes.c_int(0)
+        assert lib.fa_gpu_ssim_workspace(64, 64, 11, ctypes.byref(n)) == 0
+        return (p, p, 0, 1, c, 64, 64, xs, None, lw, p, k, 127.5, 6.5, 58.5, None, p,
+                n.value if bpp is None else bpp, None, p, p, 0, None)
+
+    for kw in ({"xs": strides}, {"lw": luma}, {"k": 4}, {"bpp": 1}, {"c": 0}, {"c": -1}):
+        want = lib.fa_gpu_ssim_once(*args(**kw))
+        assert want > 0 and fast(*args(**kw)) == want, kw
+
+
+def test_wrong_arguments_raise(both):
+    _, callers = both
+    fast = callers["fa_gpu_gmsd_backward"]
+    args = _null_args("fa_gpu_gmsd_backward")
+    with pytest.raises(TypeError):
+        fast(*args[:-1])
+    with pytest.raises(TypeError):
+        fast(*args, None)
+    with pytest.raises(TypeError):
+        fast("x", *args[1:])
+    with pytest.raises(TypeError):
+        fast(*args[:7], "x", *args[8:])
