@@ -49,7 +49,8 @@ __device__ inline uint4 ld_stream(const uint4* p) {
 }
 __device__ inline uint32_t ld_stream(const uint32_t* p) { return __builtin_nontemporal_load(p); }
 constexpr int PIX_WG_PER_CU = FA_PIX_WG_PER_CU;  // workgroups per CU the grid aims for
-constexpr int PIX_MIN_ELEMS_PER_THREAD = 64;
+constexpr int PIX_MIN_ELEMS_PER_THREAD = 16;   // of the workspace (the views' share of rows)
+constexpr int PIX_GRID_ELEMS_PER_THREAD = 32;  // of the (workgroups, images) grid
 // Images of at least this many elements get the sweep's workspace (bpi = one
 // partial per wave of one workgroup per CU).  At 4 Mi elements one round of
 // the sweep (2 strides of 256 x 512 vectors on a 256-CU part) spans no more
@@ -128,11 +129,82 @@ struct U8Lane {
   }
 };
 
-template <int OP, int V>
+// --------------------------------------------------------------------------
+// The single-launch finish of the exact uint8 sums (fa_gpu_pixel_reduce_once).
+//
+// Each workgroup adds its per-image sums, and its sum over the whole batch,
+// to caller-owned accumulator words with ONE returning device-scope atomic
+// per word that also counts the contribution: a word holds
+// (sum << FIN_COUNT_BITS) + count.  The atomic's return value is the word
+// before this add, so the workgroup whose add brings a word's count to
+// gridDim.x holds that word's complete sum in registers (every other
+// contribution is ordered before its own on that word) and finishes it
+// itself: the mean, the dB, and a reset of the word to zero.  The image words
+// and the batch word are added by different lanes of one instruction, so the
+// call's tail is one atomic round trip.  No fence and no cache write-back is
+// needed: nothing is read except through the returning atomics.  Each word
+// sits on its own 128-byte line.
+//
+// The host allows the form only where every packed sum fits: the batch's
+// n_total * max_term < 2^(64 - FIN_COUNT_BITS), which bounds the images too.
+// --------------------------------------------------------------------------
+constexpr int FIN_COUNT_BITS = 12;  // contributions per word: gridDim.x <= 4095
+constexpr int FIN_STRIDE = 16;      // uint64 words between accumulators (128 bytes)
+constexpr int SWEEP_LDS_IMAGES = 32;  // batches up to this size: waves sum in LDS, and the finish
+static_assert(FA_PIXEL_ACC_WORDS == (SWEEP_LDS_IMAGES + 1) * FIN_STRIDE,
+              "the ABI's accumulator size");
+
+struct SweepFin {
+  uint64_t* acc;  // (n_images + 1) * FIN_STRIDE words, zero on entry and on exit
+  double n_per_image, n_total, psnr_bias;
+  double *out_per_image, *out_total, *out_psnr_per_image, *out_psnr_total;
+};
+
+// Thread-level: adds sum `t` to word `i` (image i, or the batch when i ==
+// n_images), which takes `count` contributions, and finishes the word when this
+// is its last; the word's complete sum is then in *whole and the return is true.
+__device__ inline bool fin_word(const SweepFin& f, int i, int n_images, unsigned count,
+                                uint64_t t, uint64_t* whole = nullptr) {
+  uint64_t* w = f.acc + static_cast<int64_t>(i) * FIN_STRIDE;
+  const uint64_t old = __hip_atomic_fetch_add(w, (t << FIN_COUNT_BITS) + 1u, __ATOMIC_RELAXED,
+                                              __HIP_MEMORY_SCOPE_AGENT);
+  constexpr uint64_t CM = (uint64_t(1) << FIN_COUNT_BITS) - 1;
+  if ((old & CM) + 1u != count) return false;
+  __hip_atomic_store(w, uint64_t(0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (whole) *whole = (old >> FIN_COUNT_BITS) + t;
+  const bool batch = i == n_images;
+  const double v = static_cast<double>((old >> FIN_COUNT_BITS) + t) /
+                   (batch ? f.n_total : f.n_per_image);
+  double* mean = batch ? f.out_total : (f.out_per_image ? f.out_per_image + i : nullptr);
+  double* db = batch ? f.out_psnr_total
+                     : (f.out_psnr_per_image ? f.out_psnr_per_image + i : nullptr);
+  if (mean) *mean = v;
+  if (f.psnr_bias != FA_PSNR_NONE && db) *db = f.psnr_bias - 10.0 * log10(v);
+  return true;
+}
+
+// Whether the call wants a batch value.
+__device__ inline bool fin_wants_total(const SweepFin& f) {
+  return f.out_total || (f.psnr_bias != FA_PSNR_NONE && f.out_psnr_total);
+}
+
+// Thread-level, for a (gridDim.x, images) launch: image `img`'s word takes its
+// gridDim.x workgroups, and the one that completes it adds the image to the
+// batch word, which takes the images (every workgroup adding to the batch word
+// would queue them all on one address, ~12 ns each).
+__device__ inline void fin_image(const SweepFin& f, int img, int n_images, uint64_t t) {
+  uint64_t whole = 0;
+  if (fin_word(f, img, n_images, gridDim.x, t, &whole) && fin_wants_total(f))
+    fin_word(f, n_images, n_images, static_cast<unsigned>(n_images), whole);
+}
+
+// FIN (exact sums): the workgroups finish the call themselves (fin_image).
+template <int OP, int V, bool FIN = false>
 __global__ __launch_bounds__(BLOCK) void pix_u8_kernel(
     const uint8_t* __restrict__ a, const uint8_t* __restrict__ b, int64_t per,
-    int bpi, float param, void* __restrict__ partial) {
+    int bpi, float param, void* __restrict__ partial, SweepFin fin) {
   constexpr bool EXACT = (OP == FA_OP_MSE || OP == FA_OP_L1);
+  static_assert(!FIN || EXACT, "the one-launch finish takes exact sums");
   __shared__ uint64_t s_u[WAVES_PER_BLOCK];
   __shared__ double s_d[WAVES_PER_BLOCK];
 
@@ -209,7 +281,10 @@ __global__ __launch_bounds__(BLOCK) void pix_u8_kernel(
   const int64_t slot = static_cast<int64_t>(img) * bpi + blockIdx.x;
   if constexpr (EXACT) {
     const uint64_t s = block_sum(acc.exact, s_u);
-    if (threadIdx.x == 0) reinterpret_cast<uint64_t*>(partial)[slot] = s;
+    if (threadIdx.x == 0) {
+      if constexpr (FIN) fin_image(fin, img, gridDim.y, s);
+      else reinterpret_cast<uint64_t*>(partial)[slot] = s;
+    }
   } else {
     const double s = block_sum(acc.wide, s_d);
     if (threadIdx.x == 0) reinterpret_cast<double*>(partial)[slot] = s;
@@ -345,7 +420,6 @@ __global__ __launch_bounds__(BLOCK) void pix_float_kernel(
 #endif
 constexpr int SWEEP_UNROLL = FA_SWEEP_UNROLL;  // gridwide strides per round
 constexpr int SWEEP_BLOCK = FA_SWEEP_BLOCK;    // threads per workgroup (one per CU)
-constexpr int SWEEP_LDS_IMAGES = 32;           // batches up to this size sum waves in LDS
 // uint8 batches below this many bytes per tensor take the many-wave shape: 16
 // waves per CU with one 16-byte load in flight each per tensor, against 8
 // waves with two (the same bytes in flight, the same round).  Measured per
@@ -424,55 +498,6 @@ struct VecAcc {
     else return static_cast<uint64_t>(__double_as_longlong(__longlong_as_double(x) + __longlong_as_double(y)));
   }
 };
-
-// --------------------------------------------------------------------------
-// The single-launch finish of the exact uint8 sums (fa_gpu_pixel_reduce_once).
-//
-// Each workgroup adds its per-image sums, and its sum over the whole batch,
-// to caller-owned accumulator words with ONE returning device-scope atomic
-// per word that also counts the contribution: a word holds
-// (sum << FIN_COUNT_BITS) + count.  The atomic's return value is the word
-// before this add, so the workgroup whose add brings a word's count to
-// gridDim.x holds that word's complete sum in registers (every other
-// contribution is ordered before its own on that word) and finishes it
-// itself: the mean, the dB, and a reset of the word to zero.  The image words
-// and the batch word are added by different lanes of one instruction, so the
-// call's tail is one atomic round trip.  No fence and no cache write-back is
-// needed: nothing is read except through the returning atomics.  Each word
-// sits on its own 128-byte line.
-//
-// The host allows the form only where every packed sum fits: the batch's
-// n_total * max_term < 2^(64 - FIN_COUNT_BITS), which bounds the images too.
-// --------------------------------------------------------------------------
-constexpr int FIN_COUNT_BITS = 12;  // contributions per word: gridDim.x <= 4095
-constexpr int FIN_STRIDE = 16;      // uint64 words between accumulators (128 bytes)
-static_assert(FA_PIXEL_ACC_WORDS == (SWEEP_LDS_IMAGES + 1) * FIN_STRIDE,
-              "the ABI's accumulator size");
-
-struct SweepFin {
-  uint64_t* acc;  // (n_images + 1) * FIN_STRIDE words, zero on entry and on exit
-  double n_per_image, n_total, psnr_bias;
-  double *out_per_image, *out_total, *out_psnr_per_image, *out_psnr_total;
-};
-
-// Thread-level: adds workgroup sum `t` to word `i` (image i, or the batch when
-// i == n_images) and finishes the word when this is its last contribution.
-__device__ inline void fin_word(const SweepFin& f, int i, int n_images, uint64_t t) {
-  uint64_t* w = f.acc + static_cast<int64_t>(i) * FIN_STRIDE;
-  const uint64_t old = __hip_atomic_fetch_add(w, (t << FIN_COUNT_BITS) + 1u, __ATOMIC_RELAXED,
-                                              __HIP_MEMORY_SCOPE_AGENT);
-  constexpr uint64_t CM = (uint64_t(1) << FIN_COUNT_BITS) - 1;
-  if ((old & CM) + 1u != gridDim.x) return;
-  __hip_atomic_store(w, uint64_t(0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  const bool batch = i == n_images;
-  const double v = static_cast<double>((old >> FIN_COUNT_BITS) + t) /
-                   (batch ? f.n_total : f.n_per_image);
-  double* mean = batch ? f.out_total : (f.out_per_image ? f.out_per_image + i : nullptr);
-  double* db = batch ? f.out_psnr_total
-                     : (f.out_psnr_per_image ? f.out_psnr_per_image + i : nullptr);
-  if (mean) *mean = v;
-  if (f.psnr_bias != FA_PSNR_NONE && db) *db = f.psnr_bias - 10.0 * log10(v);
-}
 
 // FIN (exact uint8 sums, LDSP only): the workgroup finishes through
 // fin_word instead of writing partials; each wave also keeps its sum over the
@@ -579,18 +604,17 @@ __global__ __launch_bounds__(NT) void pix_sweep_kernel(
       uint64_t t = s_p[i * WPB];
 #pragma unroll
       for (int w = 1; w < WPB; ++w) t = Acc::add_bits(t, s_p[i * WPB + w]);
-      if constexpr (FIN) fin_word(fin, i, n_images, t);
+      if constexpr (FIN) fin_word(fin, i, n_images, gridDim.x, t);
       else reinterpret_cast<uint64_t*>(partial)[static_cast<int64_t>(i) * gridDim.x + blockIdx.x] = t;
     }
     if constexpr (FIN) {
       // the batch word, from a lane of the first wave that no image took
       // (n_images <= SWEEP_LDS_IMAGES < WAVE)
-      const bool any_total = fin.out_total || (fin.psnr_bias != FA_PSNR_NONE && fin.out_psnr_total);
-      if (static_cast<int>(threadIdx.x) == n_images && any_total) {
+      if (static_cast<int>(threadIdx.x) == n_images && fin_wants_total(fin)) {
         uint64_t t = s_all[0];
 #pragma unroll
         for (int w = 1; w < WPB; ++w) t += s_all[w];
-        fin_word(fin, n_images, n_images, t);
+        fin_word(fin, n_images, n_images, gridDim.x, t);
       }
     }
   }
@@ -629,34 +653,40 @@ static int launch_sweep_shape(hipStream_t st, const void* a, const void* b, int6
   return static_cast<int>(G * (NT / WAVE));
 }
 
-// Whether launch_sweep<T, OP> launches (the same tests, nothing launched).
+// Workgroups of the sweep, 0 when it does not apply: one per CU for the
+// workspace's slots (bpi), or, for a single small image whose launch finishes the
+// call itself and so fills no slots, one per 1024 vectors, at most one per CU.
+// (Small images whose slots happened to be a multiple of 16 were walked by one
+// workgroup per 16: 512 x 512 grey 7.8 -> 4.0 us, 3 x 512 x 512 13.9 -> 4.3 and,
+// float32, now on the per-image grid, 47.9 -> 5.5.  Small batches stay on that
+// grid: the walk takes their images one after another, 8 x 3 x 256 x 256 11.1 us
+// against 4.3.)
 template <typename T>
-static bool sweep_applies(const void* a, const void* b, int64_t n_images, int64_t per,
-                          int bpi) {
+static int64_t sweep_grid(const void* a, const void* b, int64_t n_images, int64_t per, int bpi,
+                          int64_t cus, bool fin) {
   constexpr int64_t E = 16 / static_cast<int64_t>(sizeof(T));
   const uintptr_t bases = reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b);
-  if ((bases & 15) != 0 || per % E != 0 || bpi % SWEEP_SLOTS_PER_CU != 0) return false;
+  if ((bases & 15) != 0 || per % E != 0) return 0;
   const int64_t nv = per / E;
+  const bool many = std::is_same<T, uint8_t>::value && per * n_images < SWEEP_MANY_WAVES_BELOW;
+  if (fin && n_images == 1 && per < PIX_SWEEP_MIN_ELEMS) return std::min(cus, nv / SWEEP_MANY_BLOCK);
+  if (per < PIX_SWEEP_MIN_ELEMS || bpi % SWEEP_SLOTS_PER_CU != 0) return 0;
   const int64_t G = bpi / SWEEP_SLOTS_PER_CU;
-  if (std::is_same<T, uint8_t>::value && per * n_images < SWEEP_MANY_WAVES_BELOW)
-    return nv >= G * SWEEP_MANY_BLOCK;
-  return nv >= static_cast<int64_t>(SWEEP_UNROLL) * G * SWEEP_BLOCK;
+  return nv >= G * (many ? SWEEP_MANY_BLOCK : SWEEP_UNROLL * SWEEP_BLOCK) ? G : 0;
 }
 
-// Launch of the sweep when it applies: 16-byte aligned bases, whole vectors
-// per image, bpi a multiple of SWEEP_SLOTS_PER_CU (one workgroup per CU) and
-// at least one round per image.  Returns the partial columns per image it
-// writes, -1 when it finished the call through `fin`, or 0 when it does not
-// apply and nothing was launched.
+// Launch of the sweep when it applies (sweep_grid): 16-byte aligned bases, whole
+// vectors per image and at least one round per image.  Returns the partial
+// columns per image it writes, -1 when it finished the call through `fin`, or 0
+// when it does not apply and nothing was launched.
 template <typename T, int OP>
 static int launch_sweep(hipStream_t st, const void* a, const void* b, int64_t n_images,
-                        int64_t per, int bpi, double param, void* partial,
+                        int64_t per, int bpi, int64_t cus, double param, void* partial,
                         const SweepFin* fin) {
-  constexpr int64_t E = 16 / static_cast<int64_t>(sizeof(T));
-  const uintptr_t bases = reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b);
-  if ((bases & 15) != 0 || per % E != 0 || bpi % SWEEP_SLOTS_PER_CU != 0) return 0;
-  const int64_t nv = per / E;
-  const int64_t G = bpi / SWEEP_SLOTS_PER_CU;
+  const int64_t nv = per * static_cast<int64_t>(sizeof(T)) / 16;
+  const int64_t G =
+      sweep_grid<T>(a, b, n_images, per, bpi, cus, VecAcc<T, OP>::EXACT && fin != nullptr);
+  if (G == 0) return 0;
   if (std::is_same<T, uint8_t>::value && per * n_images < SWEEP_MANY_WAVES_BELOW)
     return launch_sweep_shape<T, OP, 1, SWEEP_MANY_BLOCK>(st, a, b, n_images, nv, G, param,
                                                           partial, fin);
@@ -666,13 +696,13 @@ static int launch_sweep(hipStream_t st, const void* a, const void* b, int64_t n_
 
 template <typename T>
 static int launch_sweep_op(int op, hipStream_t st, const void* a, const void* b,
-                           int64_t n_images, int64_t per, int bpi, double param,
+                           int64_t n_images, int64_t per, int bpi, int64_t cus, double param,
                            void* partial, const SweepFin* fin = nullptr) {
   switch (op) {
-    case FA_OP_MSE: return launch_sweep<T, FA_OP_MSE>(st, a, b, n_images, per, bpi, param, partial, fin);
-    case FA_OP_L1: return launch_sweep<T, FA_OP_L1>(st, a, b, n_images, per, bpi, param, partial, fin);
-    case FA_OP_CHARB: return launch_sweep<T, FA_OP_CHARB>(st, a, b, n_images, per, bpi, param, partial, nullptr);
-    default: return launch_sweep<T, FA_OP_HUBER>(st, a, b, n_images, per, bpi, param, partial, nullptr);
+    case FA_OP_MSE: return launch_sweep<T, FA_OP_MSE>(st, a, b, n_images, per, bpi, cus, param, partial, fin);
+    case FA_OP_L1: return launch_sweep<T, FA_OP_L1>(st, a, b, n_images, per, bpi, cus, param, partial, fin);
+    case FA_OP_CHARB: return launch_sweep<T, FA_OP_CHARB>(st, a, b, n_images, per, bpi, cus, param, partial, nullptr);
+    default: return launch_sweep<T, FA_OP_HUBER>(st, a, b, n_images, per, bpi, cus, param, partial, nullptr);
   }
 }
 
@@ -742,10 +772,14 @@ __global__ __launch_bounds__(BLOCK) void pix_view_kernel(PixView v) {
 // uint8 views: crops at any byte offset, with or without luma.  A row is read
 // as dwords -- realigned with v_alignbyte when it does not start on a 4-byte
 // boundary, since the aligned dword holding any byte of the row is mapped --
-// and a lane issues the loads of VR rows x VQ dwords (rows up to 4 KiB in one
-// step) before it sums any, so enough bytes are in flight: one dword load per
+// and a lane issues the loads of VR rows x VQ dwords before it sums any, so
+// enough bytes are in flight: one dword load per
 // row at a time left this kernel latency bound (a 4-byte aligned crop of
-// configs[2] took 85 us, a byte-offset one 204 us).  With luma the three
+// configs[2] took 85 us, a byte-offset one 204 us).  Each wave takes rows of its
+// own: with the whole workgroup on one row a 1349-byte row filled a third of
+// the lanes of a step and the rows of a small crop followed one another (Y-PSNR
+// of 1 x 3 x 1021 x 1357 14.9 -> 10.2 us, of 64 x 64 91 -> 14; crops of
+// 8 x 3 x 2160 x 3840 by 4 and 1: 83.6 -> 76.2 and 105.6 -> 83.3).  With luma the three
 // channels' dwords are read and kr dR + kg dG + kb dB is formed per pixel in
 // float64 (the luma offset cancels).
 constexpr int PIX_VQ = 4;  // dwords per lane per row and step
@@ -790,7 +824,15 @@ __global__ __launch_bounds__(BLOCK) void pix_view_u8_kernel(PixView v) {
     return pix_term<OP, double>(fma(v.kb, d[2], fma(v.kg, d[1], v.kr * d[0])), pd);
   };
 
-  for (int64_t rr = r0; rr < r1; rr += VR) {  // uniform
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / WAVE);
+  const int lane = static_cast<int>(threadIdx.x) % WAVE;
+  // three channels of a row that fills a step of the whole workgroup: all waves on
+  // one row (8 x 3 x 2160 x 3840 luma: 79.3 us, 81.9 with a row per wave)
+  const bool wide = LUMA && nq >= 3 * BLOCK;
+  const int id = wide ? static_cast<int>(threadIdx.x) : lane;
+  const int span = wide ? BLOCK : WAVE;
+  const int first = wide ? 0 : wave * VR, next = wide ? VR : VR * WAVES_PER_BLOCK;
+  for (int64_t rr = r0 + first; rr < r1; rr += next) {  // uniform in the wave
     const uint8_t* pa[VR][CH];
     const uint8_t* pb[VR][CH];
     uint32_t ma[VR][CH], mb[VR][CH];
@@ -810,17 +852,17 @@ __global__ __launch_bounds__(BLOCK) void pix_view_u8_kernel(PixView v) {
         mb[q][ch] = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(pb[q][ch]) & 3);
       }
     }
-    for (int j0 = 0; j0 < nq; j0 += PIX_VQ * BLOCK) {  // uniform; one step for rows <= 4 KiB
+    for (int j0 = 0; j0 < nq; j0 += PIX_VQ * span) {  // uniform; a step is 1 (4) KiB of a row
       uint32_t xa[VR][PIX_VQ][CH], xb[VR][PIX_VQ][CH];
       uint32_t ha[VR][PIX_VQ][CH], hb[VR][PIX_VQ][CH];  // lane 63's al[j + 1]
       bool ok[VR][PIX_VQ];
-      const bool last_lane = (threadIdx.x & (WAVE - 1)) == WAVE - 1;
+      const bool last_lane = lane == WAVE - 1;
       // every load of the step first ...
 #pragma unroll
       for (int q = 0; q < VR; ++q) {
 #pragma unroll
         for (int u = 0; u < PIX_VQ; ++u) {
-          const int j = j0 + u * BLOCK + static_cast<int>(threadIdx.x);
+          const int j = j0 + u * span + id;
           ok[q][u] = rv[q] && j < nq;
           const bool feed = rv[q] && j == nq;  // loads only for its neighbour
 #pragma unroll
@@ -878,8 +920,8 @@ __global__ __launch_bounds__(BLOCK) void pix_view_u8_kernel(PixView v) {
         lane8.flush();  // at most VR * PIX_VQ = 8 dwords since the last flush
       }
     }
-    if (static_cast<int>(threadIdx.x) < tail) {  // the row's last W % 4 bytes
-      const int j = 4 * nq + static_cast<int>(threadIdx.x);
+    if (id < tail) {  // the row's last W % 4 bytes
+      const int j = 4 * nq + id;
 #pragma unroll
       for (int q = 0; q < VR; ++q) {
         if (rv[q]) {
@@ -1030,18 +1072,51 @@ int launch_finalize(const void* partial, bool exact, int nrows, int ncols,
   return FA_OK;
 }
 
+// Whether a (bpi, n_images) launch of the uint8 kernel finishes the call itself:
+// up to this many workgroups per image queue on its word (~12 ns each) for less
+// than the ~2.3 us the finalize launch costs (8 x 3 x 256 x 256 6.2 -> 4.3 us,
+// 4 x 3 x 511 x 767 7.7 -> 5.9).
+constexpr int U8_FIN_MAX_BPI = 512;
+static bool u8_finishes(int64_t n_images, int cols) {
+  return n_images <= SWEEP_LDS_IMAGES && cols <= U8_FIN_MAX_BPI;
+}
+
+// Workgroups per image of the (cols, n_images) grid, at most the workspace's
+// slots: 32 elements or more per thread, and for small images about 1024 in all (8
+// x 1080 x 1920 grey: 8.5 us with 128 per image, 10.7 with 253, whose adds queue
+// on the image's word).
+static int grid_cols(int64_t n_images, int64_t per, int bpi) {
+  constexpr int64_t per_wg = static_cast<int64_t>(BLOCK) * PIX_GRID_ELEMS_PER_THREAD;
+  int64_t c = std::max<int64_t>(1, (per + per_wg - 1) / per_wg);
+  if (per < PIX_SWEEP_MIN_ELEMS) c = std::min(c, std::max<int64_t>(16, 1024 / n_images));
+  return static_cast<int>(std::min<int64_t>(bpi, c));
+}
+
+template <int OP, bool FIN>
+static void launch_u8_v(int vec, dim3 grid, hipStream_t st, const uint8_t* a, const uint8_t* b,
+                        int64_t per, int bpi, float p, void* partial, const SweepFin& f) {
+  if (vec == 16)
+    hipLaunchKernelGGL((pix_u8_kernel<OP, 16, FIN>), grid, dim3(BLOCK), 0, st, a, b, per, bpi, p, partial, f);
+  else if (vec == 4)
+    hipLaunchKernelGGL((pix_u8_kernel<OP, 4, FIN>), grid, dim3(BLOCK), 0, st, a, b, per, bpi, p, partial, f);
+  else
+    hipLaunchKernelGGL((pix_u8_kernel<OP, 1, FIN>), grid, dim3(BLOCK), 0, st, a, b, per, bpi, p, partial, f);
+}
+
+// True when the launch finished the call itself (exact sums with `fin`).
 template <int OP>
-static void launch_u8(int vec, dim3 grid, hipStream_t st, const void* a,
-                      const void* b, int64_t per, int bpi, float p,
-                      void* partial) {
+static bool launch_u8(int vec, dim3 grid, hipStream_t st, const void* a, const void* b,
+                      int64_t per, int bpi, float p, void* partial, const SweepFin* fin) {
   const uint8_t* ua = static_cast<const uint8_t*>(a);
   const uint8_t* ub = static_cast<const uint8_t*>(b);
-  if (vec == 16)
-    hipLaunchKernelGGL((pix_u8_kernel<OP, 16>), grid, dim3(BLOCK), 0, st, ua, ub, per, bpi, p, partial);
-  else if (vec == 4)
-    hipLaunchKernelGGL((pix_u8_kernel<OP, 4>), grid, dim3(BLOCK), 0, st, ua, ub, per, bpi, p, partial);
-  else
-    hipLaunchKernelGGL((pix_u8_kernel<OP, 1>), grid, dim3(BLOCK), 0, st, ua, ub, per, bpi, p, partial);
+  if constexpr (OP == FA_OP_MSE || OP == FA_OP_L1) {
+    if (fin && u8_finishes(grid.y, bpi)) {
+      launch_u8_v<OP, true>(vec, grid, st, ua, ub, per, bpi, p, partial, *fin);
+      return true;
+    }
+  }
+  launch_u8_v<OP, false>(vec, grid, st, ua, ub, per, bpi, p, partial, SweepFin{});
+  return false;
 }
 
 template <typename T, int OP>
@@ -1118,7 +1193,8 @@ FA_API int fa_gpu_pixel_reduce_once(const void* a, const void* b, int dtype,
   if (op < 0 || op > 3) return FA_E_OP;
   if (n_images <= 0 || n_per_image <= 0 || bpi <= 0) return FA_E_SHAPE;
   if (n_images > 65535 || static_cast<int64_t>(bpi) * BLOCK > INT32_MAX) return FA_E_SHAPE;
-  const dim3 grid(static_cast<unsigned>(bpi), static_cast<unsigned>(n_images));
+  const int cols = grid_cols(n_images, n_per_image, bpi);
+  const dim3 grid(static_cast<unsigned>(cols), static_cast<unsigned>(n_images));
   const uintptr_t rel = reinterpret_cast<uintptr_t>(a) - reinterpret_cast<uintptr_t>(b);
 
   // the one-launch finish: exact uint8 sums, a wanted output, and every
@@ -1145,8 +1221,11 @@ FA_API int fa_gpu_pixel_reduce_once(const void* a, const void* b, int dtype,
     }
   }
   // a null workspace is enough only for the one-launch form
-  if (!partial && !(pfin && sweep_applies<uint8_t>(a, b, n_images, n_per_image, bpi)))
-    return FA_E_ARG;
+  const int64_t cus = cu_count(device);
+  const bool finishes =
+      pfin && (sweep_grid<uint8_t>(a, b, n_images, n_per_image, bpi, cus, true) > 0 ||
+               (n_per_image < PIX_SWEEP_MIN_ELEMS && u8_finishes(n_images, cols)));
+  if (!partial && !finishes) return FA_E_ARG;
   FA_DEVICE_SCOPE(device);
   hipStream_t st = static_cast<hipStream_t>(stream);
 
@@ -1154,17 +1233,17 @@ FA_API int fa_gpu_pixel_reduce_once(const void* a, const void* b, int dtype,
   int swept = 0;  // partial columns per image the sweep wrote, 0 if it did not run
   switch (dtype) {
     case FA_U8:
-      swept = launch_sweep_op<uint8_t>(op, st, a, b, n_images, n_per_image, bpi, param, partial,
-                                       pfin);
+      swept = launch_sweep_op<uint8_t>(op, st, a, b, n_images, n_per_image, bpi, cus, param,
+                                       partial, pfin);
       if (swept < 0) {  // finished inside the sweep
         FA_LAUNCH_CHECK();
         return FA_OK;
       }
       break;
-    case FA_F16: swept = launch_sweep_op<half_t>(op, st, a, b, n_images, n_per_image, bpi, param, partial); break;
-    case FA_BF16: swept = launch_sweep_op<bf16_t>(op, st, a, b, n_images, n_per_image, bpi, param, partial); break;
-    case FA_F32: swept = launch_sweep_op<float>(op, st, a, b, n_images, n_per_image, bpi, param, partial); break;
-    case FA_F64: swept = launch_sweep_op<double>(op, st, a, b, n_images, n_per_image, bpi, param, partial); break;
+    case FA_F16: swept = launch_sweep_op<half_t>(op, st, a, b, n_images, n_per_image, bpi, cus, param, partial); break;
+    case FA_BF16: swept = launch_sweep_op<bf16_t>(op, st, a, b, n_images, n_per_image, bpi, cus, param, partial); break;
+    case FA_F32: swept = launch_sweep_op<float>(op, st, a, b, n_images, n_per_image, bpi, cus, param, partial); break;
+    case FA_F64: swept = launch_sweep_op<double>(op, st, a, b, n_images, n_per_image, bpi, cus, param, partial); break;
     default: return FA_E_DTYPE;
   }
   if (swept) {
@@ -1173,26 +1252,31 @@ FA_API int fa_gpu_pixel_reduce_once(const void* a, const void* b, int dtype,
     const int vec = (rel & 15) == 0 ? 16 : ((rel & 3) == 0 ? 4 : 1);
     const float p = static_cast<float>(param);
     exact = (op == FA_OP_MSE || op == FA_OP_L1);
+    bool done = false;
     switch (op) {
-      case FA_OP_MSE: launch_u8<FA_OP_MSE>(vec, grid, st, a, b, n_per_image, bpi, p, partial); break;
-      case FA_OP_L1: launch_u8<FA_OP_L1>(vec, grid, st, a, b, n_per_image, bpi, p, partial); break;
-      case FA_OP_CHARB: launch_u8<FA_OP_CHARB>(vec, grid, st, a, b, n_per_image, bpi, p, partial); break;
-      default: launch_u8<FA_OP_HUBER>(vec, grid, st, a, b, n_per_image, bpi, p, partial); break;
+      case FA_OP_MSE: done = launch_u8<FA_OP_MSE>(vec, grid, st, a, b, n_per_image, cols, p, partial, pfin); break;
+      case FA_OP_L1: done = launch_u8<FA_OP_L1>(vec, grid, st, a, b, n_per_image, cols, p, partial, pfin); break;
+      case FA_OP_CHARB: launch_u8<FA_OP_CHARB>(vec, grid, st, a, b, n_per_image, cols, p, partial, nullptr); break;
+      default: launch_u8<FA_OP_HUBER>(vec, grid, st, a, b, n_per_image, cols, p, partial, nullptr); break;
+    }
+    if (done) {
+      FA_LAUNCH_CHECK();
+      return FA_OK;
     }
   } else {
     const bool vec = (rel & 15) == 0;
     switch (dtype) {
-      case FA_F16: launch_float_op<half_t>(op, vec, grid, st, a, b, n_per_image, bpi, param, partial); break;
-      case FA_BF16: launch_float_op<bf16_t>(op, vec, grid, st, a, b, n_per_image, bpi, param, partial); break;
-      case FA_F32: launch_float_op<float>(op, vec, grid, st, a, b, n_per_image, bpi, param, partial); break;
-      case FA_F64: launch_float_op<double>(op, vec, grid, st, a, b, n_per_image, bpi, param, partial); break;
+      case FA_F16: launch_float_op<half_t>(op, vec, grid, st, a, b, n_per_image, cols, param, partial); break;
+      case FA_BF16: launch_float_op<bf16_t>(op, vec, grid, st, a, b, n_per_image, cols, param, partial); break;
+      case FA_F32: launch_float_op<float>(op, vec, grid, st, a, b, n_per_image, cols, param, partial); break;
+      case FA_F64: launch_float_op<double>(op, vec, grid, st, a, b, n_per_image, cols, param, partial); break;
       default: return FA_E_DTYPE;
     }
   }
   FA_LAUNCH_CHECK();
 
   const double n_each = static_cast<double>(n_per_image);
-  return launch_finalize(partial, exact, static_cast<int>(n_images), swept ? swept : bpi,
+  return launch_finalize(partial, exact, static_cast<int>(n_images), swept ? swept : cols,
                          n_each, n_each * static_cast<double>(n_images), psnr_bias,
                          out_per_image, out_total, out_psnr_per_image, out_psnr_total, st);
 }

@@ -469,12 +469,13 @@ FA_API int fa_gpu_ssim_noalloc(const void* x, const void* y, int dtype, int N,
  * arguments, same results bit for bit) plus `acc`: FA_PIXEL_ACC_WORDS uint64
  * of device memory that is zero when the call starts and that the call leaves
  * zero when it completes.  Where the sums are exact -- dtype FA_U8, op
- * FA_OP_MSE or FA_OP_L1, contiguous batches the one-workgroup-per-CU sweep
- * takes (images of >= 4 Mi elements, 16-byte aligned), at most 32 images --
- * the sweep finishes the call itself: each workgroup adds its per-image sums
- * to `acc` with returning device-scope atomics, and the workgroup that adds
- * an image's last sum writes that image's outputs (and the batch's, after the
- * batch's last image).  One launch instead of two.  Every other call ignores
+ * FA_OP_MSE or FA_OP_L1, at most 32 contiguous images, either of fewer than
+ * 4 Mi elements (any alignment) or taken by the one-workgroup-per-CU sweep
+ * (larger, 16-byte aligned, `bpi` the workspace query's) -- the launch finishes
+ * the call itself: each workgroup adds its per-image sums to `acc` with
+ * returning device-scope atomics, and the workgroup that adds an image's last
+ * sum writes that image's outputs (and the batch's, after the batch's last
+ * image).  One launch instead of two.  Every other call ignores
  * `acc` (it may be null) and runs as fa_gpu_pixel_reduce.  `acc` is state of
  * one stream: calls that may overlap (two streams) need one buffer each.
  * `partial` may be null for a call that takes the one-launch form (it is not

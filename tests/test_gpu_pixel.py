@@ -444,3 +444,51 @@ def test_single_launch_without_workspace(gpu):
         else:
             assert rc == 5 and bool((out == -1.0).all()), (op, bp, rc)
         assert not bool(acc.any())
+
+
+# One image below the sweep's 4 Mi elements, at the edges of its walk (1024 16-byte
+# vectors a workgroup) and unaligned; batches on the per-image grid, whose last
+# workgroup finishes an image, up to the 32 the accumulator holds and one more.
+@pytest.mark.parametrize("shape,off", [
+    ((1, 1, 1, 16383), 0), ((1, 1, 1, 16384), 0), ((1, 1, 1, 16400), 0), ((1, 1, 1, 5), 0),
+    ((1, 1, 2047, 2049), 0), ((1, 1, 2048, 2047), 0), ((1, 3, 300, 333), 1),
+    ((2, 1, 1, 8192), 0), ((2, 1, 1, 8193), 3), ((32, 1, 37, 53), 0), ((33, 1, 37, 53), 0),
+    ((3, 1, 1500, 1601), 4)])
+def test_small_images_finish_exactly(gpu, shape, off):
+    """uint8 sums are integers: equal to the oracle's bit for bit, per image and
+    for the batch, with the stream's accumulator zero again after each call."""
+    from frame_analytics_amd import backend
+
+    a, b = u8_pair(shape, 9.0, seed=shape[-1] + off)
+    n = a.size
+    xs = torch.zeros(n + 16, dtype=torch.uint8, device=gpu)
+    ys = torch.zeros(n + 16, dtype=torch.uint8, device=gpu)
+    x, y = xs[off:off + n].view(shape), ys[2 * off:2 * off + n].view(shape)
+    x.copy_(torch.from_numpy(a))
+    y.copy_(torch.from_numpy(b))
+    for red in ("none", "mean"):
+        for _ in range(2):
+            assert np.array_equal(fa.mse(x, y, reduction=red).cpu().numpy(), ref.mse(a, b, red))
+            assert np.array_equal(fa.l1(x, y, reduction=red).cpu().numpy(), ref.l1(a, b, red))
+        got = fa.psnr(x, y, data_range=255.0, reduction=red).cpu().numpy()
+        assert np.allclose(got, ref.psnr(a, b, 255.0, red), rtol=1e-12, atol=0)
+    assert not any(bool(w.any()) for k, w in backend._stream_acc.items())
+
+
+@pytest.mark.parametrize("w,luma", [(61, "bt601"), (260, None), (3071, "bt601"),
+                                    (3074, "bt601"), (3079, None)])
+def test_view_rows_per_wave(gpu, w, luma):
+    """uint8 crops whose rows fill less than a wave's step, and luma rows either
+    side of the 3072 samples from which the whole workgroup shares a row; fewer
+    rows than waves and a remainder."""
+    for h in (3, 9, 14):
+        a, b = u8_pair((2, 3, h, w + 2), 9.0, seed=w + h)
+        x, y = _t(a, gpu), _t(b, gpu)
+        ca, cb = ref.crop(a, 1), ref.crop(b, 1)
+        got = fa.mse(x, y, luma=luma, crop_border=1, reduction="none").cpu().numpy()
+        if luma is None:
+            assert np.array_equal(got, ref.mse(ca, cb, "none"))
+        else:
+            want = ref.mse(ref.rgb_to_luma(ca.astype(np.float64), luma),
+                           ref.rgb_to_luma(cb.astype(np.float64), luma), "none")
+            assert np.all(np.abs(got - want) <= 1e-12 * np.abs(want))
