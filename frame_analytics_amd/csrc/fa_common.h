@@ -259,6 +259,45 @@ __device__ inline void row_store(double v, __amdgpu_buffer_rsrc_t r, uint32_t of
   __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2_t, v), r, off, 0, 0);
 }
 
+// A lane's first `n` (0 .. 4) of four consecutive columns from `col`, stored with
+// three instructions for any n: the widest that n fills, the pair and the odd
+// one, each dropped by the bounds check on the lanes that do not need it. (Four
+// dword stores, each lane's 16 bytes from the next, cover the same cache lines four
+// times over.) The offsets do not change along a strip.
+template <typename E>
+struct QuadOff {
+  uint32_t wide, pair, odd;
+  bool odd2;  // the odd one is column 2
+};
+template <typename E>
+__device__ inline QuadOff<E> quad_off(int col, int n) {
+  QuadOff<E> q;
+  // float: 16 bytes of four columns, 8 of two; double: 16 bytes of two, twice
+  q.wide = lane_off<E>(sizeof(E) == 4 ? col : col + 2, n >= 4);
+  q.pair = lane_off<E>(col, sizeof(E) == 4 ? (n == 2 || n == 3) : n >= 2);
+  q.odd2 = n == 3;
+  q.odd = lane_off<E>(q.odd2 ? col + 2 : col, n == 1 || n == 3);
+  return q;
+}
+typedef unsigned int quad_u32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned int quad_u32x2 __attribute__((ext_vector_type(2)));
+__device__ inline void quad_store(const float* v, __amdgpu_buffer_rsrc_t r, const QuadOff<float>& q) {
+  const quad_u32x4 w = {__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]),
+                        __float_as_uint(v[3])};
+  __builtin_amdgcn_raw_buffer_store_b128(w, r, q.wide, 0, 0);
+  __builtin_amdgcn_raw_buffer_store_b64(quad_u32x2{w[0], w[1]}, r, q.pair, 0, 0);
+  __builtin_amdgcn_raw_buffer_store_b32(q.odd2 ? w[2] : w[0], r, q.odd, 0, 0);
+}
+__device__ inline void quad_store(const double* v, __amdgpu_buffer_rsrc_t r, const QuadOff<double>& q) {
+  typedef double f64x2_t __attribute__((ext_vector_type(2)));
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(quad_u32x4, f64x2_t{v[0], v[1]}), r,
+                                         q.pair, 0, 0);
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(quad_u32x4, f64x2_t{v[2], v[3]}), r,
+                                         q.wide, 0, 0);
+  __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(quad_u32x2, q.odd2 ? v[2] : v[0]), r,
+                                        q.odd, 0, 0);
+}
+
 // --------------------------------------------------------------------------
 // The one-launch finish of the SSIM forwards (fa_gpu_ssim_once: the uint8
 // matrix-core kernel and the strip kernel).

@@ -35,8 +35,16 @@ namespace fa {
 // (the SSIM means or the cs means, SsimArgs::unit_s): MS-SSIM's loss reads
 // only one of them at each scale, so the maps the backward needs are these
 // times that plane's upstream gradient, and no coefficient pass runs there.
+// MODE_CSC: MODE_CSF for the cs means and without dy's map, which is every scale
+// but the coarsest of a loss on x: the luminance terms drop out of the maps and
+// a lane's four columns of each are stored at once (quad_store).  The pass is bound
+// by its instructions (74 % of the cycles in MODE_CSF): 8 x 3 x 1080 x 1920 float32
+// 407 -> 347 us, 8 x 3 x 270 x 480 float64 39 -> 36.
 enum { MODE_REDUCE = 0, MODE_MAP = 1, MODE_CS = 2, MODE_PREP = 3, MODE_PREP_CS = 4,
-       MODE_CSF = 5 };
+       MODE_CSF = 5, MODE_CSC = 6 };
+constexpr bool mode_sums_cs(int mode) {
+  return mode == MODE_CS || mode == MODE_CSF || mode == MODE_CSC;
+}
 
 // Output rows per workgroup (TH), a multiple of 4 up to 128.  A workgroup
 // walks its rows in sequence and re-reads K-1 halo rows, so a launch trades
@@ -177,6 +185,8 @@ struct SsimPol {
   CT k1;  // 2 shift^2 + C1
   CT row_s, row_cs;
   double acc_s, acc_cs;
+  QuadOff<float> qoff;  // MODE_CSC: the lane's four columns
+  float qb[COLS_PER_LANE], qc[COLS_PER_LANE], qt[COLS_PER_LANE];
   // MODE_CS pyramid step: this workgroup owns input rows [prow0, prow1) and,
   // on even lanes, the column pair starting at its column (pcol = col / 2)
   void* px;
@@ -218,7 +228,7 @@ struct SsimPol {
   // even lane.  The engine hands both rows of a pair at once, so there is no
   // row-parity branch and no state between calls.
   __device__ inline void pool2(int row, const Raw& a, const Raw& b) {
-    if constexpr (MODE == MODE_CS || MODE == MODE_CSF) {
+    if constexpr (mode_sums_cs(MODE)) {
       // prow1 is even, so row < prow1 covers row + 1 too
       if (!pool_on || row < prow0 || row >= prow1) return;  // uniform
       PA sx = static_cast<PA>(a.x) + static_cast<PA>(b.x);
@@ -295,7 +305,7 @@ struct SsimPol {
   //   A2 = 2 sigma_xy + C2,  sigma_xy = E x'y' - ux uy
   //   B2 = sigma_x^2 + sigma_y^2 + C2 = E (x'-y')^2 + A2 - (ux - uy)^2
   // `valid` masks lanes whose column lies outside the map.
-  __device__ inline void emit(int orow, int ocol, const CT* v, bool valid, const EIn&, int) {
+  __device__ inline void emit(int orow, int ocol, const CT* v, bool valid, const EIn&, int col) {
     const CT ux = v[0];
     const CT uy = v[1];
     const CT p = ux * uy;
@@ -340,6 +350,18 @@ struct SsimPol {
           oty[idx] = static_cast<float>(gS * dmuy - CT(2) * b * uy - c * ux);
         }
       }
+    } else if constexpr (MODE == MODE_CSC) {
+      // gS = 0: b = -gCS cs / B2, c = 2 gCS / B2, tx = -2 b ux - c uy = c (cs ux - uy)
+      const CT inv = CT(1) / (B1 * B2);
+      const CT iB2 = B1 * inv;
+      const CT CS = A2 * iB2;
+      row_s += valid ? A1 * (B2 * inv) * CS : CT(0);
+      row_cs += valid ? CS : CT(0);
+      const CT e = gCS * iB2;
+      const CT c = e + e;
+      qb[col] = static_cast<float>(-e * CS);
+      qc[col] = static_cast<float>(c);
+      qt[col] = static_cast<float>(c * fma(CS, ux, -uy));
     } else if (valid) {
       // the backward coefficients keep their guarded stores: issued on every
       // path (row_store) they measured slower (configs[3] 27.0 -> 32.3 us)
@@ -373,9 +395,20 @@ struct SsimPol {
     }
   }
 
+  // The lane's first output column and how many of its four exist.
+  __device__ inline void set_out(int ocol, int n) {
+    if constexpr (MODE == MODE_CSC) qoff = quad_off<float>(ocol, n);
+  }
+
   // A lane's four outputs of a phase are summed at the compute type, then
-  // folded into the float64 lane total.
-  __device__ inline void end_row() {
+  // folded into the float64 lane total.  `on` (uniform): the row exists.
+  __device__ inline void end_row(int orow, bool on) {
+    if constexpr (MODE == MODE_CSC) {
+      const int64_t o = out_off + static_cast<int64_t>(orow) * Wout;
+      quad_store(qb, row_rsrc(on ? ob + o : nullptr, Wout), qoff);
+      quad_store(qc, row_rsrc(on ? oc + o : nullptr, Wout), qoff);
+      quad_store(qt, row_rsrc(on ? otx + o : nullptr, Wout), qoff);
+    }
     acc_s += static_cast<double>(row_s);
     acc_cs += static_cast<double>(row_cs);
     row_s = CT(0);
@@ -443,7 +476,7 @@ __global__ __launch_bounds__(BLOCK) FA_SSIM_ATTR void ssim_kernel(SsimArgs a) {
     pol.gS = static_cast<CT>(a.gs[plane]) * static_cast<CT>(a.gnorm);
     pol.gCS = static_cast<CT>(a.gcs[plane]) * static_cast<CT>(a.gnorm);
   }
-  if constexpr (MODE == MODE_CSF) {
+  if constexpr (MODE == MODE_CSF || MODE == MODE_CSC) {
     pol.gS = a.unit_s ? static_cast<CT>(a.gnorm) : CT(0);
     pol.gCS = a.unit_s ? CT(0) : static_cast<CT>(a.gnorm);
   }
@@ -455,7 +488,7 @@ __global__ __launch_bounds__(BLOCK) FA_SSIM_ATTR void ssim_kernel(SsimArgs a) {
   pol.px = a.px;
   pol.py = a.py;
   pol.pool_on = false;
-  if constexpr (MODE == MODE_CS || MODE == MODE_CSF) {
+  if constexpr (mode_sums_cs(MODE)) {
     if (a.px) {
       // rows and columns of the output map this workgroup owns, extended to
       // the image edge (2 * floor(H/2), 2 * floor(W/2)) in the last chunk /
@@ -492,7 +525,7 @@ __global__ __launch_bounds__(BLOCK) FA_SSIM_ATTR void ssim_kernel(SsimArgs a) {
   } else if constexpr (MODE == MODE_MAP) {
     const double s = block_sum(pol.acc_s, sred);
     if (threadIdx.x == 0) a.partial[slot] = s;
-  } else if constexpr (MODE == MODE_CS || MODE == MODE_CSF) {
+  } else if constexpr (mode_sums_cs(MODE)) {
     double s = 0.0, scs = 0.0;
     block_sum2(pol.acc_s, pol.acc_cs, sred, &s, &scs);
     if (threadIdx.x == 0) {
@@ -589,7 +622,8 @@ struct ScatterPol {
     for (int p = 0; p < NP; ++p) v[p] = fma(w, static_cast<double>(m[p]), v[p]);
   }
 
-  __device__ inline void end_row() {}
+  __device__ inline void set_out(int, int) {}
+  __device__ inline void end_row(int, bool) {}
   __device__ inline void pool2(int, const Raw&, const Raw&) {}
 
   // A quarter of the pyramid gradient of the 2x2 block this pixel belongs
@@ -1653,8 +1687,12 @@ FA_API int fa_gpu_ssim_cs_coef(const void* x, const void* y, int dtype, int N, i
   a.oc = aux + planes * npix;
   a.otx = aux + 2 * planes * npix;
   a.oty = aux_dy ? aux + 3 * planes * npix : nullptr;
-  rc = dtype == FA_F32 ? launch_ssim_k<float, double, MODE_CSF>(K, a, planes, device, st)
-                       : launch_ssim_k<double, double, MODE_CSF>(K, a, planes, device, st);
+  if (!a.unit_s && !a.oty)
+    rc = dtype == FA_F32 ? launch_ssim_k<float, double, MODE_CSC>(K, a, planes, device, st)
+                         : launch_ssim_k<double, double, MODE_CSC>(K, a, planes, device, st);
+  else
+    rc = dtype == FA_F32 ? launch_ssim_k<float, double, MODE_CSF>(K, a, planes, device, st)
+                         : launch_ssim_k<double, double, MODE_CSF>(K, a, planes, device, st);
   if (rc != FA_OK) return rc;
   hipLaunchKernelGGL(planes2_kernel, dim3(static_cast<unsigned>(planes)), dim3(BLOCK), 0, st,
                      partial, partial_cs, a.bpp, static_cast<double>(npix), out_s, out_cs);

@@ -142,6 +142,7 @@ __device__ inline void strip_engine(Pol& pol, const float* __restrict__ win,
   // addresses into the grid; rows and columns past it are never emitted.
   using EIn = typename Pol::EIn;
   static_assert(OUTW % 2 == 0, "a lane's first output column is even");
+  pol.set_out(col0 + oc_l, max(0, min(COLS_PER_LANE, min(OUTW - oc_l, out_W - col0 - oc_l))));
   EIn ein = pol.emit_load(r0 + hrow, col0 + oc_l);
 
   for (int qc = 0; qc < nph; qc += NCYC) {
@@ -237,7 +238,7 @@ __device__ inline void strip_engine(Pol& pol, const float* __restrict__ win,
             const int oc = col0 + oc_l + k;
             pol.emit(r0 + orow_l, oc, h[k], out_lane && oc_l + k < OUTW && oc < out_W, ein, k);
           }
-          pol.end_row();
+          pol.end_row(r0 + orow_l, orow_l < rows_here);
         }
         ein = ein_next;
       }

@@ -335,6 +335,38 @@ def test_cs_coef_scatter_matches_recomputed_backward(gpu, dt, unit_s, need_dy):
             assert err <= 1e-6, err
 
 
+# map widths that end a strip (246 columns with 11 taps) or a lane's four columns at
+# each remainder, and maps narrower than four
+@pytest.mark.parametrize("k,wout", [(11, 1), (11, 2), (11, 3), (11, 246), (11, 247), (11, 249),
+                                    (11, 492), (11, 495), (3, 1), (3, 254), (3, 255), (7, 253)])
+def test_cs_coef_maps_without_dy(gpu, k, wout):
+    """The cs pass without dy's map (its own kernel) against the one with it: the
+    maps are the same float64 expressions, rearranged, so b and c agree to a
+    float32 step (2^-23 relative, and 2^-149 where they underflow); tx = c (cs ux
+    - uy) may cancel, and its float64 terms are at most |c| / 2 for samples in
+    [0, 1] about 0.5, each with a few 2^-53."""
+    from frame_analytics_amd import backend
+    from frame_analytics_amd.functional import gaussian_window_1d
+
+    win = gaussian_window_1d(k, 1.5, device=gpu, dtype=torch.float32)
+    consts = (0.5, (0.01) ** 2, (0.03) ** 2)
+    for dt, h in ((torch.float32, k + 9), (torch.float64, k + 4)):
+        xa, ya = float_pair((1, 2, h, wout + k - 1), 0.05, seed=wout + k)
+        x = torch.from_numpy(xa).to(device=gpu, dtype=dt)
+        y = torch.from_numpy(ya).to(device=gpu, dtype=dt)
+        s0, cs0, px0, py0, a0 = backend.ssim_cs_coef_forward(x, y, win, *consts, False, dt, True)
+        s1, cs1, px1, py1, a1 = backend.ssim_cs_coef_forward(x, y, win, *consts, False, dt, False)
+        assert torch.equal(px1, px0) and torch.equal(py1, py0)
+        for a, b in ((s1, s0), (cs1, cs0)):
+            assert float(((a - b).abs() / b.abs()).max()) <= 1e-13
+        b0, c0, t0 = (m.double() for m in a0[:3])
+        b1, c1, t1 = (m.double() for m in a1)
+        tiny = 2.0 ** -149
+        assert bool(((b1 - b0).abs() <= 2.0 ** -23 * b0.abs() + tiny).all())
+        assert bool(((c1 - c0).abs() <= 2.0 ** -23 * c0.abs() + tiny).all())
+        assert bool(((t1 - t0).abs() <= 2.0 ** -23 * t0.abs() + 2.0 ** -48 * c0.abs() + tiny).all())
+
+
 def test_cs_coef_path_falls_back_when_both_means_get_gradients(gpu):
     """A loss that reads both plane means of a scale made with ``use="cs"``
     (not MS-SSIM's) gets the recomputing backward: its gradient equals the one
