@@ -259,6 +259,32 @@ __device__ inline void row_store(double v, __amdgpu_buffer_rsrc_t r, uint32_t of
   __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2_t, v), r, off, 0, 0);
 }
 
+// Column k past the lane's byte offset, 0 past the row.
+template <typename E>
+__device__ inline E row_load(__amdgpu_buffer_rsrc_t r, uint32_t off, int k) {
+  if constexpr (sizeof(E) == 4) {
+    return __builtin_bit_cast(E, __builtin_amdgcn_raw_buffer_load_b32(r, off + 4u * k, 0, 0));
+  } else {
+    return __builtin_bit_cast(E, __builtin_amdgcn_raw_buffer_load_b64(r, off + 8u * k, 0, 0));
+  }
+}
+
+// The four columns from the lane's byte offset, all within the row.
+template <typename E>
+using Quad = E __attribute__((ext_vector_type(4)));
+template <typename E>
+__device__ inline Quad<E> quad_load(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+  if constexpr (sizeof(E) == 4) {
+    return __builtin_bit_cast(Quad<E>, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
+  } else {
+    typedef E pair_t __attribute__((ext_vector_type(2)));
+    const pair_t a = __builtin_bit_cast(pair_t, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
+    const pair_t b =
+        __builtin_bit_cast(pair_t, __builtin_amdgcn_raw_buffer_load_b128(r, off + 16u, 0, 0));
+    return Quad<E>{a[0], a[1], b[0], b[1]};
+  }
+}
+
 // A lane's first `n` (0 .. 4) of four consecutive columns from `col`, stored with
 // three instructions for any n: the widest that n fills, the pair and the odd
 // one, each dropped by the bounds check on the lanes that do not need it. (Four

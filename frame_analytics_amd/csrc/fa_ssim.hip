@@ -558,7 +558,7 @@ struct ScatterArgs {
                         // share (maps written by MODE_CSF for a unit gradient)
 };
 
-template <typename T, bool DY>
+template <typename T, int KW, bool DY>
 struct ScatterPol {
   static constexpr int NP = DY ? 4 : 3;
   using CT = double;
@@ -572,8 +572,7 @@ struct ScatterPol {
 
   const float* __restrict__ aux[4];  // this plane of each coefficient map
   int Hout, Wout;
-  uint32_t lcol;  // this lane's map column, clamped into the map
-  bool col_ok;    // ...and whether it was inside before clamping
+  uint32_t mcol;  // byte offset of this lane's map column, past any row when outside
   const T* __restrict__ x;
   const T* __restrict__ y;
   int64_t img_off;
@@ -588,23 +587,19 @@ struct ScatterPol {
   int Hp, Wp;        // pyramid level grid: floor(H/2) x floor(W/2)
   int64_t gp_off;    // this plane of the pyramid gradient
 
-  // Zero padding outside the Hout x Wout support, branch free: the clamped
-  // address is always loaded and the value masked.
+  // Zero padding outside the Hout x Wout support, by the bounds check of each
+  // row (a row outside is no bytes long).
   __device__ inline void set_column(int col) {
-    col_ok = col >= 0 && col < Wout;
-    lcol = static_cast<uint32_t>(col < 0 ? 0 : (col < Wout ? col : Wout - 1));
+    mcol = lane_off<float>(col, col >= 0 && col < Wout);
   }
 
   __device__ inline Raw load(int row) const {
-    const bool ok = col_ok && row >= 0 && row < Hout;
-    const uint32_t r = static_cast<uint32_t>(row < 0 ? 0 : (row < Hout ? row : Hout - 1));
-    const uint32_t o = r * static_cast<uint32_t>(Wout) + lcol;  // uniform row, lane column
+    const bool ok = row >= 0 && row < Hout;  // uniform
+    const int64_t o = static_cast<int64_t>(row) * Wout;
     Raw v;
 #pragma unroll
-    for (int p = 0; p < NP; ++p) {
-      const float t = aux[p][o];
-      v.v[p] = ok ? t : 0.0f;
-    }
+    for (int p = 0; p < NP; ++p)
+      v.v[p] = row_load<float>(row_rsrc(ok ? aux[p] + o : nullptr, Wout), mcol, 0);
     return v;
   }
 
@@ -622,8 +617,6 @@ struct ScatterPol {
     for (int p = 0; p < NP; ++p) v[p] = fma(w, static_cast<double>(m[p]), v[p]);
   }
 
-  __device__ inline void set_out(int, int) {}
-  __device__ inline void end_row(int, bool) {}
   __device__ inline void pool2(int, const Raw&, const Raw&) {}
 
   // A quarter of the pyramid gradient of the 2x2 block this pixel belongs
@@ -639,41 +632,81 @@ struct ScatterPol {
   // Without dy, what emit reads for a lane's COLS_PER_LANE outputs of one
   // row -- x, y and the pyramid gradient of the 2x2 blocks they belong to
   // (the lane's first column is even: outputs k = 0, 1 share block 0, k = 2,
-  // 3 block 1) -- is loaded a phase ahead by the strip engine.  With dy the
-  // second set of registers would take the kernel past 256 (one wave per
-  // SIMD), so emit loads it itself.
+  // 3 block 1) -- is loaded a phase ahead by the strip engine, as it lies in
+  // memory: what is past the row, absent or of the level's other element type
+  // comes back 0 from the bounds check of its row, and nothing is done with a
+  // value before its phase.  (Converted and masked when it was loaded, the level's
+  // gradient made every phase wait for its two loads in turn, and with them for
+  // the maps of the next phase: 8 x 3 x 1080 x 1920 float32 336 us, 318 as it is
+  // read now, 302 with x, y and dx four columns at a time instead of one by one;
+  // 16 x 3 x 256 x 256 without a level 34 -> 31.  It moves 1.45 GB at 4.8 TB/s.)
+  // With dy the second set of registers would take the kernel past 256 (one
+  // wave per SIMD), so emit loads it itself.
   static constexpr bool PRE = !DY;
+  // A lane's four samples come at once, from the last four of the row where it
+  // ends there (a row has at least KW); rows of three come one by one.
+  static constexpr bool QUAD = KW > 3;
   struct EInPre {
-    T x[COLS_PER_LANE], y[COLS_PER_LANE];
-    double g[2];
+    Quad<T> x, y;
+    double g64[2];
+    float g32[2];
   };
   struct EInNone {};
   using EIn = typename std::conditional<PRE, EInPre, EInNone>::type;
 
-  __device__ inline EIn emit_load(int orow, int ocol) const {
+  uint32_t xoff, goff;      // byte offset of the samples read; of the lane's block / 4
+  int xback;                // columns the samples read lie before the lane's first
+  QuadOff<T> qoff;
+  T out[COLS_PER_LANE];
+  __device__ inline void set_out(int ocol, int n) {
+    if constexpr (PRE) {
+      const int c = QUAD ? min(ocol, W - COLS_PER_LANE) : ocol;
+      xback = ocol - c;
+      xoff = static_cast<uint32_t>(c) * static_cast<uint32_t>(sizeof(T));
+      goff = static_cast<uint32_t>(ocol) * 2u;
+      qoff = quad_off<T>(ocol, n);
+    }
+  }
+
+  // the lane's column k among the samples read
+  __device__ inline T quad_at(const Quad<T>& v, int k) const {
+    T r = v[k];
+    if constexpr (QUAD) {
+#pragma unroll
+      for (int b = 1; b < COLS_PER_LANE; ++b)
+        if (k + b < COLS_PER_LANE) {
+          const T u = v[k + b];
+          r = xback == b ? u : r;
+        }
+    }
+    return r;
+  }
+
+  __device__ inline EIn emit_load(int orow, int) const {
     EIn e;
     if constexpr (PRE) {
       const int r = orow < H ? orow : H - 1;
       const int64_t base = img_off + static_cast<int64_t>(r) * W;
+      const auto xr = row_rsrc(x + base, W), yr = row_rsrc(y + base, W);
+      if constexpr (QUAD) {
+        e.x = quad_load<T>(xr, xoff);
+        e.y = quad_load<T>(yr, xoff);
+      } else {
 #pragma unroll
-      for (int k = 0; k < COLS_PER_LANE; ++k) {
-        const int c = ocol + k < W ? ocol + k : W - 1;
-        e.x[k] = x[base + c];
-        e.y[k] = y[base + c];
-      }
-      e.g[0] = 0.0;
-      e.g[1] = 0.0;
-      if (gpx && Hp > 0 && Wp > 0) {  // uniform
-        const int pr = orow >> 1;
-        const int64_t prow = gp_off + static_cast<int64_t>(pr < Hp ? pr : Hp - 1) * Wp;
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          const int pc = (ocol >> 1) + j;
-          const int64_t o = prow + (pc < Wp ? pc : Wp - 1);
-          const double t = gp_f64 ? static_cast<const double*>(gpx)[o]
-                                  : static_cast<double>(static_cast<const float*>(gpx)[o]);
-          e.g[j] = pr < Hp && pc < Wp ? 0.25 * t : 0.0;
+        for (int k = 0; k < COLS_PER_LANE; ++k) {
+          e.x[k] = row_load<T>(xr, xoff, k);
+          e.y[k] = row_load<T>(yr, xoff, k);
         }
+      }
+      const int pr = orow >> 1;
+      const bool on = gpx && pr < Hp;  // uniform
+      const int64_t prow = gp_off + static_cast<int64_t>(pr) * Wp;
+      const auto gd = row_rsrc(on && gp_f64 ? static_cast<const double*>(gpx) + prow : nullptr, Wp);
+      const auto gf = row_rsrc(on && !gp_f64 ? static_cast<const float*>(gpx) + prow : nullptr, Wp);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        e.g64[j] = row_load<double>(gd, 2u * goff, j);
+        e.g32[j] = row_load<float>(gf, goff, j);
       }
     }
     return e;
@@ -682,12 +715,10 @@ struct ScatterPol {
   __device__ inline void emit(int orow, int ocol, const double* v, bool valid, const EIn& e,
                               int k) {
     if constexpr (PRE) {
-      // every lane stores, through a row buffer resource (see row_store)
-      const double xv = static_cast<double>(e.x[k]) - shift;
-      const double yv = static_cast<double>(e.y[k]) - shift;
-      row_store(static_cast<T>(gmul * (2.0 * xv * v[0] + yv * v[1] + v[2]) + e.g[k >> 1]),
-                row_rsrc(dx ? dx + img_off + static_cast<int64_t>(orow) * W : nullptr, W),
-                lane_off<T>(ocol, valid));
+      const double xv = static_cast<double>(quad_at(e.x, k)) - shift;
+      const double yv = static_cast<double>(quad_at(e.y, k)) - shift;
+      const double g = e.g64[k >> 1] + static_cast<double>(e.g32[k >> 1]);  // one of them is 0
+      out[k] = static_cast<T>(fma(0.25, g, gmul * (2.0 * xv * v[0] + yv * v[1] + v[2])));
     } else {
       if (!valid) return;
       const int64_t o = img_off + static_cast<int64_t>(orow) * W + ocol;
@@ -700,12 +731,19 @@ struct ScatterPol {
                              pyr_grad(gpy, orow, ocol));
     }
   }
+
+  // without dy dx is wanted (the host refuses a call for neither); every lane stores
+  __device__ inline void end_row(int orow, bool on) {
+    if constexpr (PRE)
+      quad_store(out, row_rsrc(on ? dx + img_off + static_cast<int64_t>(orow) * W : nullptr, W),
+                 qoff);
+  }
 };
 
 template <typename T, int KW, bool DY>
 __global__ __launch_bounds__(BLOCK) void scatter_kernel(ScatterArgs a) {
-  constexpr int NP = ScatterPol<T, DY>::NP;
-  __shared__ double sbuf[2][PH][NP / ScatterPol<T, DY>::NSUB][HROW];
+  constexpr int NP = ScatterPol<T, KW, DY>::NP;
+  __shared__ double sbuf[2][PH][NP / ScatterPol<T, KW, DY>::NSUB][HROW];
 
   const int t = static_cast<int>(xcd_tile(blockIdx.x, gridDim.x));
   const int plane = t / a.bpp;
@@ -713,7 +751,7 @@ __global__ __launch_bounds__(BLOCK) void scatter_kernel(ScatterArgs a) {
   const int chunk = tile / a.strips;
   const int strip = tile - chunk * a.strips;
 
-  ScatterPol<T, DY> pol;
+  ScatterPol<T, KW, DY> pol;
   const int64_t aux_off = static_cast<int64_t>(plane) * a.Hout * a.Wout;
   pol.aux[0] = a.ab + aux_off;
   pol.aux[1] = a.ac + aux_off;
@@ -737,7 +775,7 @@ __global__ __launch_bounds__(BLOCK) void scatter_kernel(ScatterArgs a) {
   pol.Hp = a.H / 2;
   pol.Wp = a.W / 2;
   pol.gp_off = static_cast<int64_t>(plane) * pol.Hp * pol.Wp;
-  strip_engine<ScatterPol<T, DY>, KW>(pol, a.win, -(KW - 1), a.H, a.W, a.TH, strip, chunk,
+  strip_engine<ScatterPol<T, KW, DY>, KW>(pol, a.win, -(KW - 1), a.H, a.W, a.TH, strip, chunk,
                                       sbuf);
 }
 

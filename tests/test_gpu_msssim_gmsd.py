@@ -367,6 +367,45 @@ def test_cs_coef_maps_without_dy(gpu, k, wout):
         assert bool(((t1 - t0).abs() <= 2.0 ** -23 * t0.abs() + 2.0 ** -48 * c0.abs() + tiny).all())
 
 
+# rows that end a strip or a lane's four columns at each remainder, odd levels, and
+# the narrowest row, whose samples are read one by one
+@pytest.mark.parametrize("k,h,w", [(3, 3, 3), (3, 9, 4), (5, 7, 5), (11, 12, 245), (11, 13, 246),
+                                   (11, 21, 247), (11, 16, 248), (11, 11, 494), (9, 10, 254)])
+def test_cs_scatter_edges(gpu, k, h, w):
+    """dx of the scatter against its formula in float64 torch on the CPU, g (2 x'
+    F(b) + y' F(c) + F(tx)) + up(level) / 4 with F the transposed window: float64
+    sums of at most 2 K^2 + 4 terms (2^-44 of their magnitudes covers them), and
+    one rounding to the output type."""
+    from frame_analytics_amd import backend
+    from frame_analytics_amd.functional import gaussian_window_1d
+
+    win = gaussian_window_1d(k, 1.5, device=gpu, dtype=torch.float32)
+    w64 = win.double().cpu()
+    ker = torch.outer(w64, w64)[None, None]
+    gen = torch.Generator(device="cpu").manual_seed(w)
+    ho, wo = h - k + 1, w - k + 1
+    aux = torch.randn(3, 2, ho, wo, generator=gen)
+    g = torch.tensor([-1.25, 0.75], dtype=torch.float64)
+    for dt, gt in ((torch.float32, torch.float64), (torch.float32, torch.float32),
+                   (torch.float64, torch.float64), (torch.float32, None)):
+        x, y = (torch.rand(1, 2, h, w, generator=gen).to(dt) for _ in range(2))
+        gp = None if gt is None else torch.randn(1, 2, h // 2, w // 2, generator=gen).to(gt)
+        dx, _ = backend.ssim_cs_scatter(x.to(gpu), y.to(gpu), g.to(gpu), aux.to(gpu), win, 0.5, True,
+                                        False, None if gp is None else gp.to(gpu))
+        full = lambda m: torch.nn.functional.conv_transpose2d(m.double()[:, None], ker)[:, 0][None]
+        xs, ys, gg = x.double() - 0.5, y.double() - 0.5, g[None, :, None, None]
+        want = gg * (2 * xs * full(aux[0]) + ys * full(aux[1]) + full(aux[2]))
+        mag = gg.abs() * (2 * xs.abs() * full(aux[0].abs()) + ys.abs() * full(aux[1].abs())
+                          + full(aux[2].abs()))
+        if gp is not None:
+            up = gp.double().repeat_interleave(2, -2).repeat_interleave(2, -1) / 4
+            want[..., :2 * (h // 2), :2 * (w // 2)] += up
+            mag[..., :2 * (h // 2), :2 * (w // 2)] += up.abs()
+        eps = 2.0 ** -24 if dt == torch.float32 else 2.0 ** -53
+        err = (dx.double().cpu() - want).abs()
+        assert bool((err <= eps * want.abs() + 2.0 ** -44 * mag + 2.0 ** -149).all()), (dt, gt)
+
+
 def test_cs_coef_path_falls_back_when_both_means_get_gradients(gpu):
     """A loss that reads both plane means of a scale made with ``use="cs"``
     (not MS-SSIM's) gets the recomputing backward: its gradient equals the one
