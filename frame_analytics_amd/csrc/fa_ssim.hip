@@ -65,7 +65,8 @@ static_assert(SSIM_TH_MIN % PH == 0 && SSIM_TH_STEP % PH == 0 && SSIM_TH_MAX % S
               "TH ladder");
 
 struct Tiling {
-  int TH, strips, tiles;  // tiles = strips * chunks, per plane
+  int TH, strips, tiles;  // tiles = workgroups per plane: strips * chunks, or, with
+  int gs;                 // the last strip in groups of gs < 256 lanes, fewer
 };
 
 // The tiling of one launch over `planes` planes of an out_H x out_W grid on
@@ -85,23 +86,48 @@ struct Tiling {
 // the best, and no fit of walk_cost improved every one of them.
 constexpr WalkFit STRIP_FIT = {4, 0.5, {0.55, 0.85, 0.92}};
 
-inline Tiling tiling_for(int64_t planes, int out_H, int out_W, int K, int64_t cus, int occ,
-                         bool f64) {
-  Tiling best = {0, 0, 0};
-  double best_cost = 0.0;
+inline Tiling tiling_in(int64_t planes, int out_H, int out_W, int K, int64_t cus, int occ,
+                        bool f64, int gs, double* best_cost) {
+  Tiling best = {0, 0, 0, gs};
+  const int per = STRIP_COLS / gs;
   for (int th = SSIM_TH_MAX; th >= SSIM_TH_MIN; th -= SSIM_TH_STEP) {
     int strips = 0, chunks = 0;
     strip_grid(out_H, out_W, K, th, &strips, &chunks);
-    const int64_t wgs = planes * strips * chunks;
+    const int tiles = (strips - 1) * chunks + (chunks + per - 1) / per;
+    const int64_t wgs = planes * tiles;
     const double cost =
         f64 ? static_cast<double>((wgs + cus * occ - 1) / (cus * occ) * (th + (K + 1) / 2))
             : walk_cost(STRIP_FIT, wgs, cus, occ, th + static_cast<double>(K + 1) / 3.0);
-    if (best.TH == 0 || cost < best_cost) {
-      best_cost = cost;
-      best = Tiling{th, strips, strips * chunks};
+    if (best.TH == 0 || cost < *best_cost) {
+      *best_cost = cost;
+      best = Tiling{th, strips, tiles, gs};
     }
   }
   return best;
+}
+
+// `fold`: the kernel can walk 256 / gs chunks of a last strip that is no wider than
+// gs - (K - 1) columns in one workgroup (gs = 128 or 64): 3.25 workgroups instead of
+// 4 for the 758 output columns of a 768-wide row.  Taken where the whole strips
+// would give the compute units more than two workgroups each; below that
+// the launch waits for memory and the finer chunks of a fold only add halo rows --
+// and, where the fold's chunks are the finer ones, for 6 % or more.  fa.ssim, whole
+// strips -> folded: 8 x 3 x 512 x 768 bfloat16 46.0 -> 41.0 us, 8 x 3 x 512 x 512
+// float32 33.6 -> 27.8, 16 x 3 x 300 x 300 float16 30.1 -> 21.7, 8 x 3 x 720 x 1280
+// float32 87.3 -> 78.6; not taken, 1 x 3 x 720 x 1280 float32 19.2 -> 20.9 (two
+// workgroups each) and 1 x 3 x 1000 x 1000 bfloat16 20.1 -> 22.2 (finer, 5 %).
+inline Tiling tiling_for(int64_t planes, int out_H, int out_W, int K, int64_t cus, int occ,
+                         bool f64, bool fold) {
+  double cost = 0.0;
+  const Tiling whole = tiling_in(planes, out_H, out_W, K, cus, occ, f64, STRIP_COLS, &cost);
+  const int outw = STRIP_COLS - (K - 1);
+  const int last = out_W - (out_W - 1) / outw * outw;  // columns of the last strip
+  int gs = STRIP_COLS;
+  while (gs > WAVE && last <= gs / 2 - (K - 1)) gs /= 2;
+  if (!fold || gs == STRIP_COLS || planes * whole.tiles <= 2 * cus) return whole;
+  double folded = 0.0;
+  const Tiling t = tiling_in(planes, out_H, out_W, K, cus, occ, f64, gs, &folded);
+  return folded <= (t.TH >= whole.TH ? cost : 0.94 * cost) ? t : whole;
 }
 
 // Partial slots per plane the workspace query reports: enough for any TH.
@@ -119,7 +145,7 @@ __device__ inline double quot(double a, double b) { return a / b; }
 struct SsimArgs {
   const void* x;
   const void* y;
-  int H, W, Hout, Wout, TH, strips, bpp;
+  int H, W, Hout, Wout, TH, strips, bpp, fold;
   double shift, C1, C2;
   const float* win;
   float* map;           // MODE_MAP
@@ -154,6 +180,8 @@ template <typename T, typename CTy, int MODE, bool LUMA = false>
 struct SsimPol {
   static constexpr int NP = 4;
   static constexpr int CH = LUMA ? 3 : 1;
+  // emits only into sums, so the lanes of a wave may hold rows of several chunks
+  static constexpr bool FOLD = MODE == MODE_REDUCE && sizeof(CTy) == 4;
   using CT = CTy;
   struct Raw {
     CT x, y;
@@ -432,8 +460,23 @@ __global__ __launch_bounds__(BLOCK) FA_SSIM_ATTR void ssim_kernel(SsimArgs a) {
   const int t = static_cast<int>(xcd_tile(blockIdx.x, gridDim.x));
   const int plane = t / a.bpp;
   const int tile = t - plane * a.bpp;
-  const int chunk = tile / a.strips;
-  const int strip = tile - chunk * a.strips;
+  int chunk, strip, gs = STRIP_COLS;
+  if (Pol::FOLD && a.fold != STRIP_COLS) {
+    // the whole strips of every chunk, then the last strip's groups of chunks
+    const int whole = a.strips - 1;
+    const int n = whole * ((a.Hout + a.TH - 1) / a.TH);
+    if (tile < n) {
+      chunk = tile / whole;
+      strip = tile - chunk * whole;
+    } else {
+      gs = a.fold;
+      chunk = (tile - n) * (STRIP_COLS / gs);
+      strip = whole;
+    }
+  } else {
+    chunk = tile / a.strips;
+    strip = tile - chunk * a.strips;
+  }
 
   Pol pol;
   {
@@ -513,7 +556,7 @@ __global__ __launch_bounds__(BLOCK) FA_SSIM_ATTR void ssim_kernel(SsimArgs a) {
     }
   }
 
-  strip_engine<Pol, KW>(pol, a.win, 0, a.Hout, a.Wout, a.TH, strip, chunk, sbuf);
+  strip_engine<Pol, KW>(pol, a.win, 0, a.Hout, a.Wout, a.TH, strip, chunk, gs, sbuf);
 
   const int64_t slot = static_cast<int64_t>(plane) * a.bpp + tile;
   if constexpr (MODE == MODE_REDUCE) {
@@ -549,7 +592,7 @@ struct ScatterArgs {
   void* dx;
   void* dy;
   const float* win;
-  int H, W, Hout, Wout, TH, strips, bpp;
+  int H, W, Hout, Wout, TH, strips, bpp, fold;
   double shift;
   const void* gpx;  // optional gradient of the next pyramid level (2x2 means)
   const void* gpy;
@@ -561,6 +604,7 @@ struct ScatterArgs {
 template <typename T, int KW, bool DY>
 struct ScatterPol {
   static constexpr int NP = DY ? 4 : 3;
+  static constexpr bool FOLD = false;
   using CT = double;
   struct Raw {
     float v[NP];
@@ -775,7 +819,7 @@ __global__ __launch_bounds__(BLOCK) void scatter_kernel(ScatterArgs a) {
   pol.Hp = a.H / 2;
   pol.Wp = a.W / 2;
   pol.gp_off = static_cast<int64_t>(plane) * pol.Hp * pol.Wp;
-  strip_engine<ScatterPol<T, KW, DY>, KW>(pol, a.win, -(KW - 1), a.H, a.W, a.TH, strip, chunk,
+  strip_engine<ScatterPol<T, KW, DY>, KW>(pol, a.win, -(KW - 1), a.H, a.W, a.TH, strip, chunk, STRIP_COLS,
                                       sbuf);
 }
 
@@ -1015,12 +1059,13 @@ static bool strip_plan_ok(SsimArgs& a) {
 // Tiles `kern` over `planes` planes of an out_H x out_W grid for its
 // occupancy `occ` and launches it; a.TH / a.strips / a.bpp report the tiling.
 template <typename Args>
-static int launch_strips(void (*kern)(Args), int occ, bool f64, Args& a, int64_t planes,
+static int launch_strips(void (*kern)(Args), int occ, bool f64, bool fold, Args& a, int64_t planes,
                          int out_H, int out_W, int K, int device, hipStream_t st) {
-  const Tiling t = tiling_for(planes, out_H, out_W, K, cu_count(device), occ, f64);
+  const Tiling t = tiling_for(planes, out_H, out_W, K, cu_count(device), occ, f64, fold);
   a.TH = t.TH;
   a.strips = t.strips;
   a.bpp = t.tiles;
+  a.fold = t.gs;
   if (!strip_plan_ok(a)) return FA_E_ARG;  // nothing launched
   dim3 grid;
   const int rc = grid_of(planes, t.tiles, &grid);
@@ -1034,7 +1079,8 @@ template <typename T, typename CT, int MODE, int KW, bool LUMA>
 static int launch_ssim_kw(SsimArgs& a, int64_t planes, int device, hipStream_t st) {
   static const int occ =
       occupancy_wgs(reinterpret_cast<const void*>(&ssim_kernel<T, CT, MODE, KW, LUMA>));
-  return launch_strips(ssim_kernel<T, CT, MODE, KW, LUMA>, occ, sizeof(CT) == 8, a, planes,
+  return launch_strips(ssim_kernel<T, CT, MODE, KW, LUMA>, occ, sizeof(CT) == 8,
+                       SsimPol<T, CT, MODE, LUMA>::FOLD, a, planes,
                        a.Hout, a.Wout, KW, device, st);
 }
 
@@ -1074,7 +1120,7 @@ static int launch_ssim(int dtype, int K, bool luma, SsimArgs& a, int64_t planes,
 template <typename T, int KW, bool DY>
 static int launch_scatter_kw(ScatterArgs& a, int64_t planes, int device, hipStream_t st) {
   static const int occ = occupancy_wgs(reinterpret_cast<const void*>(&scatter_kernel<T, KW, DY>));
-  return launch_strips(scatter_kernel<T, KW, DY>, occ, true, a, planes, a.H, a.W, KW, device, st);
+  return launch_strips(scatter_kernel<T, KW, DY>, occ, true, false, a, planes, a.H, a.W, KW, device, st);
 }
 
 template <typename T, bool DY>

@@ -18,7 +18,10 @@
 //     chunks: conflict free).  Double buffering means one barrier per phase.
 //
 // A strip yields 256 - (KW-1) output columns; neighbouring strips overlap by
-// KW-1 input columns, and neighbouring row chunks by KW-1 input rows.
+// KW-1 input columns, and neighbouring row chunks by KW-1 input rows.  Where a
+// row's last strip is narrow, a policy that needs no row of its own per wave may
+// fold it (Pol::FOLD): a workgroup then walks two or four chunks of it side by
+// side.
 //
 // What the lane loads (Pol::set_column once, Pol::load(row) per row; loads are
 // branch free, out-of-grid rows and columns are clamped or zeroed by the
@@ -62,13 +65,17 @@ template <> struct LdsVec<float> { using type = float4; static constexpr int N =
 template <> struct LdsVec<double> { using type = double2; static constexpr int N = 2; };
 
 // Runs the whole strip for one (plane, strip, chunk) workgroup.
+//   gs         : Pol::FOLD only, the lanes of a group: 256, or 128 or 64 where the
+//                workgroup walks 256 / gs consecutive chunks of a strip that is
+//                no wider than gs - (KW-1) columns, a group of whole waves each
+//                (`chunk` is the first)
 //   off        : input row/column of tap 0 for output (0, 0): 0 for a valid
 //                correlation, -(KW-1) for the transposed (scatter) one
 //   out_H,out_W: output grid (the policy knows its input grid)
 template <class Pol, int KW>
 __device__ inline void strip_engine(Pol& pol, const float* __restrict__ win,
                                     int off, int out_H, int out_W, int TH,
-                                    int strip, int chunk,
+                                    int strip, int chunk, int gs,
                                     typename Pol::CT (*sbuf)[PH][Pol::NP / Pol::NSUB][HROW]) {
   using CT = typename Pol::CT;
   using Raw = typename Pol::Raw;
@@ -93,12 +100,16 @@ __device__ inline void strip_engine(Pol& pol, const float* __restrict__ win,
   }
 
   const int lane = threadIdx.x;
+  const int gmask = Pol::FOLD ? gs - 1 : STRIP_COLS - 1;
+  const int glog = Pol::FOLD ? 31 - __builtin_clz(gs) : 8;
   const int col0 = strip * OUTW;          // first output column of the strip
-  const int in_col = col0 + off + lane;   // this lane's input column
-  const int r0 = chunk * TH;              // first output row of the chunk
-  const int rows_here = min(TH, out_H - r0);
-  const int in_row0 = r0 + off;           // input row of tap 0 for output row r0
-  const int nph = (rows_here + PH - 1) / PH;
+  const int in_col = col0 + off + (lane & gmask);  // this lane's input column
+  // a folded strip: the chunk whose column this lane walks is the wave's
+  const int fold_c = Pol::FOLD ? __builtin_amdgcn_readfirstlane(lane >> glog) : 0;
+  const int r0 = chunk * TH;              // first output row of the (first) chunk
+  const int in_row0 = r0 + fold_c * TH + off;  // input row of tap 0 for its output row 0
+  const int outw = Pol::FOLD ? gs - (KW - 1) : OUTW;  // output columns of a group
+  const int nph = (min(TH, out_H - r0) + PH - 1) / PH;
 
   // The column is per lane and fixed for the whole strip; the row is uniform
   // across the workgroup, so every row address is scalar arithmetic and a load
@@ -133,7 +144,10 @@ __device__ inline void strip_engine(Pol& pol, const float* __restrict__ win,
   // wave emits is uniform, so a policy can address its output row with a
   // scalar buffer resource
   const int hrow = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / WAVE);
-  const int oc_l = COLS_PER_LANE * (threadIdx.x % WAVE);  // strip-local output column
+  const int lds_c = COLS_PER_LANE * (threadIdx.x % WAVE);  // first LDS column of the lane's taps
+  const int oc_l = lds_c & gmask;                          // strip-local output column
+  // rows of the chunk the lane's outputs belong to
+  const int rows_here = min(TH, out_H - r0 - (Pol::FOLD ? lds_c >> glog : 0) * TH);
 
   // What emit reads from memory for the lane's outputs (Pol::EIn: the input
   // samples of the scatter, an upstream gradient map) is loaded one phase
@@ -164,7 +178,7 @@ __device__ inline void strip_engine(Pol& pol, const float* __restrict__ win,
         // float64 forward splits its four moments in two, which halves its
         // LDS per workgroup and lets more workgroups share a CU.)
         const int orow_l = q * PH + hrow;
-        const bool out_lane = orow_l < rows_here && oc_l < OUTW;
+        const bool out_lane = orow_l < rows_here && oc_l < outw;
         CT h[COLS_PER_LANE][NP];
         EIn ein_next;
 #pragma unroll
@@ -197,7 +211,7 @@ __device__ inline void strip_engine(Pol& pol, const float* __restrict__ win,
 
           // ---- horizontal taps, from LDS --------------------------------
           // Every lane runs them (a lane past the strip's outputs reads
-          // columns up to oc_l + 15 < HROW) and every lane emits, with
+          // columns up to lds_c + 15 < HROW) and every lane emits, with
           // `valid` false where there is no output: the policies' stores are
           // then issued on every path, so the wait for the next phase's loads
           // does not wait for them (a store on some paths only made the
@@ -206,7 +220,7 @@ __device__ inline void strip_engine(Pol& pol, const float* __restrict__ win,
 #pragma unroll
             for (int p = 0; p < NPL; ++p) {
               CT in[16];
-              const V16* src = reinterpret_cast<const V16*>(&dst[hrow][p][oc_l]);
+              const V16* src = reinterpret_cast<const V16*>(&dst[hrow][p][lds_c]);
 #pragma unroll
               for (int r = 0; r < NREAD; ++r) {
                 const V16 t = src[r];
@@ -236,7 +250,7 @@ __device__ inline void strip_engine(Pol& pol, const float* __restrict__ win,
 #pragma unroll
           for (int k = 0; k < COLS_PER_LANE; ++k) {
             const int oc = col0 + oc_l + k;
-            pol.emit(r0 + orow_l, oc, h[k], out_lane && oc_l + k < OUTW && oc < out_W, ein, k);
+            pol.emit(r0 + orow_l, oc, h[k], out_lane && oc_l + k < outw && oc < out_W, ein, k);
           }
           pol.end_row(r0 + orow_l, orow_l < rows_here);
         }

@@ -15,7 +15,7 @@ import torch
 
 import frame_analytics_amd as fa
 from oracle import reference as ref
-from tests.conftest import natural_pair, u8_pair
+from tests.conftest import float_pair, natural_pair, u8_pair
 
 pytestmark = pytest.mark.gpu
 
@@ -337,3 +337,25 @@ def test_strip_one_launch_finish_carries_nan(gpu):
     per = fa.ssim(xb, y, data_range=255.0, reduction="none").cpu().numpy()
     assert np.isnan(per[0]) and np.isnan(per[2]) and abs(per[1] - p2[1]) <= 1e-12 * abs(p2[1])
     assert np.isnan(float(fa.ssim(xb, y, data_range=255.0)))
+
+
+# launches whose last strip is walked in groups of 64 lanes (at most 54 of 246 columns
+# with 11 taps) and of 128 (at most 118), the widths either side of each, a strip
+# that is the only one, chunk counts that leave groups empty, and other windows
+@pytest.mark.parametrize("shape,k", [
+    ((24, 3, 120, 310), 11), ((24, 3, 117, 311), 11), ((24, 3, 101, 374), 11),
+    ((24, 3, 120, 375), 11), ((48, 3, 121, 64), 11), ((48, 3, 90, 65), 11), ((48, 3, 93, 128), 11),
+    ((24, 3, 110, 257), 11), ((40, 3, 61, 318), 3), ((40, 3, 67, 60), 7), ((24, 3, 99, 766), 9)])
+def test_folded_last_strip(gpu, shape, k):
+    """The last strip's chunks side by side in a workgroup, against the oracle at the
+    file's bar and against the mean of the map, whose kernel does not fold: the
+    same float32 values, at most 1, rounded once on their way to the map and three
+    times in a lane's sum of four (2^-24 each)."""
+    a, b = float_pair(shape, 0.05, seed=shape[-1] + k)
+    x, y = torch.from_numpy(a).to(gpu), torch.from_numpy(b).to(gpu)
+    got = fa.ssim(x, y, data_range=1.0, win_size=k, reduction="none").double()
+    m = fa.ssim(x, y, data_range=1.0, win_size=k, return_map=True)
+    per = m.double().mean(dim=(1, 2, 3))
+    assert float((got - per).abs().max()) <= 5 * 2.0 ** -24
+    want = ref.ssim(a[:2], b[:2], 1.0, win_size=k, reduction="none")
+    assert max(_rel(float(g), float(w)) for g, w in zip(got[:2], want)) <= REL
