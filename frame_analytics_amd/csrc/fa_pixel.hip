@@ -381,7 +381,7 @@ __global__ __launch_bounds__(BLOCK) void pix_float_kernel(
 // consecutive vectors from each tensor, so at any moment the workgroups read
 // a compact window of a few MB.  HBM3E serves that with better row locality
 // than a (bpi, N) grid whose workgroups stream every image at once (measured
-// on MI355X: configs[2] 55.4 us against 58.8 us per launch, 89.8% against
+// on MI355X: 8 x 3 x 2160 x 3840 55.4 us against 58.8 us per launch, 89.8% against
 // 84.6% of 8 TB/s; 8 x 3 x 1080 x 1920 uint8 15.7 against 16.1 us).
 //
 // Images are contiguous, so a wave's vectors move from image to image as the
@@ -403,7 +403,7 @@ __global__ __launch_bounds__(BLOCK) void pix_float_kernel(
 // --------------------------------------------------------------------------
 // Launch shape, from a sweep on MI355X (uint8 MSE kernel time; one workgroup
 // per CU unless noted):
-//   U x threads      4Kx8   1080p RGB x8   1080p RGB x32
+//   U x threads      RGB 4K x8           1080p RGB x8   1080p RGB x32
 //   4 x 256           55.7-56.1 us        16.8-17.2 us   58.3-58.6 us
 //   2 x 512           55.7                15.9-16.2      56.5-58.8
 //   2 x 256, 2/CU     56.6-56.7           16.0-16.4      56.4
@@ -675,6 +675,17 @@ static int64_t sweep_grid(const void* a, const void* b, int64_t n_images, int64_
   return nv >= G * (many ? SWEEP_MANY_BLOCK : SWEEP_UNROLL * SWEEP_BLOCK) ? G : 0;
 }
 
+// Whether `bpi` cuts uint8 images into whole rounds of the sweep: what a call without
+// a workspace has to ask for.  Below PIX_SWEEP_MIN_ELEMS such a call is finished
+// by the small walk or by the per-image grid, which read no `bpi` slots.
+static bool sweep_cut(const void* a, const void* b, int64_t n_images, int64_t per, int bpi) {
+  const uintptr_t bases = reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b);
+  if ((bases & 15) != 0 || per % 16 != 0 || bpi % SWEEP_SLOTS_PER_CU != 0) return false;
+  const bool many = per * n_images < SWEEP_MANY_WAVES_BELOW;
+  return per / 16 >= static_cast<int64_t>(bpi / SWEEP_SLOTS_PER_CU) *
+                         (many ? SWEEP_MANY_BLOCK : SWEEP_UNROLL * SWEEP_BLOCK);
+}
+
 // Launch of the sweep when it applies (sweep_grid): 16-byte aligned bases, whole
 // vectors per image and at least one round per image.  Returns the partial
 // columns per image it writes, -1 when it finished the call through `fin`, or 0
@@ -775,7 +786,7 @@ __global__ __launch_bounds__(BLOCK) void pix_view_kernel(PixView v) {
 // and a lane issues the loads of VR rows x VQ dwords before it sums any, so
 // enough bytes are in flight: one dword load per
 // row at a time left this kernel latency bound (a 4-byte aligned crop of
-// configs[2] took 85 us, a byte-offset one 204 us).  Each wave takes rows of its
+// 8 x 3 x 2160 x 3840 took 85 us, a byte-offset one 204 us).  Each wave takes rows of its
 // own: with the whole workgroup on one row a 1349-byte row filled a third of
 // the lanes of a step and the rows of a small crop followed one another (Y-PSNR
 // of 1 x 3 x 1021 x 1357 14.9 -> 10.2 us, of 64 x 64 91 -> 14; crops of
@@ -990,7 +1001,7 @@ static int launch_view_dtype(int dtype, int op, dim3 grid, hipStream_t st, const
 // --------------------------------------------------------------------------
 // The finalize's workgroup size: the partials come from other XCDs' L2s, so
 // every round of dependent loads waits the full memory latency; with 1024
-// lanes and 8 loads in flight per lane the total of a configs[2] PSNR
+// lanes and 8 loads in flight per lane the total of an 8 x 3 x 2160 x 3840 PSNR
 // (8 x 2048 partials) is two rounds (256 lanes took 5.5 us for it).
 constexpr int FIN_BLOCK = 1024;
 
@@ -1220,12 +1231,10 @@ FA_API int fa_gpu_pixel_reduce_once(const void* a, const void* b, int dtype,
       pfin = &fin;
     }
   }
-  // a null workspace is enough only for the one-launch form
+  // a null workspace is enough only for the one-launch form, and only for a `bpi`
+  // that cuts the images as the sweep does (every such call finishes)
   const int64_t cus = cu_count(device);
-  const bool finishes =
-      pfin && (sweep_grid<uint8_t>(a, b, n_images, n_per_image, bpi, cus, true) > 0 ||
-               (n_per_image < PIX_SWEEP_MIN_ELEMS && u8_finishes(n_images, cols)));
-  if (!partial && !finishes) return FA_E_ARG;
+  if (!partial && !(pfin && sweep_cut(a, b, n_images, n_per_image, bpi))) return FA_E_ARG;
   FA_DEVICE_SCOPE(device);
   hipStream_t st = static_cast<hipStream_t>(stream);
 

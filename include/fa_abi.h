@@ -419,7 +419,7 @@ FA_API int fa_gpu_ms_ssim_head_backward(const double* const* terms, int M,
  * acc: null, or FA_MS_SSIM_ACC_WORDS uint64 of device memory, zero when the
  * call starts; the call leaves it zero.  With it, uint8 input without luma
  * whose every scale fits the matrix-core kernel (widths a multiple of 8 at
- * every scale, e.g. W % 128 == 0 at M = 5; K <= 16; C1, C2 > 0; N * C <= 256;
+ * every scale, e.g. W % 128 == 0 at M = 5, or planes of 2^17 samples and more; K <= 16; C1, C2 > 0; N * C <= 256;
  * 3 <= M <= 5) runs as three launches: scale 0, scale 1 (which also writes
  * levels 3 and 4), and scales 2 .. M - 1 side by side in one launch whose last
  * workgroup finishes the reduction from per-(scale, plane) fixed-point sums
@@ -479,8 +479,9 @@ FA_API int fa_gpu_ssim_noalloc(const void* x, const void* y, int dtype, int N,
  * `acc` (it may be null) and runs as fa_gpu_pixel_reduce.  `acc` is state of
  * one stream: calls that may overlap (two streams) need one buffer each.
  * `partial` may be null for a call that takes the one-launch form (it is not
- * read); a call with a null `partial` that cannot returns FA_E_ARG before
- * launching anything.
+ * read) with 16-byte aligned images and a `bpi` that is a multiple of 16 and cuts
+ * them into whole rounds of the sweep; any other call with a null `partial`
+ * returns FA_E_ARG before launching anything.
  */
 #define FA_PIXEL_ACC_WORDS ((32 + 1) * 16)
 FA_API int fa_gpu_pixel_reduce_once(const void* a, const void* b, int dtype,
