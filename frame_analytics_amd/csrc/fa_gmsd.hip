@@ -52,7 +52,7 @@ constexpr int G_OUTW_NARROW = WAVE - 2;    // ... 1 column per lane
 // at most this many waves per SIMD in the one round of resident waves: more
 // waves give each wave a shorter run, whose prologue (two window rows, the
 // first loads' latency) and final reductions then weigh more; measured
-// slower at 7 and 8 on configs[4]
+// slower at 7 and 8 on 8 x 3 x 1080 x 1920
 constexpr int G_MAX_WAVES_PER_SIMD = 6;
 
 struct GView {

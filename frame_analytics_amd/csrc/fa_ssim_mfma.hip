@@ -1004,7 +1004,7 @@ __device__ __attribute__((always_inline)) inline void mf_walk(
         // MF_MAP's stores.  A lane holds rows 4g .. 4g+3 of one column, so
         // stored straight from the fragment each store instruction covers 64
         // bytes of four rows, most pieces split over two 128-byte lines (map
-        // rows of 7640 bytes at configs[1]); the texture units then spent ~51
+        // rows of 7640 bytes at W = 1920); the texture units then spent ~51
         // cycles per store and were 83 % busy.  Instead the four waves stage
         // the workgroup's 16 x 64 block in LDS (rows padded to 68 floats:
         // conflict-free both ways, double-buffered so one barrier per step
@@ -1406,7 +1406,7 @@ MfArgs args_of(const SsimMfmaCall& c) {
 // order on each XCD, so the drain at the end of the launch -- the last
 // workgroups running on emptying SIMDs -- lasts one small chunk instead of one
 // of the uniform size.  Keeping the chunk count, the first half of a column's
-// chunks get weight 1 and the rest 0.4 (on configs[1] 17,17,17,16 blocks
+// chunks get weight 1 and the rest 0.4 (on 8 x 3 x 1080 x 1920 17,17,17,16 blocks
 // become 24,24,10,9: 82.1 against 84.3 us per call over rotated input pairs,
 // the same work and workgroup count).  It needs each XCD's range of tiles to
 // hold whole planes (the count of planes a multiple of 8); walked plane by
@@ -1630,7 +1630,7 @@ int ssim_mfma_ms(const SsimMfmaMs& c, int device, hipStream_t st, bool* done) {
     return FA_OK;
   // The coarse scales share one round of resident workgroups: starting from
   // one chunk per column, the scale with the longest chunks is split once
-  // more while the launch still fits the round (on configs[4]: 3, 1 and 2
+  // more while the launch still fits the round (on 8 x 3 x 1080 x 1920: 3, 1 and 2
   // chunks, 720 of 768 workgroups).  Measured: these passes are bound by
   // instruction issue, so more workgroups than the round holds only add the
   // extra block of rows each chunk starts with; planned one scale at a time
