@@ -250,7 +250,8 @@ def gaussian_window_1d(win_size: int = 11, sigma: float = 1.5, *, device=None,
     normalised 2-D window.  Cached per (size, sigma, device, dtype) so that no
     call after the first performs a host-to-device copy.
     """
-    key = (win_size, sigma, device, dtype)
+    # by value: a tensor sigma hashes by identity
+    key = (int(win_size), float(sigma), device, dtype)
     w = _window_cache.get(key)
     if w is None:
         half = (win_size - 1) / 2.0

@@ -276,3 +276,19 @@ def test_private_accumulator_scope_is_per_thread():
         t.join()
     assert seen["other"] is None
     assert getattr(backend._private, "store", None) is None
+
+
+def test_window_cache_keys_on_the_value_of_sigma():
+    """A tensor sigma that changes in place, or a new one per call, is cached by its
+    value: neither an old window nor an entry per call."""
+    from frame_analytics_amd import functional as fn
+
+    sigma = torch.tensor(1.5)
+    assert torch.equal(fn.gaussian_window_1d(11, sigma), fn.gaussian_window_1d(11, 1.5))
+    sigma.fill_(3.0)
+    assert torch.equal(fn.gaussian_window_1d(11, sigma), fn.gaussian_window_1d(11, 3.0))
+    n = len(fn._window_cache)
+    for _ in range(8):
+        fn.gaussian_window_1d(11, torch.tensor(1.5))
+        fn.gaussian_window_1d(np.int64(11), np.float32(1.5))
+    assert len(fn._window_cache) == n
