@@ -17,6 +17,7 @@ import concurrent.futures as _cf
 import os
 import shutil
 import subprocess
+import sys
 import sysconfig
 from pathlib import Path
 from typing import List, Sequence
@@ -48,6 +49,10 @@ def readbw_library_path() -> Path:
 
 def call_module_path() -> Path:
     return LIBDIR / f"{CALL_NAME}.so"
+
+
+def python_include() -> Path:
+    return Path(sysconfig.get_paths()["include"])
 
 
 def call_sources() -> List[Path]:
@@ -136,17 +141,31 @@ def build_call(verbose: bool = False) -> Path:
     out = call_module_path()
     tmp = out.with_name(f".{out.name}.{os.getpid()}.tmp")
     _run([cxx(), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", f"-I{INCLUDE}",
-          f"-I{sysconfig.get_paths()['include']}", *map(str, call_sources()), "-o", str(tmp)],
+          f"-I{python_include()}", *map(str, call_sources()), "-o", str(tmp)],
          verbose)
     os.replace(tmp, out)
     return out
 
 
+def try_build_call(verbose: bool = False) -> bool:
+    """:func:`build_call`, reported and not raised where it fails (no Python
+    headers, no host compiler): without the module the library is called through
+    ctypes.  One of an earlier build is removed then."""
+    try:
+        build_call(verbose)
+    except Exception as exc:
+        call_module_path().unlink(missing_ok=True)
+        print(f"{CALL_NAME} was not built, the library is called through ctypes: {exc}",
+              file=sys.stderr, flush=True)
+        return False
+    return True
+
+
 def build(verbose: bool = False, jobs: int = 0) -> Path:
     """Compile every kernel source and link ``libfa_gpu.so`` (and build
-    ``libfa_cpu.so`` and ``_fa_call``); returns the GPU library's path."""
+    ``libfa_cpu.so`` and, where it can be built, ``_fa_call``); returns the GPU
+    library's path."""
     build_cpu(verbose)
-    build_call(verbose)
     cc = hipcc()
     objdir = PKG / "_build"
     objdir.mkdir(exist_ok=True)
@@ -174,13 +193,17 @@ def build(verbose: bool = False, jobs: int = 0) -> Path:
     _run(link, verbose)
     os.replace(tmp, out)  # atomic: a concurrent loader never sees half a file
     os.replace(rb_tmp, rb)
+    try_build_call(verbose)
     return out
 
 
 def is_stale() -> bool:
-    """True when a library is missing or older than any source or header."""
-    for lib, srcs in ((library_path(), sources()), (cpu_library_path(), cpu_sources()),
-                      (call_module_path(), call_sources())):
+    """True when a library, or a call module that can be built, is missing or older
+    than any source or header."""
+    built = [(library_path(), sources()), (cpu_library_path(), cpu_sources())]
+    if (python_include() / "Python.h").exists():
+        built.append((call_module_path(), call_sources()))
+    for lib, srcs in built:
         if not lib.exists():
             return True
         t = lib.stat().st_mtime

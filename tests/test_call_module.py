@@ -69,3 +69,30 @@ def test_wrong_arguments_raise(both):
         fast("x", *args[1:])
     with pytest.raises(TypeError):
         fast(*args[:7], "x", *args[8:])
+
+
+def test_build_without_python_headers(monkeypatch, tmp_path, capsys):
+    """A machine that cannot compile the module still gets the libraries, the
+    fallback to ctypes, and no build that stays stale for the module's sake."""
+    monkeypatch.setattr(_build, "LIBDIR", tmp_path)
+    monkeypatch.setattr(_build, "python_include", lambda: tmp_path / "none")
+    made = []
+    real = _build._run
+
+    def run(cmd, verbose):  # the kernels' compiler leaves its outputs, nothing else
+        if cmd[0] == "hipcc-stub":
+            made.append(cmd[-1])
+            open(cmd[-1], "wb").close()
+        else:
+            real(cmd, verbose)
+
+    monkeypatch.setattr(_build, "_run", run)
+    monkeypatch.setattr(_build, "hipcc", lambda: "hipcc-stub")
+    monkeypatch.setattr(_build, "PKG", tmp_path)
+    _build.call_module_path().write_bytes(b"of an earlier build")
+    assert _build.build() == _build.library_path() and _build.library_path().exists()
+    assert len(made) == len(_build.sources()) + 2
+    assert not _build.call_module_path().exists()
+    assert "Python.h" in capsys.readouterr().err
+    assert not _build.is_stale()
+    assert _cabi.load_callers(None) == {}
