@@ -48,7 +48,8 @@ def readbw_library_path() -> Path:
 
 
 def call_module_path() -> Path:
-    return LIBDIR / f"{CALL_NAME}.so"
+    """With the interpreter's ABI tag: another Python never imports it."""
+    return LIBDIR / f"{CALL_NAME}{sysconfig.get_config_var('EXT_SUFFIX')}"
 
 
 def python_include() -> Path:

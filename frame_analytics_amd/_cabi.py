@@ -157,25 +157,34 @@ def load_gpu(path: Optional[Path] = None) -> Tuple[ctypes.CDLL, str]:
     return lib, origin
 
 
+# ctypes argument type -> its letter in _fa_call's prototypes
+_LETTER = {_P: "p", _I: "i", _L: "l", _D: "d"}
+
+
 def load_callers(lib: ctypes.CDLL) -> dict:
     """Entry point name -> callable of the ``_fa_call`` extension module for the
     entry points of ``lib`` that are called often (the rest stay with ctypes).
-    Empty where the module cannot be built or loaded (no Python headers): the
-    same library is then called through ctypes, ~2.5 us a call slower."""
+    The module holds prototypes of its own, so only those that are the ones
+    ctypes would use are taken.  Empty where the module cannot be built or loaded (no
+    Python headers) or is of another ABI version: the same library is then called
+    through ctypes, ~2.5 us a call slower."""
     p = _build.call_module_path()
+    out = {}
     try:
         if not p.exists():
             _build.build_call(verbose=_verbose())
         spec = importlib.util.spec_from_file_location(_build.CALL_NAME, p)
         module = importlib.util.module_from_spec(spec)
         spec.loader.exec_module(module)
+        if module.abi_version != FA_ABI_VERSION:
+            return {}
+        for name, (args, _) in SIGNATURES.items():
+            fn = module.entry(name, ctypes.cast(getattr(lib, name), ctypes.c_void_p).value,
+                              "".join(_LETTER.get(a, "?") for a in args))
+            if fn is not None:
+                out[name] = fn
     except Exception:
         return {}
-    out = {}
-    for name in SIGNATURES:
-        fn = module.entry(name, ctypes.cast(getattr(lib, name), ctypes.c_void_p).value)
-        if fn is not None:
-            out[name] = fn
     return out
 
 

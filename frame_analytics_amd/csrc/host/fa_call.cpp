@@ -6,8 +6,11 @@
 // prototype (include/fa_abi.h) is taken apart at compile time, so an argument is
 // one PyLong / PyFloat conversion.
 //
-// entry(name, address) returns a callable for the entry point `name` at
-// `address` (where the caller's loaded library has it): integers, floats, None or
+// entry(name, address, prototype) returns a callable for the entry point `name` at
+// `address` (where the caller's loaded library has it), or None unless the
+// argument types compiled in here are `prototype`, one letter each (p pointer, i
+// int, l int64, d double): a module older than the library never calls through
+// another prototype.  Its arguments: integers, floats, None or
 // an address for pointers, or an object with a buffer (a ctypes array) for a
 // host array.  A wrong count or type raises before the library is entered.  The
 // GIL is released around the call, as ctypes does.
@@ -106,13 +109,29 @@ PyObject* call(int (*)(A...), PyObject* self, PyObject* const* args, size_t narg
                 std::index_sequence_for<A...>{});
 }
 
+template <typename T>
+constexpr char letter() {
+  if constexpr (std::is_pointer<T>::value) return 'p';
+  else if constexpr (std::is_same<T, double>::value) return 'd';
+  else if constexpr (std::is_same<T, int>::value) return 'i';
+  else if constexpr (std::is_same<T, int64_t>::value) return 'l';
+  else return '!';  // none that Python can name
+}
+
+template <typename... A>
+const char* prototype(int (*)(A...)) {
+  static const char s[] = {letter<A>()..., '\0'};
+  return s;
+}
+
 #define FA_ENTRY(NAME)                                                                   \
-  {#NAME, [](PyObject* self, PyObject* const* args, size_t n, PyObject* kw) -> PyObject* { \
+  {#NAME, prototype(decltype(&NAME)(nullptr)), [](PyObject* self, PyObject* const* args, size_t n, PyObject* kw) -> PyObject* { \
      return call(decltype(&NAME)(nullptr), self, args, n, kw);                           \
    }}
 
 struct Known {
   const char* name;
+  const char* types;
   vectorcallfunc fn;
 };
 
@@ -143,14 +162,15 @@ PyTypeObject entry_type = [] {
 PyObject* make_entry(PyObject*, PyObject* args) {
   const char* name = nullptr;
   PyObject* address = nullptr;
-  if (!PyArg_ParseTuple(args, "sO", &name, &address)) return nullptr;
+  const char* types = nullptr;
+  if (!PyArg_ParseTuple(args, "sOs", &name, &address, &types)) return nullptr;
   void* p = PyLong_AsVoidPtr(address);
   if (!p) {
     if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "null address");
     return nullptr;
   }
   for (const Known& k : KNOWN) {
-    if (std::strcmp(k.name, name) != 0) continue;
+    if (std::strcmp(k.name, name) != 0 || std::strcmp(k.types, types) != 0) continue;
     Entry* e = PyObject_New(Entry, &entry_type);
     if (!e) return nullptr;
     e->vectorcall = k.fn;
@@ -158,11 +178,11 @@ PyObject* make_entry(PyObject*, PyObject* args) {
     e->name = k.name;
     return reinterpret_cast<PyObject*>(e);
   }
-  Py_RETURN_NONE;  // not one of the calls that run often: ctypes serves it
+  Py_RETURN_NONE;  // not one of the calls that run often, or another: ctypes serves it
 }
 
 PyMethodDef methods[] = {
-    {"entry", make_entry, METH_VARARGS, "entry(name, address) -> callable, or None"},
+    {"entry", make_entry, METH_VARARGS, "entry(name, address, prototype) -> callable, or None"},
     {nullptr, nullptr, 0, nullptr},
 };
 
@@ -173,5 +193,10 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_fa_call", nullptr, -1, methods,
 
 PyMODINIT_FUNC PyInit__fa_call() {
   if (PyType_Ready(&entry_type) < 0) return nullptr;
-  return PyModule_Create(&module);
+  PyObject* m = PyModule_Create(&module);
+  if (m && PyModule_AddIntConstant(m, "abi_version", FA_ABI_VERSION) != 0) {
+    Py_DECREF(m);
+    return nullptr;
+  }
+  return m;
 }

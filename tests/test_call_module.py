@@ -5,6 +5,7 @@ GPU is needed."""
 from __future__ import annotations
 
 import ctypes
+import sysconfig
 
 import pytest
 
@@ -96,3 +97,22 @@ def test_build_without_python_headers(monkeypatch, tmp_path, capsys):
     assert "Python.h" in capsys.readouterr().err
     assert not _build.is_stale()
     assert _cabi.load_callers(None) == {}
+
+
+def test_module_of_another_interface_is_not_called(both, monkeypatch, tmp_path):
+    """A module whose prototypes, ABI version or interpreter are not those of the
+    library and of ctypes: its entries are left to ctypes."""
+    lib, callers = both
+    name = "fa_gpu_gmsd_once"
+    args, res = _cabi.SIGNATURES[name]
+    swapped = list(args)  # the same count: a double for an int
+    swapped[swapped.index(ctypes.c_int)] = ctypes.c_double
+    monkeypatch.setitem(_cabi.SIGNATURES, name, (swapped, res))
+    assert set(callers) - set(_cabi.load_callers(lib)) == {name}
+    monkeypatch.setattr(_cabi, "FA_ABI_VERSION", _cabi.FA_ABI_VERSION + 1)
+    assert _cabi.load_callers(lib) == {}
+    assert sysconfig.get_config_var("EXT_SUFFIX") in _build.call_module_path().name
+    monkeypatch.undo()
+    monkeypatch.setattr(_build, "LIBDIR", tmp_path)
+    _build.call_module_path().write_bytes(b"no module")
+    assert _cabi.load_callers(lib) == {}
