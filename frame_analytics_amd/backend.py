@@ -254,7 +254,8 @@ def call_gpu(name: str, *args) -> int:
     else:
         try:
             code = fast(*args)
-        except TypeError:  # an argument only ctypes takes (byref, a ctypes scalar)
+        except (TypeError, OverflowError):  # an argument only ctypes takes (byref, a
+            # ctypes scalar, a number past 64 bits), or refuses
             code = getattr(ext.gpu, name)(*args)
     native_calls[name] += 1
     return int(code)

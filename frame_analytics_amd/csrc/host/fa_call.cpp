@@ -11,7 +11,7 @@
 // argument types compiled in here are `prototype`, one letter each (p pointer, i
 // int, l int64, d double): a module older than the library never calls through
 // another prototype.  Its arguments: integers, floats, None or
-// an address for pointers, or an object with a buffer (a ctypes array) for a
+// an address for pointers, or a ctypes array for a
 // host array.  A wrong count or type raises before the library is entered.  The
 // GIL is released around the call, as ctypes does.
 #define PY_SSIZE_T_CLEAN
@@ -39,6 +39,8 @@ struct Borrowed {
   }
 };
 
+PyObject* array_type = nullptr;  // ctypes.Array
+
 template <typename T>
 bool convert(PyObject* o, T* out, Borrowed& held) {
   if constexpr (std::is_pointer<T>::value) {
@@ -51,6 +53,14 @@ bool convert(PyObject* o, T* out, Borrowed& held) {
       if (!p && PyErr_Occurred()) return false;
       *out = reinterpret_cast<T>(p);
       return true;
+    }
+    // ctypes arrays alone: another object with a buffer may stand for an address
+    // (a ctypes.c_void_p is one, whose buffer holds it), which ctypes resolves
+    const int is_array = PyObject_IsInstance(o, array_type);
+    if (is_array <= 0) {
+      if (is_array == 0)
+        PyErr_Format(PyExc_TypeError, "no address or ctypes array: %.80s", Py_TYPE(o)->tp_name);
+      return false;
     }
     if (held.n == Borrowed::MAX) {
       PyErr_SetString(PyExc_TypeError, "too many array arguments");
@@ -193,6 +203,11 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_fa_call", nullptr, -1, methods,
 
 PyMODINIT_FUNC PyInit__fa_call() {
   if (PyType_Ready(&entry_type) < 0) return nullptr;
+  PyObject* ctypes = PyImport_ImportModule("ctypes");
+  if (!ctypes) return nullptr;
+  array_type = PyObject_GetAttrString(ctypes, "Array");
+  Py_DECREF(ctypes);
+  if (!array_type) return nullptr;
   PyObject* m = PyModule_Create(&module);
   if (m && PyModule_AddIntConstant(m, "abi_version", FA_ABI_VERSION) != 0) {
     Py_DECREF(m);

@@ -116,3 +116,35 @@ def test_module_of_another_interface_is_not_called(both, monkeypatch, tmp_path):
     monkeypatch.setattr(_build, "LIBDIR", tmp_path)
     _build.call_module_path().write_bytes(b"no module")
     assert _cabi.load_callers(lib) == {}
+
+
+@pytest.mark.parametrize("kind", ["void_p", "byref", "bytes", "big"])
+def test_what_only_ctypes_takes(both, kind, monkeypatch):
+    """Arguments that ctypes resolves in its own way reach the library as through
+    ctypes: a c_void_p stands for the address it holds, not for its own."""
+    from frame_analytics_amd import backend
+
+    lib, callers = both
+    native = backend._Native()
+    native.gpu, native.callers = lib, callers
+    monkeypatch.setattr(backend, "_ext", native)
+    name = "fa_gpu_ssim_once"
+    buf = ctypes.create_string_buffer(64)
+    p = ctypes.addressof(buf)
+    n, x, k = 1, p, 4  # k = 4: refused after the pointers, before any launch
+    if kind == "void_p":
+        x = ctypes.c_void_p(None)  # a null pointer: refused as one
+        k = 11
+    elif kind == "byref":
+        x = ctypes.byref(buf)
+    elif kind == "bytes":
+        x = bytes(64)
+    else:
+        n = 1 << 70  # its low bits: no image
+    args = (x, p, 0, n, 1, 64, 64, None, None, None, p, k, 127.5, 6.5, 58.5, None, p, 4096,
+            None, p, p, 0, None)
+    want = lib.fa_gpu_ssim_once(*args)
+    assert want > 0 and backend.call_gpu(name, *args) == want
+    arr = memoryview(bytearray(64))  # refused by ctypes, refused still
+    with pytest.raises(ctypes.ArgumentError):
+        backend.call_gpu(name, arr, *args[1:])
