@@ -1066,7 +1066,8 @@ def gmsd_stats_bwd(x, y, mean, std, g_mean, g_std, T, eps, downsample, need_dx, 
     dev, stream = _site(x)
     _run("fa_gpu_gmsd_backward", _ptr(x), _ptr(y), _DTYPE_CODE[x.dtype], n, c, h, w,
          float(T), float(eps), int(bool(downsample)), _ptr(mean), _ptr(std), _ptr(gm),
-         _ptr(gs), None, _ptr(dx), _ptr(dy), dev, stream)
+         _ptr(gs), _ptr(mean),  # the scratch, which is not touched but not null either
+         _ptr(dx), _ptr(dy), dev, stream)
     return dx, dy
 
 

@@ -1321,15 +1321,14 @@ FA_API int fa_gpu_gmsd_once(const void* x, const void* y, int dtype, int N, int 
 // with respect to contiguous x and y (N x C x H x W, FA_F32 or FA_F64); mean /
 // std are fa_gpu_gmsd's outputs for the same inputs; g_mean / g_std are
 // device arrays of N (either may be null: zero); aux, which earlier builds
-// kept coefficient maps in, is not used; dx / dy (either may be null) are
-// written in full.
+// kept coefficient maps in, is not touched, and refused as null as it was then;
+// dx / dy (either may be null) are written in full.
 FA_API int fa_gpu_gmsd_backward(const void* x, const void* y, int dtype, int N, int C, int H,
                                 int W, double Tc, double eps, int downsample,
                                 const double* mean, const double* std_dev,
                                 const double* g_mean, const double* g_std, double* aux,
                                 void* dx, void* dy, int device, void* stream) {
-  (void)aux;
-  if (!x || !y || !mean || !std_dev) return FA_E_ARG;
+  if (!x || !y || !mean || !std_dev || !aux) return FA_E_ARG;
   if (!dx && !dy) return FA_E_ARG;
   if (dtype != FA_F32 && dtype != FA_F64) return FA_E_DTYPE;
   if (N <= 0 || C <= 0) return FA_E_SHAPE;

@@ -336,8 +336,9 @@ FA_API int fa_gpu_ssim_cs_scatter(const void* x, const void* y, int dtype,
  * with respect to contiguous x and y (N x C x H x W of dtype FA_F32 or
  * FA_F64), computed in float64.  mean / std_dev: fa_gpu_gmsd's outputs for
  * the same inputs (device, N each); g_mean / g_std: device arrays of N (either
- * may be null: zero); aux: not used (may be null); dx / dy: either
- * may be null, written in full (zero on the row / column a downsample drops).
+ * may be null: zero); aux: the scratch of earlier builds, not touched but still
+ * refused as null; dx / dy: either may be null, written in full (zero on the row /
+ * column a downsample drops).
  */
 FA_API int fa_gpu_gmsd_backward(const void* x, const void* y, int dtype, int N,
                                 int C, int H, int W, double Tc, double eps,

@@ -147,6 +147,8 @@ def test_argument_validation_before_any_gpu_work(lib):
                                     p, None, 0, None) == 1  # uint8 has no gradient
     assert lib.fa_gpu_gmsd_backward(p, p, 3, 1, 1, 64, 64, 170.0, 0.0, 1, p, p, None, None, p,
                                     None, None, 0, None) == 5  # neither dx nor dy
+    assert lib.fa_gpu_gmsd_backward(p, p, 3, 1, 1, 64, 64, 170.0, 0.0, 1, p, p, None, None,
+                                    None, p, None, 0, None) == 5  # no aux
     ptrs = (ctypes.c_void_p * 5)(p, p, p, p, p)
     wts = (ctypes.c_double * 5)(0.0448, 0.2856, 0.3001, 0.2363, 0.1333)
     slots = (ctypes.c_int * 5)(4, 4, 4, 4, 4)
