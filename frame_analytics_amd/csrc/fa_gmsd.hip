@@ -847,8 +847,15 @@ struct GbRaw {
   GbPair<T> x[DOWN ? 2 : 1], y[DOWN ? 2 : 1];
 };
 
+// float64 samples (EXACT): every digit of the result is a digit of the caller's, so
+// the divisions and roots are IEEE's and the column differences come before
+// the sums of three (a pedestal under the samples then cancels without a
+// rounding).  Sums of float32 samples are exact in float64 either way and the
+// gradient is rounded to 24 bits: there the iterations above and the shorter
+// form serve.
 template <typename T, bool DOWN, bool DX, bool DY>
 __global__ __launch_bounds__(BLOCK) void gmsd_backward_kernel(GmsdBwdArgs a) {
+  constexpr bool EXACT = std::is_same<T, double>::value;
   const int64_t wg = xcd_tile(blockIdx.x, gridDim.x);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int64_t task = wg * WAVES_PER_BLOCK + wave;
@@ -905,39 +912,62 @@ __global__ __launch_bounds__(BLOCK) void gmsd_backward_kernel(GmsdBwdArgs a) {
   // of the two output rows before this step's: hx = Gx(c) - Gx(c - 2),
   // hy = Gy(c) + Gy(c - 1) + Gy(c - 2)
   double xa = 0.0, xb = 0.0, ya = 0.0, yb = 0.0;
+  double ex[2] = {0.0, 0.0}, ey[2] = {0.0, 0.0};  // EXACT: their column differences
   double hx1[2] = {0.0, 0.0}, hy1[2] = {0.0, 0.0}, hx2[2] = {0.0, 0.0}, hy2[2] = {0.0, 0.0};
   const bool col_on = c >= 0 && c < a.Wout;                       // an output column
   const bool own = lane >= 2 && lane < WAVE - 2 && c < a.Wd;      // a gradient column
 
+  auto col_diff = [](double t) { return t - wave_next(wave_next(t)); };
   auto step = [&](int s, const GbRaw<T, DOWN>& raw) {
     const double xc = sample(raw.x), yc = sample(raw.y);
     // raw Prewitt sums of the window rows s - 2 .. s (output row i = s - 2)
-    auto prewitt_at = [&](double t0, double t1, double t2, double& gx, double& gy) {
-      const double cs = t0 + t1 + t2, rd = t0 - t2;
+    auto prewitt_at = [&](double t0, double t1, double t2, double (&e)[2], double& gx,
+                          double& gy) {
+      const double rd = t0 - t2;
       const double rd1 = wave_next(rd);
-      gx = cs - wave_next(wave_next(cs));
       gy = rd + rd1 + wave_next(rd1);
+      if constexpr (EXACT) {
+        const double e2 = col_diff(t2);
+        gx = e[0] + e[1] + e2;
+        e[0] = e[1];
+        e[1] = e2;
+      } else {
+        gx = col_diff(t0 + t1 + t2);
+      }
     };
     double gx1, gy1, gx2, gy2;
-    prewitt_at(xa, xb, xc, gx1, gy1);
-    prewitt_at(ya, yb, yc, gx2, gy2);
+    prewitt_at(xa, xb, xc, ex, gx1, gy1);
+    prewitt_at(ya, yb, yc, ey, gx2, gy2);
     xa = xb;
     xb = xc;
     ya = yb;
     yb = yc;
     const double G1 = fma(k2, fma(gx1, gx1, gy1 * gy1), eps);
     const double G2 = fma(k2, fma(gx2, gx2, gy2 * gy2), eps);
-    double g1, i1, g2, i2;
-    gb_sqrt(G1, g1, i1);
-    gb_sqrt(G2, g2, i2);
-    const double gs = g1 + g2;
     const double D = G1 + G2 + Tc;
-    const double iD = gb_rcp(D), is = gb_rcp(gs);
-    const double q = fma(2.0 * g1, g2, Tc) * iD;
-    const double w = fma(ks, q - m, wm);
     // g2 - g1 = (G2 - G1) / (g1 + g2), with G2 - G1 in factored form
     const double dG = k2 * fma(gx2 - gx1, gx2 + gx1, (gy2 - gy1) * (gy2 + gy1));
-    const double f = w * w2 * (dG * is) * (iD * iD);
+    double g1, i1, g2, i2, gs, q, dg, iD2;
+    if constexpr (EXACT) {
+      g1 = sqrt(G1);
+      g2 = sqrt(G2);
+      i1 = 1.0 / g1;
+      i2 = 1.0 / g2;
+      gs = g1 + g2;
+      q = fma(2.0 * g1, g2, Tc) / D;
+      dg = dG / gs;
+      iD2 = 1.0 / (D * D);
+    } else {
+      gb_sqrt(G1, g1, i1);
+      gb_sqrt(G2, g2, i2);
+      gs = g1 + g2;
+      const double iD = gb_rcp(D);
+      q = fma(2.0 * g1, g2, Tc) * iD;
+      dg = dG * gb_rcp(gs);
+      iD2 = iD * iD;
+    }
+    const double w = fma(ks, q - m, wm);
+    const double f = w * w2 * dg * iD2;
     const int i = s - 2;
     const bool on = col_on && i >= 0 && i < a.Hout;  // outside the map: no share
     auto adjoint = [&](double t, double gx, double gy, double (&hx)[2], double (&hy)[2]) {
@@ -985,6 +1015,12 @@ __global__ __launch_bounds__(BLOCK) void gmsd_backward_kernel(GmsdBwdArgs a) {
   ya = sample(p0.y);
   xb = sample(p1.x);
   yb = sample(p1.y);
+  if constexpr (EXACT) {
+    ex[0] = col_diff(xa);
+    ex[1] = col_diff(xb);
+    ey[0] = col_diff(ya);
+    ey[1] = col_diff(yb);
+  }
   for (int j = 0; j < steps; j += 2) {  // uniform
     const GbRaw<T, DOWN> cur0 = buf0, cur1 = buf1;
     buf0 = load(s0 + j + 2);

@@ -642,6 +642,31 @@ def test_gms_gradient_strip_edges(gpu, hw, wrt):
                 assert t.grad is None
 
 
+@pytest.mark.parametrize("down", [False, True])
+@pytest.mark.parametrize("raised", [False, True])
+def test_gms_gradient_float64_digits(gpu, down, raised):
+    """float64 samples keep their digits, also above a pedestal that fills the word
+    (multiples of 2^-10 above 2^42, or above 2^40 where 2 x 2 sums of them are formed:
+    53 bits either way), so that a sum of three would round.  Differences of exact
+    samples are exact, so the gradient is that of the samples alone: ~60
+    roundings of 2^-53 under q - m's cancellation (~10), 1e-13 max-normwise."""
+    from frame_analytics_amd import backend
+
+    rng = np.random.default_rng(9)
+    pedestal = (2.0 ** 40 if down else 2.0 ** 42) if raised else 0.0
+    a = rng.integers(0, 1025, (2, 2, 41, 131)) / 1024.0
+    b = np.clip(a + rng.integers(-96, 97, a.shape) / 1024.0, 0, 1)
+    T, eps = 170.0 / 255.0 ** 2, 1e-12
+    m, s = ref.gmsd_stats(a, b, 1.0, downsample=down)
+    gm, gs = np.array([0.7, -1.2]), np.array([1.4, 0.5])
+    to = lambda v: torch.from_numpy(np.ascontiguousarray(v)).to(gpu)  # noqa: E731
+    got = backend.gmsd_stats_bwd(to(a + pedestal), to(b + pedestal), to(m), to(s), to(gm), to(gs),
+                                 T, eps, down, True, True)
+    want = ref.gms_stats_grad(a, b, 1.0, downsample=down, g_mean=gm, g_std=gs)
+    for g, w in zip(got, want):
+        assert np.abs(g.cpu().numpy() - w).max() <= 1e-13 * np.abs(w).max()
+
+
 def test_gms_loss_gradient_finite(gpu):
     x = torch.rand(1, 1, 64, 64, device=gpu, requires_grad=True)
     y = x.detach().clone()
