@@ -1359,8 +1359,18 @@ bool mfma_fits(const SsimMfmaCall& c, int src, int mode) {
 // lane reads whole dwords from at most 11 bytes before its row's last
 // dword, so rows are at least 16 samples.  The map stays there: per pixel its
 // float32 sums are closer than the 22-bit operands here; so do single CS passes.
+//
+// rag_constants: these kernels centre the samples on 128 whatever the data range,
+// and their moments, up to 128^2, carry 2^-22: a variance is off by up to ~0.004,
+// which C2 has to outweigh.  The default constants at a data range of 255
+// (6.5025, 58.5225) and larger ones do; with those of a range of 1 (masks as
+// bytes, C2 = 9e-4) the mean came out as NaN where the strip kernel, which centres
+// on half the range, is 1e-6 off.
+constexpr double RAG_MIN_C1 = 6.5, RAG_MIN_C2 = 58.5;
+bool rag_constants(double C1, double C2) { return C1 >= RAG_MIN_C1 && C2 >= RAG_MIN_C2; }
+
 bool mfma_rag(const SsimMfmaCall& c) {
-  if (c.K > MF_MAX_K || c.W < 16) return false;
+  if (c.K > MF_MAX_K || c.W < 16 || !rag_constants(c.C1, c.C2)) return false;
   return (static_cast<int64_t>(c.H) + 48) * std::max(c.xsh, c.ysh) + 16 <= INT32_MAX;
 }
 
@@ -1582,7 +1592,9 @@ int ssim_mfma_ms(const SsimMfmaMs& c, int device, hipStream_t st, bool* done) {
     } else {
       rag[i] = pitch != W;
     }
-    if (rag[i] && static_cast<int64_t>(c.H) * c.W < MS_RAG_MIN_PLANE) return FA_OK;
+    if (rag[i] && (static_cast<int64_t>(c.H) * c.W < MS_RAG_MIN_PLANE ||
+                   !rag_constants(c.C1, c.C2)))
+      return FA_OK;
     if (i > 0) {
       SsimMfmaCall q = k;  // the padded rows meet the alignment
       q.W = pitch;

@@ -587,3 +587,25 @@ def test_ragged_ms_ssim_matches_oracle(gpu, shape, scales):
         got = float(fa.ms_ssim(x, y, data_range=255.0, weights=w))
         assert abs(got - want) <= 2e-7 * abs(want)
     assert backend.native_calls["fa_gpu_ms_ssim"] == n.get("fa_gpu_ms_ssim", 0) + 2
+
+
+@pytest.mark.parametrize("shape", [(1, 3, 395, 693), (2, 1, 61, 75)])
+@pytest.mark.parametrize("what", ["masks", "small_k"])
+def test_ragged_rows_with_small_constants(gpu, shape, what):
+    """Bytes of another range than 255 on rows that are no multiple of 8: 0/1 masks
+    scored at a data range of 1, and constants a thousandth of the usual.  Moments of
+    samples centred on half the range are at most a quarter of its square and
+    carry 2^-24, against C2 = 9e-4 of it (2^-24 / 4 / 9e-4 = 1.7e-5 of a flat
+    pixel); with the small constants, on noise, sigma^2 outweighs them."""
+    a, b = u8_pair(shape, 9.0, seed=shape[-1])
+    L, K = 255.0, (1e-5, 3e-5)
+    if what == "masks":
+        a, L, K = (a > 127).astype(np.uint8), 1.0, (0.01, 0.03)
+        b = a ^ (b % 31 == 0)
+    x, y = torch.from_numpy(a).to(gpu), torch.from_numpy(b).to(gpu)
+    want = np.array([ref.ssim(a[i:i + 1], b[i:i + 1], L, K=K) for i in range(shape[0])])
+    got = fa.ssim(x, y, data_range=L, K=K, reduction="none").cpu().numpy()
+    assert np.all(np.abs(got - want) <= 2e-5 * np.abs(want)), (got, want)
+    if shape[-2] >= 176:
+        want = ref.ms_ssim(a.astype(np.float64), b.astype(np.float64), L, K=K)
+        assert abs(float(fa.ms_ssim(x, y, data_range=L, K=K)) - want) <= 2e-5 * abs(want)
