@@ -609,3 +609,34 @@ def test_ragged_rows_with_small_constants(gpu, shape, what):
     if shape[-2] >= 176:
         want = ref.ms_ssim(a.astype(np.float64), b.astype(np.float64), L, K=K)
         assert abs(float(fa.ms_ssim(x, y, data_range=L, K=K)) - want) <= 2e-5 * abs(want)
+
+
+def _frame_pair(n, h, w, seed):
+    """Smooth shapes, texture and grain with a mild distortion, as bytes."""
+    gen = torch.Generator().manual_seed(seed)
+
+    def field(step):
+        g = torch.rand(n, 1, h // step + 2, w // step + 2, generator=gen)
+        return torch.nn.functional.interpolate(g, size=(h, w), mode="bilinear",
+                                               align_corners=False)
+
+    x = 0.55 * field(64) + 0.30 * field(12) + 0.15 * torch.rand(n, 1, h, w, generator=gen)
+    y = x + 0.03 * torch.randn(n, 1, h, w, generator=gen)
+    return tuple((255.0 * t.clamp(0, 1)).round().to(torch.uint8) for t in (x, y))
+
+
+def test_ragged_means_no_further_off_than_float32(gpu, monkeypatch):
+    """Rows that are no multiple of 8: over picture-like frames the matrix cores' mean
+    SSIM is no further from the oracle (rms) than the float32 strip kernel's, which
+    FA_SSIM_MFMA=0 selects."""
+    err = {"1": [], "0": []}
+    for i, (h, w) in enumerate(((363, 369), (367, 421), (405, 331), (362, 363), (511, 517))):
+        a, b = _frame_pair(3, h, w, i)
+        x, y = a.to(gpu), b.to(gpu)
+        want = ref.ssim(a.numpy(), b.numpy(), 255.0, reduction="none")
+        for env in err:
+            monkeypatch.setenv("FA_SSIM_MFMA", env)
+            got = fa.ssim(x, y, data_range=255.0, reduction="none").cpu().numpy()
+            err[env].append(got / want - 1.0)
+    rms = {k: np.sqrt((np.array(v) ** 2).mean()) for k, v in err.items()}
+    assert rms["1"] <= rms["0"], rms
