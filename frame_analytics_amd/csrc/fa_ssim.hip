@@ -1457,9 +1457,14 @@ struct MsPlan {
   int level_dtype[MS_MAX_SCALES];  // element type of level i (i >= 1)
   int64_t level_x[MS_MAX_SCALES], level_y[MS_MAX_SCALES];  // byte offsets (i >= 1)
   int64_t pcs[MS_MAX_SCALES], ps_last, scratch, total;
+  int64_t own_words, own_images;  // `padded` only
 };
 
-static int ms_plan(int dtype, int N, int C, int H, int W, int K, int M, bool luma, MsPlan* p) {
+// `padded`: with what uint8 rows of any width take in the three-launch form, levels of
+// rows padded to 8 samples and words of the call's own; *padded is left false (and the
+// plan is the other one) where the sizes rule that form out.
+static int ms_plan(int dtype, int N, int C, int H, int W, int K, int M, bool luma, MsPlan* p,
+                   bool* padded = nullptr) {
   if (dtype < FA_U8 || dtype > FA_F64) return FA_E_DTYPE;
   if (M <= 0 || M > MS_MAX_SCALES || N <= 0 || C <= 0) return FA_E_SHAPE;
   if (luma && C != 3) return FA_E_SHAPE;
@@ -1467,6 +1472,9 @@ static int ms_plan(int dtype, int N, int C, int H, int W, int K, int M, bool lum
   p->cout = luma ? 1 : C;
   const int64_t planes = static_cast<int64_t>(N) * p->cout;
   const bool u8 = dtype == FA_U8 && !luma;
+  const int64_t own =
+      u8 && padded && *padded ? ssim_mfma_ms_own_words(N, C, H, W, K, M) : 0;
+  if (padded) *padded = own > 0;
   int64_t off = 0;
   auto take = [&](int64_t bytes) {
     const int64_t at = off;
@@ -1484,9 +1492,7 @@ static int ms_plan(int dtype, int N, int C, int H, int W, int K, int M, bool lum
       p->level_dtype[i] = u8 ? (i == 1 ? FA_F16 : FA_F32) : FA_F64;
       p->in_dtype[i] = u8 ? (p->level_dtype[i] | FA_DTYPE_U8_PYRAMID) : FA_F64;
       const int64_t eb = p->level_dtype[i] == FA_F16 ? 2 : p->level_dtype[i] == FA_F32 ? 4 : 8;
-      // (rows of a uint8 pyramid's levels with room for the three-launch form's
-      // padding; the per-scale form packs them)
-      const int64_t lb = planes * p->H[i] * (u8 ? mf_level_pitch(p->W[i]) : p->W[i]) * eb;
+      const int64_t lb = planes * p->H[i] * (own ? mf_level_pitch(p->W[i]) : p->W[i]) * eb;
       p->level_x[i] = take(lb);
       p->level_y[i] = take(lb);
     } else {
@@ -1496,6 +1502,8 @@ static int ms_plan(int dtype, int N, int C, int H, int W, int K, int M, bool lum
     p->pcs[i] = take(planes * p->bpp[i] * 8);
   }
   p->ps_last = take(planes * p->bpp[M - 1] * 8);
+  p->own_words = own ? take(own * 8) : 0;
+  p->own_images = own ? take(static_cast<int64_t>(N) * 8) : 0;
   p->scratch = take(static_cast<int64_t>(M) * planes * 8);
   p->total = off;
   return FA_OK;
@@ -1883,7 +1891,8 @@ FA_API int fa_gpu_ms_ssim_workspace(int dtype, int N, int C, int H, int W, int K
                                     int luma, int64_t* out_bytes) {
   if (!out_bytes) return FA_E_ARG;
   MsPlan p;
-  const int rc = ms_plan(dtype, N, C, H, W, K, M, luma != 0, &p);
+  bool padded = true;
+  const int rc = ms_plan(dtype, N, C, H, W, K, M, luma != 0, &p, &padded);
   if (rc != FA_OK) return rc;
   *out_bytes = p.total;
   return FA_OK;
@@ -1901,12 +1910,19 @@ FA_API int fa_gpu_ms_ssim(const void* x, const void* y, int dtype, int N, int C,
   if (!x || !y || !win || !weights || !workspace) return FA_E_ARG;
   if (!out_per_image && !out_total) return FA_E_ARG;
   if (luma && C != 3) return FA_E_SHAPE;
+  // a workspace of the packed plan's size, without room for padded levels, is enough
+  // for the per-scale form
   MsPlan p;
-  int rc = ms_plan(dtype, N, C, H, W, K, M, luma != nullptr, &p);
+  bool padded = true;
+  int rc = ms_plan(dtype, N, C, H, W, K, M, luma != nullptr, &p, &padded);
+  if (rc == FA_OK && padded && workspace_bytes < p.total) {
+    padded = false;
+    rc = ms_plan(dtype, N, C, H, W, K, M, luma != nullptr, &p);
+  }
   if (rc != FA_OK) return rc;
   if (workspace_bytes < p.total) return FA_E_ARG;
   char* ws = static_cast<char*>(workspace);
-  if (acc && dtype == FA_U8 && !luma) {
+  if (dtype == FA_U8 && !luma) {
     // three launches, the reduction finished in the last (ssim_mfma_ms)
     SsimArgs v = {};
     rc = set_views(v, C, H, W, x_strides, y_strides, nullptr);
@@ -1935,6 +1951,10 @@ FA_API int fa_gpu_ms_ssim(const void* x, const void* y, int dtype, int N, int C,
       mc.ly[i] = ws + p.level_y[i];
     }
     mc.words = acc;
+    if (padded) {
+      mc.own_words = reinterpret_cast<uint64_t*>(ws + p.own_words);
+      mc.own_images = reinterpret_cast<double*>(ws + p.own_images);
+    }
     mc.out_per_image = out_per_image;
     mc.out_total = out_total;
     bool done = false;

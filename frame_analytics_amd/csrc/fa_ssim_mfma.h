@@ -72,14 +72,22 @@ struct SsimMfmaMs {
   void* lx[8];                 // level i >= 1 of x and y: floor(H / 2^i) rows of
   void* ly[8];                 //   mf_level_pitch(floor(W / 2^i)) samples per plane,
                                //   float16 (i = 1), float32
-  uint64_t* words;             // FA_MS_SSIM_ACC_WORDS, zero; left zero
+  uint64_t* words;             // null, or FA_MS_SSIM_ACC_WORDS, zero; left zero
+  uint64_t* own_words;         // null, or ssim_mfma_ms_own_words of workspace ...
+  double* own_images;          // ... and N doubles: what ragged rows may take
   double* out_per_image;
   double* out_total;
 };
 
-// Launches it when the input fits ssim_mfma's rules (any width and alignment),
-// C1 and C2 positive, and sets *done; otherwise launches nothing
-// and leaves *done false, for the per-scale path.
+// Workspace words of a call whose input may have scales that need the RAG kernels, 0
+// where its sizes rule them out.
+int64_t ssim_mfma_ms_own_words(int N, int C, int H, int W, int K, int M);
+
+// Launches it and sets *done when the input fits ssim_mfma's rules (any width and
+// alignment) with C1 and C2 positive: input aligned at every scale where `words` is
+// set and N * C <= 256, other input (from 2^17 samples a plane, the default constants
+// or larger) always, given the workspace's own words.  Otherwise leaves *done
+// false, for the per-scale path.
 int ssim_mfma_ms(const SsimMfmaMs& c, int device, hipStream_t st, bool* done);
 
 }  // namespace fa

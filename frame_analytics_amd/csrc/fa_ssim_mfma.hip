@@ -1198,11 +1198,11 @@ constexpr int MS_WORD_SCALES = 8;
 constexpr int MS_FIN_MAX_PLANES = 256;
 // Scales whose rows need the RAG kernels are taken from this many samples of an
 // input plane on: 151 -> 88 us for fa.ssim and fa.ms_ssim together at 4 x 3 x 767 x
-// 1366, 43 -> 23 us for fa.ms_ssim at 1 x 3 x 600 x 601.  Smaller planes would gain
-// too (38 -> 22 us at 2 x 3 x 352 x 360, 92 -> 46 at 32 x 3 x 250 x 300), but there
-// the per-scale path's results are pinned to the last bits between batch sizes,
-// with and without an accumulator and to the single CS passes, which stay on
-// the vector-ALU kernel.
+// 1366, 43 -> 23 us for fa.ms_ssim at 1 x 3 x 600 x 601.  It is no limit of speed:
+// smaller planes would gain too (38 -> 22 us at 2 x 3 x 352 x 360, 92 -> 46 at 32 x 3 x
+// 250 x 300).  But the single CS passes (fa_gpu_ssim_cs*) of such rows stay on the
+// vector-ALU kernel, and where the RAG form is taken the result is no longer their
+// product to the last bits (9e-9 apart); below this size it still is.
 constexpr int64_t MS_RAG_MIN_PLANE = int64_t(1) << 17;
 static_assert(FA_MS_SSIM_ACC_WORDS == (MS_WORD_SCALES * MS_FIN_MAX_PLANES + 1) * MF_STRIDE,
               "the ABI's accumulator size");
@@ -1578,23 +1578,18 @@ int ssim_mfma(const SsimMfmaCall& c, int device, hipStream_t st, int* tiles) {
   return FA_OK;
 }
 
-int ssim_mfma_ms(const SsimMfmaMs& c, int device, hipStream_t st, bool* done) {
-  *done = false;
+namespace {
+
+// Every scale's call of the three-launch MS-SSIM and whether it takes a RAG kernel;
+// false where a scale fits no kernel.  Levels are rows padded to 8 samples
+// (ms_plan sizes them so); a scale whose rows need the padding, or a uint8 input that
+// misses the alignment, takes the RAG form of its kernel.
+bool ms_calls(const SsimMfmaMs& c, SsimMfmaCall* calls, bool* rag) {
   const int M = c.M;
-  const int64_t planes = static_cast<int64_t>(c.N) * c.C;
-  if (!mfma_enabled() || !c.words || M < 3 || M > 2 + MS_TAIL_MAX) return FA_OK;
-  if (planes > MS_FIN_MAX_PLANES || !(c.C1 > 0.0) || !(c.C2 > 0.0)) return FA_OK;
-  if (!c.out_per_image && !c.out_total) return FA_OK;
-  // every scale's call, checked before anything is launched
-  // Levels are rows padded to 8 samples (ms_plan sizes them so); a scale whose
-  // rows need the padding, or a uint8 input that misses the alignment, takes the
-  // RAG form of its kernel.
-  MfArgs a[2 + MS_TAIL_MAX];
-  bool rag[2 + MS_TAIL_MAX] = {};
-  double finv[MS_WORD_SCALES] = {}, npix[MS_WORD_SCALES] = {};
   int H = c.H, W = c.W;
   for (int i = 0; i < M; ++i) {
-    SsimMfmaCall k = {};
+    SsimMfmaCall& k = calls[i];
+    k = SsimMfmaCall{};
     k.x = i == 0 ? c.x : c.lx[i];
     k.y = i == 0 ? c.y : c.ly[i];
     k.src = i == 0 ? SsimMfmaCall::U8 : i == 1 ? SsimMfmaCall::F16_LEVEL : SsimMfmaCall::F32_LEVEL;
@@ -1624,34 +1619,49 @@ int ssim_mfma_ms(const SsimMfmaMs& c, int device, hipStream_t st, bool* done) {
     }
     const int src = i == 0 ? SRC_U8 : i == 1 ? SRC_F16 : SRC_F32;
     const int mode = i + 1 < M ? MF_CSO : MF_CS;
-    if (k.Hout < 1 || k.Wout < 1) return FA_OK;
+    if (k.Hout < 1 || k.Wout < 1) return false;
     if (i == 0) {
       rag[i] = !mfma_fits(k, src, mode);
-      if (rag[i] && !mfma_rag(k)) return FA_OK;
+      if (rag[i] && !mfma_rag(k)) return false;
     } else {
       rag[i] = pitch != W;
     }
     if (rag[i] && (static_cast<int64_t>(c.H) * c.W < MS_RAG_MIN_PLANE ||
                    !rag_constants(c.C1, c.C2)))
-      return FA_OK;
+      return false;
     if (i > 0) {
       SsimMfmaCall q = k;  // the padded rows meet the alignment
       q.W = pitch;
-      if (!mfma_fits(q, src, mode)) return FA_OK;
+      if (!mfma_fits(q, src, mode)) return false;
     }
     if (i == 1)
       for (int d = 0; d < 2; ++d)
         if (3 + d < M && (reinterpret_cast<uintptr_t>(c.lx[3 + d]) |
                           reinterpret_cast<uintptr_t>(c.ly[3 + d])) & 15)
-          return FA_OK;
-    a[i] = args_of(k);
-    a[i].lpitch = mf_level_pitch(W / 2);
-    for (int d = 0; d < 2; ++d) a[i].dpitch[d] = mf_level_pitch(W >> (d + 2));
-    npix[i] = static_cast<double>(k.Hout) * k.Wout;
-    fixed_scale(npix[i], &a[i].fscale, &finv[i]);
-    a[i].acc = c.words + static_cast<int64_t>(i) * planes * MF_STRIDE;
+          return false;
     H /= 2;
     W /= 2;
+  }
+  return true;
+}
+
+// The three launches over at most MS_FIN_MAX_PLANES planes; nothing launched and
+// *done left false where they cannot be planned.
+int ms_three(const SsimMfmaMs& c, int device, hipStream_t st, bool* done) {
+  const int M = c.M;
+  const int64_t planes = static_cast<int64_t>(c.N) * c.C;
+  SsimMfmaCall calls[2 + MS_TAIL_MAX];
+  MfArgs a[2 + MS_TAIL_MAX];
+  bool rag[2 + MS_TAIL_MAX] = {};
+  double finv[MS_WORD_SCALES] = {}, npix[MS_WORD_SCALES] = {};
+  if (!ms_calls(c, calls, rag)) return FA_OK;
+  for (int i = 0; i < M; ++i) {
+    a[i] = args_of(calls[i]);
+    a[i].lpitch = mf_level_pitch(calls[i].W / 2);
+    for (int d = 0; d < 2; ++d) a[i].dpitch[d] = mf_level_pitch(calls[i].W >> (d + 2));
+    npix[i] = static_cast<double>(calls[i].Hout) * calls[i].Wout;
+    fixed_scale(npix[i], &a[i].fscale, &finv[i]);
+    a[i].acc = c.words + static_cast<int64_t>(i) * planes * MF_STRIDE;
   }
   // scale 1 also writes the levels of scales 3 and 4
   for (int d = 0; d < 2; ++d) {
@@ -1751,6 +1761,79 @@ int ssim_mfma_ms(const SsimMfmaMs& c, int device, hipStream_t st, bool* done) {
                      st, t);
   FA_LAUNCH_CHECK();
   *done = true;
+  return FA_OK;
+}
+
+// n of the words that ms_three takes zeroed (a memset would be a graph node of its own
+// kind in a capture).
+__global__ __launch_bounds__(BLOCK) void ms_zero_kernel(uint64_t* words, int n) {
+  const int i = static_cast<int>(blockIdx.x) * BLOCK + static_cast<int>(threadIdx.x);
+  if (i < n) words[static_cast<int64_t>(i) * MF_STRIDE] = 0;
+}
+
+// The batch mean of per-image values, in the tail kernel's order.
+__global__ __launch_bounds__(BLOCK) void ms_mean_kernel(const double* per_image, int N,
+                                                        double* out) {
+  __shared__ double sred[2 * WAVES_PER_BLOCK];
+  double tot = 0.0;
+  for (int n = threadIdx.x; n < N; n += BLOCK) tot += per_image[n];
+  tot = block_sum(tot, sred);
+  if (threadIdx.x == 0) *out = tot / static_cast<double>(N);
+}
+
+}  // namespace
+
+int64_t ssim_mfma_ms_own_words(int N, int C, int H, int W, int K, int M) {
+  if (M < 3 || M > 2 + MS_TAIL_MAX || K > MF_MAX_K || C > MS_FIN_MAX_PLANES ||
+      static_cast<int64_t>(H) * W < MS_RAG_MIN_PLANE)
+    return 0;
+  const int64_t images = std::min<int64_t>(N, MS_FIN_MAX_PLANES / C);
+  return (M * images * C + 1) * MF_STRIDE;
+}
+
+int ssim_mfma_ms(const SsimMfmaMs& c, int device, hipStream_t st, bool* done) {
+  *done = false;
+  if (!mfma_enabled() || c.M < 3 || c.M > 2 + MS_TAIL_MAX) return FA_OK;
+  if (c.C > MS_FIN_MAX_PLANES || !(c.C1 > 0.0) || !(c.C2 > 0.0)) return FA_OK;
+  if (!c.out_per_image && !c.out_total) return FA_OK;
+  SsimMfmaCall calls[2 + MS_TAIL_MAX];
+  bool rag[2 + MS_TAIL_MAX] = {};
+  if (!ms_calls(c, calls, rag)) return FA_OK;
+  bool any_rag = false;
+  for (int i = 0; i < c.M; ++i) any_rag = any_rag || rag[i];
+  const int per = MS_FIN_MAX_PLANES / c.C;  // images of one group
+  if (!any_rag) {
+    // aligned scales have the same arithmetic in the per-scale passes
+    return c.words && c.N <= per ? ms_three(c, device, st, done) : FA_OK;
+  }
+  // A RAG scale differs from its per-scale pass, the float32 strip kernel, by ~1e-8:
+  // one input has one result, so every call that can take these kernels does, in
+  // groups of images and on words of the workspace where it has no accumulator.
+  if (!c.own_words) return FA_OK;
+  SsimMfmaMs g = c;
+  if (!c.words) {
+    const int n = c.M * std::min(c.N, per) * c.C + 1;
+    g.words = c.own_words;
+    hipLaunchKernelGGL(ms_zero_kernel, dim3((n + BLOCK - 1) / BLOCK), dim3(BLOCK), 0, st, g.words,
+                       n);
+    FA_LAUNCH_CHECK();
+  }
+  if (c.N <= per) return ms_three(g, device, st, done);
+  double* each = c.out_per_image ? c.out_per_image : c.own_images;
+  for (int n0 = 0; n0 < c.N; n0 += per) {
+    g.x = static_cast<const uint8_t*>(c.x) + n0 * c.xsn;
+    g.y = static_cast<const uint8_t*>(c.y) + n0 * c.ysn;
+    g.N = std::min(per, c.N - n0);
+    g.out_per_image = each + n0;
+    g.out_total = nullptr;
+    *done = false;
+    const int rc = ms_three(g, device, st, done);
+    if (rc != FA_OK || !*done) return rc;
+  }
+  if (c.out_total) {
+    hipLaunchKernelGGL(ms_mean_kernel, dim3(1), dim3(BLOCK), 0, st, each, c.N, c.out_total);
+    FA_LAUNCH_CHECK();
+  }
   return FA_OK;
 }
 

@@ -413,18 +413,25 @@ FA_API int fa_gpu_ms_ssim_head_backward(const double* const* terms, int M,
  * with no host work between them.  x / y: N x C x H x W of any dtype, with
  * optional strides and luma as in fa_gpu_ssim_ex; weights: host array of M.
  * workspace: at least fa_gpu_ms_ssim_workspace's bytes of device memory
- * (levels, partial sums, scratch).  Every scale's shape is checked before
+ * (levels, partial sums, scratch).  (For uint8 planes of 2^17 samples and more that
+ * is a few percent more than packed levels take; the smaller size of earlier
+ * builds is still accepted and serves the one-launch-per-scale form.)  Every
+ * scale's shape is checked before
  * anything is launched.  out_per_image (N) / out_total (1) float64: either
  * may be null, not both.
  *
  * acc: null, or FA_MS_SSIM_ACC_WORDS uint64 of device memory, zero when the
  * call starts; the call leaves it zero.  With it, uint8 input without luma
  * whose every scale fits the matrix-core kernel (widths a multiple of 8 at
- * every scale, e.g. W % 128 == 0 at M = 5, or planes of 2^17 samples and more; K <= 16; C1, C2 > 0; N * C <= 256;
+ * every scale, e.g. W % 128 == 0 at M = 5; K <= 16; C1, C2 > 0; N * C <= 256;
  * 3 <= M <= 5) runs as three launches: scale 0, scale 1 (which also writes
  * levels 3 and 4), and scales 2 .. M - 1 side by side in one launch whose last
  * workgroup finishes the reduction from per-(scale, plane) fixed-point sums
  * (about 1e-13 relative from the float64 reduction, the same bits run to run).
+ * Rows of other widths or alignments run so from planes of 2^17 samples on
+ * (C <= 256, C1 >= 6.5, C2 >= 58.5), with `acc` or without and in groups of up to
+ * 256 planes, so that neither changes an image's value; it is ~1e-8 from the
+ * product of fa_gpu_ssim_cs's means, which such rows get from another kernel.
  * Other calls ignore acc.  `acc` is state of one stream: calls that overlap
  * on it (two streams, graph replays beside eager calls) race.  After a
  * non-zero status its contents are unknown (a failure between the launches

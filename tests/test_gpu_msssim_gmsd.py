@@ -153,9 +153,10 @@ def test_ms_ssim_too_small(gpu):
     assert float(fa.ms_ssim(z, z, data_range=1.0)) == pytest.approx(1.0)
 
 
-def _ms_call(x, y, weights, k=11, acc=None):
-    """fa_gpu_ms_ssim through the C ABI over a workspace filled with 0xFF:
-    (per-image values, batch mean, the workspace afterwards)."""
+def _ms_call(x, y, weights, k=11, acc=None, nbytes=None):
+    """fa_gpu_ms_ssim through the C ABI over a workspace (the queried size or
+    ``nbytes``) filled with 0xFF: (per-image values, batch mean, the workspace
+    afterwards)."""
     import ctypes
 
     from frame_analytics_amd import backend
@@ -167,6 +168,9 @@ def _ms_call(x, y, weights, k=11, acc=None):
     nb = ctypes.c_int64(0)
     assert backend.call_gpu("fa_gpu_ms_ssim_workspace", 0, n, c, h, w, k, m, 0,
                             ctypes.byref(nb)) == 0
+    if nbytes is not None:
+        assert nbytes <= nb.value
+        nb.value = nbytes
     ws = torch.full((nb.value,), 0xFF, dtype=torch.uint8, device=x.device)
     out = torch.full((n + 1,), -7.0, dtype=torch.float64, device=x.device)
     x, xs = backend._view_strides(x)
@@ -267,6 +271,85 @@ def test_ms_ssim_three_launch_path(gpu, shape, weights, k, crop):
     want = ref.ms_ssim(x.cpu().numpy().astype(np.float64), y.cpu().numpy().astype(np.float64),
                        255.0, win_size=k, weights=w, reduction="none")
     assert np.all(np.abs(per - want) <= REL * np.abs(want)), (per, want)
+
+
+def _packed_workspace(n, c, h, w, k, m):
+    """Bytes of the per-scale form's workspace: the levels packed, partial sums of
+    4-row chunks, the reduction's scratch, each piece 256-byte aligned."""
+    up = lambda v: (v + 255) // 256 * 256  # noqa: E731
+    total, slots = 0, 0
+    for i in range(m):
+        ho, wo = (h >> i) - k + 1, (w >> i) - k + 1
+        if i:
+            total += 2 * up(n * c * (h >> i) * (w >> i) * (2 if i == 1 else 4))
+        slots = -(-wo // (256 - k + 1)) * -(-ho // 4)
+        total += up(n * c * slots * 8)
+    return total + up(n * c * slots * 8) + up(m * n * c * 8)
+
+
+@pytest.mark.parametrize("shape,scales,k", [((3, 3, 362, 363), 5, 11), ((2, 1, 433, 421), 4, 7),
+                                            ((1, 3, 592, 600), 3, 11), ((130, 2, 363, 364), 5, 11),
+                                            ((2, 3, 512, 512), 5, 11)])
+def test_ragged_ms_ssim_has_one_result(gpu, shape, scales, k):
+    """Planes of 2^17 samples and more whose rows are no multiple of 8 at some scale:
+    the three launches, with and without an accumulator, alone and in a batch (here
+    also more than the 256 planes of one group), eager and captured, over a
+    workspace full of NaN: the sums are integers, so the same bits per image; the
+    batch mean adds them in another order (1e-14).  The last shape is aligned
+    at every scale but read in place at an odd offset."""
+    from frame_analytics_amd import backend
+
+    n, c, h, w = shape
+    wts = (0.0448, 0.2856, 0.3001, 0.2363, 0.1333)[:scales]
+    a, b = u8_pair((min(n, 3), c, h, w + 3), 9.0, seed=h)
+    a, b = (np.tile(v, (-(-n // len(v)), 1, 1, 1))[:n] for v in (a, b))
+    x, y = torch.from_numpy(a).to(gpu)[..., 1:w + 1], torch.from_numpy(b).to(gpu)[..., 2:w + 2]
+    if w % 8:
+        x, y = x.contiguous(), y.contiguous()
+    acc = torch.zeros(backend._ACC_WORDS["ms"], dtype=torch.int64, device=gpu)
+    per, tot, ws = _ms_call(x, y, wts, k, acc=acc)
+    scratch = scales * n * c * 8
+    start = -((scratch + 255) // 256 * 256)
+    assert bool((ws[start:start + scratch] == 0xFF).all())  # not the per-scale form
+    assert not bool(acc.any())
+    per0, tot0, ws = _ms_call(x, y, wts, k)
+    assert bool((ws[start:start + scratch] == 0xFF).all())
+    assert np.array_equal(per0, per) and abs(tot0 - tot) <= 1e-14
+    one = [_ms_call(x[i:i + 1], y[i:i + 1], wts, k, acc=acc)[0][0] for i in range(min(n, 3))]
+    assert np.array_equal(np.resize(one, n), per) and abs(tot - per.mean()) <= 1e-14
+    kw = dict(data_range=255.0, weights=wts, win_size=k, reduction="none")
+    want = ref.ms_ssim(x[:3].cpu().numpy().astype(np.float64),
+                       y[:3].cpu().numpy().astype(np.float64), **kw)
+    assert np.all(np.abs(per[:len(want)] - want) <= 1e-7 * np.abs(want))
+    eager = fa.ms_ssim(x, y, **kw)
+    assert np.array_equal(eager.cpu().numpy(), per)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = fa.ms_ssim(x, y, **kw)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        assert torch.equal(out, eager)
+        assert torch.equal(fa.ms_ssim(x, y, **kw), eager)
+
+
+def test_ragged_ms_ssim_takes_the_packed_workspace(gpu):
+    """A workspace of packed levels, all that the per-scale form needs, is still
+    accepted and serves it; one byte less is refused, and so is no workspace."""
+    from frame_analytics_amd import backend
+
+    wts = (0.0448, 0.2856, 0.3001, 0.2363, 0.1333)
+    for shape in ((2, 3, 391, 411), (1, 3, 250, 300)):
+        a, b = u8_pair(shape, 9.0, seed=3)
+        x, y = torch.from_numpy(a).to(gpu), torch.from_numpy(b).to(gpu)
+        nb = _packed_workspace(*shape, 11, 5)
+        acc = torch.zeros(backend._ACC_WORDS["ms"], dtype=torch.int64, device=gpu)
+        got = [_ms_call(x, y, wts, nbytes=nb, acc=v)[0] for v in (None, acc)]
+        assert np.array_equal(*got) and not bool(acc.any())
+        want = ref.ms_ssim(a.astype(np.float64), b.astype(np.float64), 255.0, reduction="none")
+        assert np.all(np.abs(got[0] - want) <= REL * np.abs(want))
+        with pytest.raises(AssertionError, match="5"):
+            _ms_call(x, y, wts, nbytes=nb - 1)
 
 
 @pytest.mark.parametrize("recompute", ["0", "1"])
