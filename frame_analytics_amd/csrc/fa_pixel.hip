@@ -804,7 +804,11 @@ constexpr int PIX_VIEW_WG_PER_CU = 4;
 // row, so they are mapped.  All loads of a step are issued before the first
 // DPP move: a move per load, between the loads, made the compiler wait for
 // each load in turn (crop at a byte offset: 355 us against 232).
-template <int OP, bool LUMA>
+//
+// WIDE: all four waves on one row, else a row per wave; a template, because with the
+// strides of either in registers the luma of 2 (8, at an odd offset) x 3 x 2160 x 3840
+// took 26.0 (92.0) us and not 24.6 (88.4).
+template <int OP, bool LUMA, bool WIDE>
 __global__ __launch_bounds__(BLOCK) void pix_view_u8_kernel(PixView v) {
   constexpr bool EXACT = !LUMA && (OP == FA_OP_MSE || OP == FA_OP_L1);
   constexpr int CH = LUMA ? 3 : 1;
@@ -837,12 +841,10 @@ __global__ __launch_bounds__(BLOCK) void pix_view_u8_kernel(PixView v) {
 
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / WAVE);
   const int lane = static_cast<int>(threadIdx.x) % WAVE;
-  // three channels of a row that fills a step of the whole workgroup: all waves on
-  // one row (8 x 3 x 2160 x 3840 luma: 79.3 us, 81.9 with a row per wave)
-  const bool wide = LUMA && nq >= 3 * BLOCK;
-  const int id = wide ? static_cast<int>(threadIdx.x) : lane;
-  const int span = wide ? BLOCK : WAVE;
-  const int first = wide ? 0 : wave * VR, next = wide ? VR : VR * WAVES_PER_BLOCK;
+  const int id = WIDE ? static_cast<int>(threadIdx.x) : lane;
+  constexpr int span = WIDE ? BLOCK : WAVE;
+  const int first = WIDE ? 0 : wave * VR;
+  constexpr int next = WIDE ? VR : VR * WAVES_PER_BLOCK;
   for (int64_t rr = r0 + first; rr < r1; rr += next) {  // uniform in the wave
     const uint8_t* pa[VR][CH];
     const uint8_t* pb[VR][CH];
@@ -964,9 +966,14 @@ __global__ __launch_bounds__(BLOCK) void pix_view_u8_kernel(PixView v) {
 
 template <typename T, int OP, bool LUMA>
 static void launch_view(dim3 grid, hipStream_t st, const PixView& v) {
-  if constexpr (std::is_same<T, uint8_t>::value)
-    hipLaunchKernelGGL((pix_view_u8_kernel<OP, LUMA>), grid, dim3(BLOCK), 0, st, v);
-  else
+  if constexpr (std::is_same<T, uint8_t>::value) {
+    // three channels of a row that fills a step of the whole workgroup: all waves on
+    // one row (8 x 3 x 2160 x 3840 luma: 79.3 us, 81.9 with a row per wave)
+    if (LUMA && v.W / 4 >= 3 * BLOCK)
+      hipLaunchKernelGGL((pix_view_u8_kernel<OP, LUMA, LUMA>), grid, dim3(BLOCK), 0, st, v);
+    else
+      hipLaunchKernelGGL((pix_view_u8_kernel<OP, LUMA, false>), grid, dim3(BLOCK), 0, st, v);
+  } else
     hipLaunchKernelGGL((pix_view_kernel<T, OP, LUMA>), grid, dim3(BLOCK), 0, st, v);
 }
 
