@@ -36,10 +36,11 @@ namespace fa {
 // only one of them at each scale, so the maps the backward needs are these
 // times that plane's upstream gradient, and no coefficient pass runs there.
 // MODE_CSC: MODE_CSF for the cs means and without dy's map, which is every scale
-// but the coarsest of a loss on x: the luminance terms drop out of the maps and
-// a lane's four columns of each are stored at once (quad_store).  The pass is bound
-// by its instructions (74 % of the cycles in MODE_CSF): 8 x 3 x 1080 x 1920 float32
-// 407 -> 347 us, 8 x 3 x 270 x 480 float64 39 -> 36.
+// but the coarsest of a loss on x: the luminance terms drop out of the maps (they are
+// still formed for the SSIM means) and a lane's four columns of each are stored at
+// once (quad_store).  The pass is bound by its instructions (74 % of the cycles in
+// MODE_CSF): 8 x 3 x 1080 x 1920 float32 traced 390 -> 359 us, 8 x 3 x 270 x 480 float64
+// 39 -> 36.
 enum { MODE_REDUCE = 0, MODE_MAP = 1, MODE_CS = 2, MODE_PREP = 3, MODE_PREP_CS = 4,
        MODE_CSF = 5, MODE_CSC = 6 };
 constexpr bool mode_sums_cs(int mode) {
@@ -78,7 +79,10 @@ struct Tiling {
 // forward launches (128 x 128 patches to eight RGB 1080p frames): the pick is 1.4 %
 // slower than the best TH on average, rounds of resident workgroups were 4 %
 // and up to 18 % (fa.ssim on a 1021 x 1357 luma plane 17.8 -> 15 us, on 1 x 3 x
-// 512 x 512 float32 13.3 -> 12.1, on 8 x 3 x 1080 x 1920 164 -> 157).
+// 512 x 512 float32 13.3 -> 12.1, on 8 x 3 x 1080 x 1920 164 -> 157).  Over 151 other
+// calls of fa.ssim it and the folds are 9 % faster in the mean; a few lose (one RGB 1080p float16
+// frame 30.0 -> 30.8, 2 x 3 x 767 x 1366 float32 with 7 taps 22.1 -> 23.7, the map of 4 x
+// 3 x 360 x 641 float32 18.0 -> 19.1).
 //
 // float64 kernels (2 or 3): rounds of resident workgroups x (TH + (K + 1) / 2); a
 // halo row only forms its moments, so the K - 1 halo rows weigh about half.
@@ -115,7 +119,10 @@ inline Tiling tiling_in(int64_t planes, int out_H, int out_W, int K, int64_t cus
 // strips -> folded: 8 x 3 x 512 x 768 bfloat16 46.0 -> 41.0 us, 8 x 3 x 512 x 512
 // float32 33.6 -> 27.8, 16 x 3 x 300 x 300 float16 30.1 -> 21.7, 8 x 3 x 720 x 1280
 // float32 87.3 -> 78.6; not taken, 1 x 3 x 720 x 1280 float32 19.2 -> 20.9 (two
-// workgroups each) and 1 x 3 x 1000 x 1000 bfloat16 20.1 -> 22.2 (finer, 5 %).
+// workgroups each) and 1 x 3 x 1000 x 1000 bfloat16 20.1 -> 22.2 (finer, 5 %).  Over 58
+// drawn calls with a narrow last strip this rule is 1.7 % off the better of the two on
+// average (at most 8 %), never folding 8.0 % and always folding 1.0 %: the two
+// conditions keep calls like the two above and cost a little in the mean.
 inline Tiling tiling_for(int64_t planes, int out_H, int out_W, int K, int64_t cus, int occ,
                          bool f64, bool fold) {
   double cost = 0.0;
@@ -592,7 +599,7 @@ struct ScatterArgs {
   void* dx;
   void* dy;
   const float* win;
-  int H, W, Hout, Wout, TH, strips, bpp, fold;
+  int H, W, Hout, Wout, TH, strips, bpp;
   double shift;
   const void* gpx;  // optional gradient of the next pyramid level (2x2 means)
   const void* gpy;
@@ -681,9 +688,9 @@ struct ScatterPol {
   // comes back 0 from the bounds check of its row, and nothing is done with a
   // value before its phase.  (Converted and masked when it was loaded, the level's
   // gradient made every phase wait for its two loads in turn, and with them for
-  // the maps of the next phase: 8 x 3 x 1080 x 1920 float32 336 us, 318 as it is
-  // read now, 302 with x, y and dx four columns at a time instead of one by one;
-  // 16 x 3 x 256 x 256 without a level 34 -> 31.  It moves 1.45 GB at 4.8 TB/s.)
+  // the maps of the next phase: 8 x 3 x 1080 x 1920 float32 traced 336 us, 306 as it
+  // is read now, with x, y and dx four columns at a time instead of one by one; 16 x
+  // 3 x 256 x 256 without a level 31.1 -> 30.5.  It moves 1.45 GB at 4.8 TB/s.)
   // With dy the second set of registers would take the kernel past 256 (one
   // wave per SIMD), so emit loads it itself.
   static constexpr bool PRE = !DY;
@@ -1065,7 +1072,7 @@ static int launch_strips(void (*kern)(Args), int occ, bool f64, bool fold, Args&
   a.TH = t.TH;
   a.strips = t.strips;
   a.bpp = t.tiles;
-  a.fold = t.gs;
+  if constexpr (std::is_same<Args, SsimArgs>::value) a.fold = t.gs;
   if (!strip_plan_ok(a)) return FA_E_ARG;  // nothing launched
   dim3 grid;
   const int rc = grid_of(planes, t.tiles, &grid);

@@ -1197,7 +1197,7 @@ constexpr int MS_TAIL_MAX = 3;         // scales 2 .. 4 of a five-scale pyramid
 constexpr int MS_WORD_SCALES = 8;
 constexpr int MS_FIN_MAX_PLANES = 256;
 // Scales whose rows need the RAG kernels are taken from this many samples of an
-// input plane on: 151 -> 88 us for fa.ssim and fa.ms_ssim together at 4 x 3 x 767 x
+// input plane on: 151 -> 90 us for fa.ssim and fa.ms_ssim together at 4 x 3 x 767 x
 // 1366, 43 -> 23 us for fa.ms_ssim at 1 x 3 x 600 x 601.  It is no limit of speed:
 // smaller planes would gain too (38 -> 22 us at 2 x 3 x 352 x 360, 92 -> 46 at 32 x 3 x
 // 250 x 300).  But the single CS passes (fa_gpu_ssim_cs*) of such rows stay on the
@@ -1393,8 +1393,8 @@ bool mfma_fits(const SsimMfmaCall& c, int src, int mode) {
 
 // The RAG kernels: uint8 rows of any width and alignment, for the forward's mean
 // and for the three-launch MS-SSIM.  Against the vector-ALU kernel that
-// took such rows, 4 x 3 x 767 x 1366: fa.ssim 49.0 -> 31 us, fa.ms_ssim 102 ->
-// 59 us (8 x 3 x 1080 x 1912: 173.6 -> 132), errors against float64 alike.  A
+// took such rows, 4 x 3 x 767 x 1366: fa.ssim 48.5 -> 31.4 us, fa.ms_ssim 102 ->
+// 61.7 us, errors against float64 no larger (hmfma).  A
 // lane reads whole dwords from at most 11 bytes before its row's last
 // dword, so rows are at least 16 samples.  The map stays there: per pixel its
 // float32 sums are closer than the 22-bit operands here; so do single CS passes.
